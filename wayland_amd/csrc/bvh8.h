@@ -11,10 +11,13 @@
 //   byte   15      imask       bit s set: slot s is an inner node
 //   bytes  16..19  child_base  inner child of slot s lives at child_base + s
 //   bytes  20..23  tri_base    first triangle record of this node's leaves
-//   bytes  24..31  meta[8]     leaf slot: (offset << 2) | (count - 1);
-//                              empty slot: 0xFF
-//   bytes  32..127 q[6][8]     quantised child boxes: lo_x, lo_y, lo_z,
-//                              hi_x, hi_y, hi_z; plane = p + scale * q, q an
+//   bytes  24..27  trivalid    nibble s: the triangles of leaf slot s, bits
+//                              0 .. count - 1 (0: inner or empty slot); the
+//                              leaves' records follow each other in slot
+//                              order from tri_base
+//   bytes  28..31  unused
+//   bytes  32..127 q[6][8]     quantised child boxes: lo_x, hi_x, lo_y, hi_y,
+//                              lo_z, hi_z; plane = p + scale * q, q an
 //                              integer 0..2047 held as binary16 (exact), so
 //                              gfx950's v_fma_mix_f32 reads it directly.
 // Child boxes are rounded outward and padded by one quantum, so the decoded
@@ -48,7 +51,8 @@ struct alignas(16) WlBvh8Node
     uint8_t imask;
     uint32_t child_base;
     uint32_t tri_base;
-    uint8_t meta[8];
+    uint32_t trivalid;
+    uint32_t pad_;
     uint16_t q[6][8];
 };
 
@@ -64,3 +68,10 @@ struct alignas(16) WlTriRecord
 
 static_assert(sizeof(WlBvh8Node) == 128, "BVH8 node must be 128 bytes");
 static_assert(sizeof(WlTriRecord) == 48, "triangle record must be 48 bytes");
+
+// Whether byte offsets of 32 bits reach every node and triangle record: the
+// traversal kernels then address them from a uniform base.
+static inline bool wl_bvh8_narrow(uint64_t nodes, uint64_t tris)
+{
+    return nodes * sizeof(WlBvh8Node) <= (1ull << 32) && tris * sizeof(WlTriRecord) < (1ull << 32);
+}

@@ -364,11 +364,10 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
         std::memset(&node, 0, sizeof node);
         for (int s = 0; s < 8; ++s)
         {
-            node.meta[s] = 0xFF;
             for (int k = 0; k < 3; ++k)
             {
-                node.q[k][s] = kHalfMaxFinite;
-                node.q[3 + k][s] = 0;
+                node.q[2 * k][s] = kHalfMaxFinite;
+                node.q[2 * k + 1][s] = 0;
             }
         }
         // quantisation frame = this node's box
@@ -395,7 +394,6 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
         }
         node.tri_base = (uint32_t)out->tris.size();
         // leaves in slot order
-        uint32_t tri_off = 0;
         for (int s = 0; s < 8; ++s)
         {
             int i = -1;
@@ -411,18 +409,17 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
                 double qhi = std::ceil(((double)k.box.hi[a] - node.p[a]) / scale[a]) + 1.0;
                 qlo = std::max(qlo, 0.0);
                 qhi = std::min(qhi, (double)kQMax);
-                node.q[a][s] = half_of_int((int)qlo);
-                node.q[3 + a][s] = half_of_int((int)qhi);
+                node.q[2 * a][s] = half_of_int((int)qlo);
+                node.q[2 * a + 1][s] = half_of_int((int)qhi);
             }
             if (k.count == 0)
             {
                 node.imask |= (uint8_t)(1u << s);
-                node.meta[s] = (uint8_t)s;
                 queue.push_back({ kids[i], node.child_base + (uint32_t)s, w.depth + 1 });
             }
             else
             {
-                node.meta[s] = (uint8_t)((tri_off << 2) | (k.count - 1));
+                node.trivalid |= ((1u << k.count) - 1u) << (4 * s);
                 for (uint32_t t = 0; t < k.count; ++t)
                 {
                     uint32_t p = b.prims[k.first + t];
@@ -433,7 +430,6 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
                     r.local = p;
                     out->tris.push_back(r);
                 }
-                tri_off += k.count;
                 out->leaves++;
                 if (root_area > 0)
                     sah += k.box.area() / root_area * k.count;

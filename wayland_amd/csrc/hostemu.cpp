@@ -90,26 +90,10 @@ uint64_t wlh_trace(void *p, const float *rays, uint32_t n, float *hits,
             wl::TravResult res;
             if (any)
                 res = wl::trav_run<true, true, 1>(h->bvh.nodes.data(), h->bvh.tris.data(),
-                                                  tr, true, stack, nn, nt);
+                                                  tr, true, stack, 0, nn, nt);
             else
-            {
-                // the closest-hit kernels' step: one node or one triangle
-                wl::TravState st;
-                wl::trav_init(st, tr, true);
-                for (;;)
-                {
-                    const bool tri = st.trimask != 0;
-                    if (wl::trav_step_one<1>(h->bvh.nodes.data(), h->bvh.tris.data(), tr, st,
-                                             stack))
-                        break;
-                    if (tri)
-                        ++nt;
-                    else
-                        ++nn;
-                }
-                wl::trav_finish(st.res);
-                res = st.res;
-            }
+                res = wl::trav_run<false, true, 1>(h->bvh.nodes.data(), h->bvh.tris.data(),
+                                                   tr, true, stack, 0, nn, nt);
             float *o = hits + 4 * (size_t)i;
             o[0] = res.t;
             std::memcpy(&o[1], &res.prim, 4);

@@ -174,8 +174,8 @@ void k_extend(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs
     auto load = [&](uint32_t i, TravRay &r) { load_eps(i, r, eps); };
     auto store = [&](uint32_t i, const TravResult &h) { store_hit_nt(B.hits, i, h); };
     if constexpr (MULTI) // S.nodes / S.tris: the arena of the requests' BVHs
-        trav_persistent<false, kPtBlock, false, true, false, 8, 20>(
-            S.nodes, S.tris, count, stack + threadIdx.x,
+        trav_persistent<false, kPtBlock, STACK != 16, true, false, 8, 20>(
+            S.nodes, S.tris, count, stack,
             [&](uint32_t i, TravRay &r, uint32_t &root) {
                 const PtReq &rq = reqs[qreq[i]];
                 root = rq.root;
@@ -183,8 +183,9 @@ void k_extend(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs
             },
             store);
     else
-        trav_persistent<false, kPtBlock, false, false, false, 0, 20>(
-            S.nodes, S.tris, count, stack + threadIdx.x, load, store,
+        trav_persistent<false, kPtBlock, STACK != 16, false, false, 0, 20, 0, 256,
+                        pt_top_nodes<STACK, false>() != 0>(
+            S.nodes, S.tris, count, stack, load, store,
             reinterpret_cast<const WlBvh8Node *>(top), ntop);
 }
 
@@ -212,8 +213,9 @@ void k_extend_first(PtParams P, PtScene S, PtBuffers B)
         trav_setup(r, o.x, o.y, o.z, d.x, d.y, d.z, P.epsilon, 1e30f);
     };
     auto store = [&](uint32_t i, const TravResult &h) { store_hit_nt(B.hits, i, h); };
-    trav_persistent<false, kPtBlock, false, false, false, 0, 20>(
-        S.nodes, S.tris, count, stack + threadIdx.x, load, store,
+    trav_persistent<false, kPtBlock, STACK != 16, false, false, 0, 20, 0, 256,
+                    pt_top_nodes<STACK, false>() != 0>(
+        S.nodes, S.tris, count, stack, load, store,
         reinterpret_cast<const WlBvh8Node *>(top), ntop);
 }
 
@@ -923,16 +925,17 @@ void k_shadow(PtScene S, PtBuffers B, const PtReq *__restrict__ reqs)
         }
     };
     if constexpr (MULTI) // S.nodes / S.tris: the arena of the requests' BVHs
-        trav_persistent<true, kPtBlock, false, true, false, 8, 20>(
-            S.nodes, S.tris, count, stack + threadIdx.x,
+        trav_persistent<true, kPtBlock, STACK != 16, true, false, 8, 20>(
+            S.nodes, S.tris, count, stack,
             [&](uint32_t i, TravRay &r, uint32_t &root) {
                 root = B.sreq[i];
                 load(i, r);
             },
             add);
     else
-        trav_persistent<true, kPtBlock, false, false, false, 2, 20>(
-            S.nodes, S.tris, count, stack + threadIdx.x, load, add,
+        trav_persistent<true, kPtBlock, STACK != 16, false, false, 2, 20, 0, 256,
+                        pt_top_nodes<STACK, false>() != 0>(
+            S.nodes, S.tris, count, stack, load, add,
             reinterpret_cast<const WlBvh8Node *>(top), ntop);
 }
 
@@ -1197,8 +1200,9 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B,
 {
     const uint32_t npaths = P.npix * P.nsamples;
     const uint32_t blocks_all = (npaths + kPtBlock - 1) / kPtBlock;
-    // a BVH at most 16 deep needs at most 15 stack entries per lane
-    const bool shallow = S.bvh_depth <= 16;
+    // a BVH at most 16 deep needs at most 15 stack entries per lane; those
+    // kernels also address nodes and triangles with 32-bit offsets
+    const bool shallow = S.bvh_depth <= 16 && wl_bvh8_narrow(S.num_nodes, S.num_tris);
     // persistent traversal grids: the workgroups that fit the GPU at once
     static int occ16 = 0, occ32 = 0, occf16 = 0, occf32 = 0;
     if (!occ16)

@@ -67,8 +67,9 @@ void k_trace_closest_p(
     __shared__ uint4 top[8 * (top_nodes<STACK>() ? top_nodes<STACK>() : 1)];
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
-    trav_persistent<false, kTraceBlock, false, false, true, 0, kRefillLanes, 2, kTraceChunk>(
-        nodes, tris, n, stack + threadIdx.x,
+    trav_persistent<false, kTraceBlock, STACK != 16, false, true, 0, kRefillLanes, 2,
+                    kTraceChunk, top_nodes<STACK>() != 0>(
+        nodes, tris, n, stack,
         [&](uint32_t i, TravRay &r) { load_ray(rays, i, r); },
         [&](uint32_t i, const TravResult &h) { store_hit_nt(hits, i, h); },
         reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u, sched,
@@ -85,8 +86,9 @@ void k_trace_any_p(const WlBvh8Node *__restrict__ nodes, const WlTriRecord *__re
     __shared__ uint4 top[8 * (top_nodes<STACK>() ? top_nodes<STACK>() : 1)];
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
-    trav_persistent<true, kTraceBlock, false, false, true, 0, kRefillLanes, 2, kTraceChunk>(
-        nodes, tris, n, stack + threadIdx.x,
+    trav_persistent<true, kTraceBlock, STACK != 16, false, true, 0, kRefillLanes, 2,
+                    kTraceChunk, top_nodes<STACK>() != 0>(
+        nodes, tris, n, stack,
         [&](uint32_t i, TravRay &r) { load_ray(rays, i, r); },
         [&](uint32_t i, const TravResult &h) {
             if (h.prim != WL_INVALID)
@@ -112,8 +114,8 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_closest_counted(
     else
         trav_setup(r, 0, 0, 0, 1, 0, 0, 0, 0);
     uint32_t nn = 0, nt = 0;
-    TravResult h = trav_run<false, true, kTraceBlock>(nodes, tris, r, active,
-                                                     stack + threadIdx.x, nn, nt);
+    TravResult h = trav_run<false, true, kTraceBlock>(nodes, tris, r, active, stack,
+                                                     threadIdx.x, nn, nt);
     if (active)
     {
         reinterpret_cast<float4 *>(hits)[rid] =
@@ -131,7 +133,11 @@ __global__ void k_zero_words(uint32_t *words, uint32_t nwords)
         words[k] = 0;
 }
 
-static inline bool shallow(const wl_accel_s *a) { return a->info.depth <= 16; }
+// The 16-entry stack kernels: also 32-bit node and triangle offsets.
+static inline bool shallow(const wl_accel_s *a)
+{
+    return a->info.depth <= 16 && wl_bvh8_narrow(a->num_nodes, a->num_tri_records);
+}
 
 // Persistent grid: the workgroups that fit the GPU at once (the launch then
 // takes at most one workgroup per 256 rays).

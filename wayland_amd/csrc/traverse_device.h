@@ -9,18 +9,18 @@
 // conservative).
 //
 // Traversal state per lane: a current node group (child_base, hit mask in
-// key space), a triangle mask of the node just visited, and an LDS stack of
-// 4-byte group entries, WL_BVH8_STACK_DEPTH deep, laid out [depth][lane] so
-// the 64 lanes of a wave touch 64 consecutive words.
+// key space), the pending triangles of the node visited last, and an LDS
+// stack of 4-byte group entries, WL_BVH8_STACK_DEPTH deep, laid out
+// [depth][lane] so the 64 lanes of a wave touch 64 consecutive words.
 //
-// Two step shapes share the node and triangle code.  trav_step visits a node
-// and then tests all of its triangles (the instrumented kernel and the
-// one-ray-to-completion loop).  The persistent kernels, closest and any-hit,
-// step with trav_step_one instead: a lane tests one pending triangle per
-// step, and visits its next node once none is pending (in the same step as
-// its last triangle), so lanes with several triangles do not hold the whole
-// wave in a triangle loop.  Both visit the same nodes and test the same
-// triangles in the same order, so the results are the same.
+// A ray alternates two steps: trav_node (the next node of the group: eight
+// child boxes) while no triangle is pending, and trav_tri (one pending
+// triangle).  It is finished once its group and its pending triangles are
+// both empty.  trav_run takes one ray to completion (the instrumented kernel,
+// the example program, the CPU emulation); the persistent kernels
+// (traverse_persistent.h) choose per wave which of the two steps to run.  A
+// ray's own steps come in the same order either way, so the results are the
+// same.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -49,15 +49,12 @@ struct TravRay
     float tmin, tmax;
     float inv[3];
     float Sx, Sy, Sz;
-    // bits 0-2: bit k set for d_k < 0 (slot ^ neg ^ 7 = visit order key, near
-    // first); bits 3-8: kx | ky << 2 | kz << 4 (the triangle test's axis order)
+    // bits 0-2: visit key, bit k clear for d_k < 0 (slots in increasing
+    // slot ^ key order are near first); bits 4-6: bit 4 + k set for d_k < 0
+    // (16 x bit = the byte offset of the near plane in its lo / hi pair);
+    // bits 8, 9: the largest component is x, y (else z); bit 31: it is < 0
     uint32_t code;
 };
-
-WL_HD float sel3(int k, float a, float b, float c)
-{
-    return k == 0 ? a : (k == 1 ? b : c);
-}
 
 WL_HD void trav_setup(TravRay &r, float ox, float oy,
                                            float oz, float dx, float dy,
@@ -69,24 +66,18 @@ WL_HD void trav_setup(TravRay &r, float ox, float oy,
     r.tmin = tmin;
     r.tmax = tmax;
     float d[3] = { dx, dy, dz };
-    int kz = 0;
-    if (fabsf(d[1]) > fabsf(d[kz]))
-        kz = 1;
-    if (fabsf(d[2]) > fabsf(d[kz]))
-        kz = 2;
-    int kx = kz + 1 == 3 ? 0 : kz + 1;
-    int ky = kx + 1 == 3 ? 0 : kx + 1;
-    float dkz = sel3(kz, dx, dy, dz);
-    if (dkz < 0.0f)
-    {
-        int t = kx;
-        kx = ky;
-        ky = t;
-    }
-    const uint32_t kxyz = (uint32_t)kx | (uint32_t)ky << 2 | (uint32_t)kz << 4;
-    r.Sx = sel3(kx, dx, dy, dz) / dkz;
-    r.Sy = sel3(ky, dx, dy, dz) / dkz;
+    // axes (kx, ky, kz), kz the largest component of d: y z x, z x y or x y z
+    // (the winding swap of kx and ky for d[kz] < 0 is tri_test's sign)
+    const bool cy = fabsf(dy) > fabsf(dx);
+    const float dm = cy ? dy : dx;
+    const bool cz = fabsf(dz) > fabsf(dm);
+    const float dkz = cz ? dz : dm;
+    const float dkx = cz ? dx : (cy ? dz : dy);
+    const float dky = cz ? dy : (cy ? dx : dz);
+    r.Sx = dkx / dkz;
+    r.Sy = dky / dkz;
     r.Sz = 1.0f / dkz;
+    const uint32_t axis = (cz ? 0u : (cy ? 2u << 8 : 1u << 8)) | (dkz < 0.0f ? 1u << 31 : 0u);
     uint32_t neg = 0;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -104,7 +95,7 @@ WL_HD void trav_setup(TravRay &r, float ox, float oy,
         if (r.inv[i] < 0.0f)
             neg |= 1u << i;
     }
-    r.code = neg | kxyz << 3;
+    r.code = (neg ^ 7u) | neg << 4 | axis;
 }
 
 // Watertight test; returns true and (t, b1, b2) for tmin <= t <= tmax.
@@ -113,21 +104,29 @@ WL_HD bool tri_test(const TravRay &r, const float4 w0,
                                          float tmax, float &t_out, float &b1_out,
                                          float &b2_out)
 {
-    // A = v0 - o, B = v1 - o, C = v2 - o, components permuted (kx, ky, kz)
-    const int kx = (int)((r.code >> 3) & 3u), ky = (int)((r.code >> 5) & 3u),
-              kz = (int)((r.code >> 7) & 3u);
-    // subtract in world axes, then permute (the same differences, fewer selects)
+    // A = v0 - o, B = v1 - o, C = v2 - o, subtracted in world axes, then the
+    // components permuted to (kx, ky, kz)
+    const bool zx = (r.code & 1u << 8) != 0, zy = (r.code & 2u << 8) != 0;
     const float A0 = w0.x - r.o[0], A1 = w0.y - r.o[1], A2 = w0.z - r.o[2];
     const float B0 = w0.w - r.o[0], B1 = w1.x - r.o[1], B2 = w1.y - r.o[2];
     const float C0 = w1.z - r.o[0], C1 = w1.w - r.o[1], C2 = w2.x - r.o[2];
-    const float Akx = sel3(kx, A0, A1, A2), Aky = sel3(ky, A0, A1, A2), Akz = sel3(kz, A0, A1, A2);
-    const float Bkx = sel3(kx, B0, B1, B2), Bky = sel3(ky, B0, B1, B2), Bkz = sel3(kz, B0, B1, B2);
-    const float Ckx = sel3(kx, C0, C1, C2), Cky = sel3(ky, C0, C1, C2), Ckz = sel3(kz, C0, C1, C2);
-    const float Ax = Akx - r.Sx * Akz;
+    const float Akx = zx ? A1 : (zy ? A2 : A0), Aky = zx ? A2 : (zy ? A0 : A1),
+                Akz = zx ? A0 : (zy ? A1 : A2);
+    const float Bkx = zx ? B1 : (zy ? B2 : B0), Bky = zx ? B2 : (zy ? B0 : B1),
+                Bkz = zx ? B0 : (zy ? B1 : B2);
+    const float Ckx = zx ? C1 : (zy ? C2 : C0), Cky = zx ? C2 : (zy ? C0 : C1),
+                Ckz = zx ? C0 : (zy ? C1 : C2);
+    // The published test swaps kx and ky where d[kz] < 0, which turns each
+    // product pair below round: U = Cx By - Cy Bx becomes Cy Bx - Cx By.
+    // Flipping the sign of the three x components gives exactly that,
+    // signed zeros included, for three instructions instead of six more
+    // selection conditions.
+    auto flip = [&](float x) { return wl_u2f(wl_f2u(x) ^ (r.code & 0x80000000u)); };
+    const float Ax = flip(Akx - r.Sx * Akz);
     const float Ay = Aky - r.Sy * Akz;
-    const float Bx = Bkx - r.Sx * Bkz;
+    const float Bx = flip(Bkx - r.Sx * Bkz);
     const float By = Bky - r.Sy * Bkz;
-    const float Cx = Ckx - r.Sx * Ckz;
+    const float Cx = flip(Ckx - r.Sx * Ckz);
     const float Cy = Cky - r.Sy * Ckz;
     float U = Cx * By - Cy * Bx;
     float V = Ax * Cy - Ay * Cx;
@@ -179,19 +178,20 @@ struct TravResult
     uint32_t input, local; // build input and input-local index (AUX only)
 };
 
-// Resumable traversal state of one ray: the current node group (child_base,
-// hit mask in key space), the node to visit next, the stack depth and the
-// best hit so far.  The stack itself lives in LDS.
+// Resumable traversal state of one ray: the current node group, the stack
+// position, the pending triangles and the best hit so far.  The stack itself
+// lives in LDS: sp indexes it as lane + BLOCK x depth.
 struct TravState
 {
     TravResult res;
-    uint32_t grp_base, grp_mask, node;
-    int sp;
-    bool visit;
-    uint32_t trimask, tri_base; // pending triangles (trav_step_one)
+    uint32_t grp_base, grp_mask;
+    uint32_t sp;
+    uint32_t trimask, trivalid, tri_base; // pending triangles (see NodeHits)
 };
 
-WL_HD void trav_init(TravState &st, const TravRay &r, bool active)
+// Starts (active) at node `root`, the only member of the first group.
+WL_HD void trav_init(TravState &st, const TravRay &r, bool active, uint32_t lane,
+                     uint32_t root = 0)
 {
     st.res.t = r.tmax;
     st.res.prim = WL_INVALID;
@@ -199,53 +199,67 @@ WL_HD void trav_init(TravState &st, const TravRay &r, bool active)
     st.res.b2 = 0.0f;
     st.res.input = WL_INVALID;
     st.res.local = WL_INVALID;
-    st.sp = 0;
-    st.grp_base = 0;
-    st.grp_mask = 0;
-    st.node = 0;
-    st.visit = active;
+    st.sp = lane;
+    st.grp_base = root;
+    st.grp_mask = active ? 1u << (r.code & 7u) : 0u; // slot 0's key
     st.trimask = 0;
+    st.trivalid = 0;
     st.tri_base = 0;
 }
 
 // The eight child boxes of `node` against [tmin, min(t_best, ...)]: inner
-// hits in key space (bit s ^ neg ^ 7), and the triangle bits of the hit leaves.
+// hits in key space (bit s ^ key), and the triangles of the hit leaves: bit
+// 4 s + i for triangle i of leaf slot s, whose record is tri_base + the number
+// of trivalid bits below it.
 struct NodeHits
 {
-    uint32_t child_base, tri_base, inner, trimask;
+    uint32_t child_base, tri_base, inner, trimask, trivalid;
 };
 
-// top (optional): a copy of nodes [0, ntop) in LDS, read instead of memory
-// for those nodes (the builder lays the top levels out first).
+// TOP: nodes [0, ntop) are also held in LDS at `top`, read there instead of
+// from memory (the builder lays the top levels out first).  WIDE: 64-bit
+// addresses per lane; otherwise a byte offset of 32 bits from the uniform base
+// (wl_bvh8_narrow), which the LDS path shares.
+template <bool TOP, bool WIDE>
 WL_HD NodeHits node_visit(const WlBvh8Node *__restrict__ nodes, uint32_t node,
                           const TravRay &r, float t_best, const WlBvh8Node *top = nullptr,
                           uint32_t ntop = 0)
 {
-    // near/far quantised planes chosen by the ray's direction signs
-    // (lo planes at words 2-4, hi planes at 5-7: a per-lane offset picks them)
-    const uint32_t nx = r.code & 1u, ny = (r.code >> 1) & 1u, nz = (r.code >> 2) & 1u;
+    // near/far quantised planes chosen by the ray's direction signs: the lo and
+    // hi planes of an axis are a 16-byte aligned pair, so a per-lane bit of the
+    // address picks one and its complement the other
+    const uint32_t at = WIDE ? 0u : node << 7;
+    const uint32_t nx = at | (r.code & 16u), ny = at | ((r.code >> 1) & 16u),
+                   nz = at | ((r.code >> 2) & 16u);
     uint4 h0, h1, nqx, fqx, nqy, fqy, nqz, fqz;
-    auto fetch = [&](auto np) {
-        h0 = np[0];
-        h1 = np[1];
-        nqx = np[2 + 3 * nx];
-        fqx = np[5 - 3 * nx];
-        nqy = np[3 + 3 * ny];
-        fqy = np[6 - 3 * ny];
-        nqz = np[4 + 3 * nz];
-        fqz = np[7 - 3 * nz];
+    auto fetch = [&](auto base, auto as) {
+        auto ld = [&](uint32_t off, uint32_t imm) { return *as(base + off + imm); };
+        h0 = ld(at, 0);
+        h1 = ld(at, 16);
+        nqx = ld(nx, 32);
+        fqx = ld(nx ^ 16u, 32);
+        nqy = ld(ny, 64);
+        fqy = ld(ny ^ 16u, 64);
+        nqz = ld(nz, 96);
+        fqz = ld(nz ^ 16u, 96);
     };
 #if defined(__HIP_DEVICE_COMPILE__)
     // distinct address spaces keep the two paths apart: LDS reads for the
     // cached nodes, global loads for the rest (not one generic-pointer load)
     typedef __attribute__((address_space(3))) const uint4 lds_u4;
     typedef __attribute__((address_space(1))) const uint4 glb_u4;
-    if (node < ntop)
-        fetch((lds_u4 *)(reinterpret_cast<const uint4 *>(top + node)));
+    typedef __attribute__((address_space(3))) const char lds_c;
+    typedef __attribute__((address_space(1))) const char glb_c;
+    auto as_lds = [](lds_c *p) { return (lds_u4 *)p; };
+    auto as_glb = [](glb_c *p) { return (glb_u4 *)p; };
+    static_assert(!(TOP && WIDE), "the LDS copy is read with 32-bit offsets");
+    if (TOP && node < ntop)
+        fetch((lds_c *)reinterpret_cast<const char *>(top), as_lds);
     else
-        fetch((glb_u4 *)(reinterpret_cast<const uint4 *>(nodes + node)));
+        fetch((glb_c *)reinterpret_cast<const char *>(WIDE ? nodes + node : nodes), as_glb);
 #else
-    fetch(reinterpret_cast<const uint4 *>(node < ntop ? top + node : nodes + node));
+    auto as_any = [](const char *p) { return reinterpret_cast<const uint4 *>(p); };
+    fetch(reinterpret_cast<const char *>(WIDE ? nodes + node : nodes), as_any);
 #endif
     const float px = wl_u2f(h0.x), py = wl_u2f(h0.y), pz = wl_u2f(h0.z);
     const uint32_t ew = h0.w;
@@ -253,7 +267,6 @@ WL_HD NodeHits node_visit(const WlBvh8Node *__restrict__ nodes, uint32_t node,
     const float sy = wl_u2f(((ew >> 8) & 0xFFu) << 23);
     const float sz = wl_u2f(((ew >> 16) & 0xFFu) << 23);
     const uint32_t imask = ew >> 24;
-    const uint32_t meta_lo = h1.z, meta_hi = h1.w;
     // per-axis plane parameters: t = q * sinv + adj
     const float ax = (px - r.o[0]) * r.inv[0];
     const float ay = (py - r.o[1]) * r.inv[1];
@@ -300,41 +313,36 @@ WL_HD NodeHits node_visit(const WlBvh8Node *__restrict__ nodes, uint32_t node,
     NodeHits h;
     h.child_base = h1.x;
     h.tri_base = h1.y;
-    // inner hits to key space: bit s -> bit s ^ k, k = neg ^ 7 (xor of a 3-bit index
-    // = swaps of single bits, pairs and nibbles)
+    h.trivalid = h1.z;
+    // hit leaves: every slot's bit to a nibble, the nibbles' valid triangles
+    uint32_t x = hitmask;
+    x = (x | x << 12) & 0x000F000Fu;
+    x = (x | x << 6) & 0x03030303u;
+    x = (x | x << 3) & 0x11111111u;
+    h.trimask = ((x << 4) - x) & h.trivalid;
+    // inner hits to key space: bit s -> bit s ^ k (xor of a 3-bit index =
+    // swaps of single bits, pairs and nibbles)
     uint32_t m = hitmask & imask;
-    const uint32_t k = (r.code & 7u) ^ 7u;
+    const uint32_t k = r.code;
     m = (k & 1u) ? (((m & 0x55u) << 1) | ((m >> 1) & 0x55u)) : m;
     m = (k & 2u) ? (((m & 0x33u) << 2) | ((m >> 2) & 0x33u)) : m;
     m = (k & 4u) ? (((m & 0x0Fu) << 4) | ((m >> 4) & 0x0Fu)) : m;
     h.inner = m;
-    // hit leaves: their triangle ranges (few per node, so a loop)
-    uint32_t trimask = 0;
-    uint32_t leaf = hitmask & ~imask;
-    while (leaf)
-    {
-        const uint32_t s = __builtin_ctz(leaf);
-        leaf &= leaf - 1u;
-        const uint32_t mm = ((s < 4 ? meta_lo : meta_hi) >> (8 * (s & 3))) & 0xFFu;
-        // 0xFF marks an empty slot (its inverted box can still pass the
-        // padded test on a tiny node)
-        if (mm != 0xFFu)
-        {
-            const uint32_t off = mm >> 2, cnt = (mm & 3u) + 1u;
-            trimask |= ((1u << cnt) - 1u) << off;
-        }
-    }
-    h.trimask = trimask;
     return h;
 }
 
-// Test triangle tri_base + i; keeps the closest hit (ties to the smaller
+// Test triangle record i; keeps the closest hit (ties to the smaller
 // primitive id).  Returns true for an accepted hit.
-template <bool ANY, bool AUX>
-WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t tri_base, uint32_t i,
-                     const TravRay &r, TravState &st)
+template <bool ANY, bool AUX, bool WIDE>
+WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t i, const TravRay &r,
+                     TravState &st)
 {
-    const float4 *tp = reinterpret_cast<const float4 *>(tris + tri_base + i);
+    const float4 *tp;
+    if (WIDE)
+        tp = reinterpret_cast<const float4 *>(tris + i);
+    else // 48 i as shifts: the full 32-bit multiply is a quarter-rate instruction
+        tp = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(tris) +
+                                              (((i << 1) + i) << 4));
     const float4 w0 = tp[0], w1 = tp[1], w2 = tp[2];
     float t, b1, b2;
     // the best hit so far bounds t: closest hit keeps only t <= res.t (ties to
@@ -371,108 +379,64 @@ WL_HD uint32_t dyn_xcd_chunks(uint32_t n, uint32_t xcd, uint32_t chunk)
     return (hi - lo + chunk - 1u) / chunk;
 }
 
-// Next node from the current group, else from the stack; false when none.
-template <int BLOCK>
-WL_HD bool next_node(const TravRay &r, TravState &st, uint32_t *lds_stack_lane)
-{
-    if (st.grp_mask == 0)
-    {
-        if (st.sp == 0)
-            return false;
-        --st.sp;
-        const uint32_t e = lds_stack_lane[st.sp * BLOCK];
-        st.grp_base = (e >> 8) << 3;
-        st.grp_mask = e & 0xFFu;
-    }
-    const uint32_t pos = __builtin_ctz(st.grp_mask);
-    st.grp_mask &= st.grp_mask - 1u;
-    st.node = st.grp_base + (pos ^ (r.code & 7u) ^ 7u);
-    if (st.grp_mask)
-    {
-        lds_stack_lane[st.sp * BLOCK] = ((st.grp_base >> 3) << 8) | st.grp_mask;
-        ++st.sp;
-    }
-    return true;
-}
+// Whether the ray has nothing left to do.
+WL_HD bool trav_done(const TravState &st) { return (st.grp_mask | st.trimask) == 0; }
 
-// One step: visit the pending node (8 child boxes), test the triangles of its
-// leaves, then pick the next node from the current group or the stack.
-// Returns true when the ray is finished (stack empty, or first hit for ANY).
-template <bool ANY, bool COUNT, int BLOCK, bool AUX = false>
-WL_HD bool trav_step(const WlBvh8Node *__restrict__ nodes,
-                     const WlTriRecord *__restrict__ tris, const TravRay &r,
-                     TravState &st, uint32_t *lds_stack_lane, uint32_t &n_nodes,
-                     uint32_t &n_tris, const WlBvh8Node *top = nullptr, uint32_t ntop = 0)
+// One node: the next of the current group (which must not be empty; no
+// triangle may be pending).  Its hit children become the group, with what was
+// left of the old one pushed; without any, the group goes on, and once it is
+// used up the stack's top is popped.  So the group is empty only when the
+// stack is, and a node without inner hits touches the stack at most once.
+template <int BLOCK, bool TOP = false, bool WIDE = true>
+WL_HD bool trav_node(const WlBvh8Node *__restrict__ nodes, const TravRay &r, TravState &st,
+                     uint32_t *lds_stack, const WlBvh8Node *top = nullptr, uint32_t ntop = 0)
 {
-    uint32_t trimask = 0, tri_base = 0;
-    if (st.visit)
+    const uint32_t pos = __builtin_ctz(st.grp_mask);
+    const uint32_t rest = st.grp_mask & (st.grp_mask - 1u);
+    const uint32_t node = st.grp_base + (pos ^ (r.code & 7u));
+    WL_TRAV_CHECK(node < wl_trav_nodes_bound, "node index");
+    const NodeHits h = node_visit<TOP, WIDE>(nodes, node, r, st.res.t, top, ntop);
+    st.trimask = h.trimask;
+    st.trivalid = h.trivalid;
+    st.tri_base = h.tri_base;
+    if (h.inner)
     {
-        WL_TRAV_CHECK(st.node < wl_trav_nodes_bound, "node index");
-        const NodeHits h = node_visit(nodes, st.node, r, st.res.t, top, ntop);
-        if (COUNT)
-            ++n_nodes;
-        trimask = h.trimask;
-        tri_base = h.tri_base;
+        if (rest)
+        {
+            WL_TRAV_CHECK(st.sp < WL_BVH8_STACK_DEPTH * BLOCK, "stack depth");
+            lds_stack[st.sp] = st.grp_base << 5 | rest; // base / 8 in the upper 24 bits
+            st.sp += BLOCK;
+        }
         st.grp_base = h.child_base;
         st.grp_mask = h.inner;
-        st.visit = false;
     }
-    // ---- triangles of the node just visited
-    while (trimask)
+    else
     {
-        const uint32_t i = __builtin_ctz(trimask);
-        trimask &= trimask - 1u;
-        WL_TRAV_CHECK((size_t)tri_base + i < wl_trav_tris_bound, "triangle index");
-        if (COUNT)
-            ++n_tris;
-        if (tri_visit<ANY, AUX>(tris, tri_base, i, r, st) && ANY)
-            return true;
+        st.grp_mask = rest;
+        if (rest == 0 && st.sp >= BLOCK)
+        {
+            st.sp -= BLOCK;
+            const uint32_t e = lds_stack[st.sp];
+            st.grp_base = e >> 5 & ~7u;
+            st.grp_mask = e & 0xFFu;
+        }
     }
-    // ---- next node: from the current group, else from the stack
-    WL_TRAV_CHECK((st.grp_mask & (st.grp_mask - 1u)) == 0u || st.sp < WL_BVH8_STACK_DEPTH,
-                  "stack depth");
-    if (!next_node<BLOCK>(r, st, lds_stack_lane))
-        return true;
-    st.visit = true;
     return false;
 }
 
-// Persistent-kernel step: one pending triangle, then, once no triangle is
-// pending, one node (the next from the group or the stack, then its box
-// test).  A lane that tests its node's last triangle goes on to the next node
-// in the same step: the order of tests is that of doing the two one after the
-// other, and the wave's node branch runs with more of its lanes.  Returns
-// true when the ray is finished (no node left, or with ANY its first hit).
-template <int BLOCK, bool AUX = false, bool ANY = false>
-WL_HD bool trav_step_one(const WlBvh8Node *__restrict__ nodes,
-                         const WlTriRecord *__restrict__ tris, const TravRay &r,
-                         TravState &st, uint32_t *lds_stack_lane,
-                         const WlBvh8Node *top = nullptr, uint32_t ntop = 0)
+// One pending triangle (there must be one).  A hit of an any-hit ray ends it.
+template <bool ANY, bool AUX = false, bool WIDE = true>
+WL_HD bool trav_tri(const WlTriRecord *__restrict__ tris, const TravRay &r, TravState &st)
 {
-    if (st.trimask)
+    const uint32_t b = __builtin_ctz(st.trimask);
+    st.trimask &= st.trimask - 1u;
+    const uint32_t i = st.tri_base + (uint32_t)__builtin_popcount(st.trivalid & ((1u << b) - 1u));
+    WL_TRAV_CHECK(i < wl_trav_tris_bound, "triangle index");
+    if (tri_visit<ANY, AUX, WIDE>(tris, i, r, st) && ANY)
     {
-        const uint32_t i = __builtin_ctz(st.trimask);
-        st.trimask &= st.trimask - 1u;
-        WL_TRAV_CHECK((size_t)st.tri_base + i < wl_trav_tris_bound, "triangle index");
-        if (tri_visit<ANY, AUX>(tris, st.tri_base, i, r, st) && ANY)
-            return true;
-        if (st.trimask)
-            return false;
+        st.trimask = 0;
+        st.grp_mask = 0;
     }
-    if (!st.visit)
-    {
-        WL_TRAV_CHECK((st.grp_mask & (st.grp_mask - 1u)) == 0u || st.sp < WL_BVH8_STACK_DEPTH,
-                  "stack depth");
-        if (!next_node<BLOCK>(r, st, lds_stack_lane))
-            return true;
-    }
-    WL_TRAV_CHECK(st.node < wl_trav_nodes_bound, "node index");
-    const NodeHits h = node_visit(nodes, st.node, r, st.res.t, top, ntop);
-    st.trimask = h.trimask;
-    st.tri_base = h.tri_base;
-    st.grp_base = h.child_base;
-    st.grp_mask = h.inner;
-    st.visit = false;
     return false;
 }
 
@@ -482,20 +446,29 @@ WL_HD void trav_finish(TravResult &res)
         res.t = wl_u2f(0x7F800000u); // +inf
 }
 
-// Traverse one ray to completion.
+// Traverse one ray to completion.  lane: the ray's first entry of the stack.
 template <bool ANY, bool COUNT, int BLOCK, bool AUX = false>
-WL_HD TravResult
-trav_run(const WlBvh8Node *__restrict__ nodes,
-         const WlTriRecord *__restrict__ tris, const TravRay &r, bool active,
-         uint32_t *lds_stack_lane, uint32_t &n_nodes, uint32_t &n_tris)
+WL_HD TravResult trav_run(const WlBvh8Node *__restrict__ nodes,
+                          const WlTriRecord *__restrict__ tris, const TravRay &r, bool active,
+                          uint32_t *lds_stack, uint32_t lane, uint32_t &n_nodes,
+                          uint32_t &n_tris)
 {
     TravState st;
-    trav_init(st, r, active);
-    if (active)
-        while (!trav_step<ANY, COUNT, BLOCK, AUX>(nodes, tris, r, st, lds_stack_lane,
-                                                 n_nodes, n_tris))
+    trav_init(st, r, active, lane);
+    while (st.grp_mask)
+    {
+        if (trav_node<BLOCK>(nodes, r, st, lds_stack))
+            break; // CPU emulation only: an index out of range
+        if (COUNT)
+            ++n_nodes;
+        while (st.trimask)
         {
+            if (COUNT)
+                ++n_tris;
+            if (trav_tri<ANY, AUX>(tris, r, st))
+                break;
         }
+    }
     trav_finish(st.res);
     return st.res;
 }

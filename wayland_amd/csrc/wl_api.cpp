@@ -215,15 +215,15 @@ static bool validate_bvh8(const wl::Bvh8Host &b, std::string *err)
                 }
                 queue.push_back((uint32_t)c);
             }
-            else if (n.meta[s] != 0xFF)
-            {
-                uint32_t off = n.meta[s] >> 2, cnt = (n.meta[s] & 3u) + 1u;
-                if (off + cnt > 32 || (size_t)n.tri_base + off + cnt > nt)
-                {
-                    *err = "BVH8 leaf triangle range out of range";
-                    return false;
-                }
-            }
+        }
+        uint32_t inner = 0; // the nibbles of inner slots
+        for (int s = 0; s < 8; ++s)
+            inner |= (n.imask & (1u << s)) ? 0xFu << (4 * s) : 0u;
+        if ((n.trivalid & inner) != 0 ||
+            (size_t)n.tri_base + (size_t)__builtin_popcount(n.trivalid) > nt)
+        {
+            *err = "BVH8 leaf triangle range out of range";
+            return false;
         }
     }
     return true;

@@ -56,6 +56,7 @@ struct PtScene
     const uint32_t *texels;
     uint32_t bvh_depth;
     uint32_t num_nodes; // BVH8 nodes (the top ones are copied to LDS by traversal)
+    uint32_t num_tris;  // triangle records
 };
 
 // One batch = pixels [pix0, pix0 + npix) x samples [frame0, frame0 + nsamples)
@@ -166,7 +167,7 @@ struct PtMultiLaunch
     const WlBvh8Node *nodes;
     const WlTriRecord *tris;
     uint32_t max_depth;  // bounces enqueued (maximum over the requests)
-    uint32_t stack16;    // every BVH at most 16 levels deep
+    uint32_t stack16;    // every BVH at most 16 levels deep, the arena within 32-bit offsets
     uint32_t capacity;   // paths the buffers hold
     uint32_t shade_blocks_per_cu;
 };

@@ -72,6 +72,7 @@ PtScene pt_scene_view(wl_scene s)
     S.texels = s->d_texels;
     S.bvh_depth = s->accel->info.depth;
     S.num_nodes = s->accel->num_nodes;
+    S.num_tris = s->accel->num_tri_records;
     return S;
 }
 

@@ -340,7 +340,7 @@ wl_status run_lane(wl_server s, const wl_serve_config &cfg, const wl_render_requ
     L.nodes = s->d_arena_nodes;
     L.tris = s->d_arena_tris;
     L.max_depth = max_depth;
-    L.stack16 = max_bvh <= 16 ? 1u : 0u;
+    L.stack16 = max_bvh <= 16 && wl_bvh8_narrow(arena_nodes, arena_tris) ? 1u : 0u;
     L.capacity = s->capacity;
     L.shade_blocks_per_cu = cfg.shade_blocks_per_cu;
 

@@ -133,7 +133,7 @@ typedef struct wl_hit
 
 /* wl_trace_closest and wl_trace_any hand the rays out to the GPU's waves at
  * run time from a small block of counters kept per stream (the context's):
- * the first trace on a stream allocates that block (256 bytes, freed with the
+ * the first trace on a stream allocates that block (2 KB, freed with the
  * context) and synchronises the device, so a caller that captures traces
  * into a graph makes one trace on that stream before capturing.  Traces on
  * one stream are ordered; traces on different streams share nothing. */

@@ -1,0 +1,84 @@
+"""The traversal kernels at the edges of their dispatch: the deep-BVH kernels
+(32-entry stack, 64-bit addresses), the change of the raw traces' chunk size
+and ray counts around a chunk and an XCD's share."""
+import numpy as np
+import pytest
+
+import oracle_bind as ob
+from wayland_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _deep_scene():
+    """Triangles shrinking by 0.55 each towards the origin: a BVH8 deeper than
+    the 16-entry stack's kernels take."""
+    rng = np.random.default_rng(1)
+    n = 160
+    s = (0.55 ** np.arange(n))[:, None, None]
+    t = ((rng.uniform(-1, 1, (n, 3, 3)) * 0.4 + np.array([1.0, 0.3, -0.2])) * s)
+    mesh = scenes.soup_mesh(t.astype(np.float32), scenes.matte_material((0.7, 0.6, 0.5)))
+    light = scenes.soup_mesh(np.float32([[[-2, 2.5, -2], [2, 2.5, -2], [2, 2.5, 2]],
+                                         [[-2, 2.5, -2], [2, 2.5, 2], [-2, 2.5, 2]]]),
+                             scenes.matte_material((0, 0, 0)))
+    light.light_L, light.two_sided = (4.0, 4.0, 4.0), True
+    cam = scenes.pinhole_camera([0.3, 0.2, 3.0], [0, 0, -1], [0, 1, 0], 40.0, 64, 48)
+    return scenes.Scene([mesh, light], cam, (0.2, 0.2, 0.2), "deep")
+
+
+def _hits(accel, rays_np):
+    import torch
+    import wayland_amd as wl
+    rays = torch.from_numpy(np.ascontiguousarray(rays_np)).cuda()
+    hits, bits = accel.trace_closest(rays), accel.trace_any(rays)
+    torch.cuda.synchronize()
+    return wl.hits_to_numpy(hits), wl.unpack_bits(bits, rays_np.shape[0])
+
+
+def _same(h, ref):
+    hit = ref["prim"] != 0xFFFFFFFF
+    assert np.array_equal(h["prim"], ref["prim"])
+    assert np.array_equal(h["t"].view(np.uint32), ref["t"].view(np.uint32))
+    for b in ("b1", "b2"):
+        assert np.array_equal(h[b][hit].view(np.uint32), ref[b][hit].view(np.uint32))
+
+
+def test_deep_bvh_traces_and_render(gpu_ctx):
+    import wayland_amd as wl
+    sc = _deep_scene()
+    accel = wl.Accel(gpu_ctx, sc)
+    assert accel.info()["depth"] > 16
+    print(f"case: deep BVH {accel.info()}", flush=True)
+    rng = np.random.default_rng(3)
+    rays = scenes.traversal_rays(20000, seed=3)
+    # half the rays aim at the origin, where the small triangles are
+    rays[:, 0:3] = rays[:, 0:3] * 3 - 1
+    aim = rng.uniform(-1, 1, (10000, 3)) * (0.55 ** rng.uniform(0, 60, 10000))[:, None]
+    rays[:10000, 4:7] = aim - rays[:10000, 0:3]
+    tris = sc.triangles()
+    h, occ = _hits(accel, rays)
+    _same(h, ob.closest_brute(tris, rays))
+    assert np.array_equal(occ, ob.any_brute(tris, rays))
+    pt, opt = wl.PathTracer(gpu_ctx, accel, sc), ob.OraclePT(sc)
+    g = pt.render_samples(wl.pt_config(64, 48, max_depth=8), 1).cpu().numpy()
+    o, _ = opt.render_frame(opt.config(64, 48, max_depth=8), 1)
+    err = np.abs(g - o) / np.maximum(np.abs(o), 1e-6)
+    assert (err.reshape(-1, 3).max(1) <= 1e-5).mean() >= 0.995
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 512, 513, 8 * 64 * 3 + 1,
+                               786_431, 786_432, 786_433, 1_000_003])
+def test_ray_counts_around_the_chunk_sizes(gpu_ctx, n):
+    """Chunks of 64 rays below 128 per resident wave (786,432 rays on 256 CUs
+    with 24 waves each), 128 from there on: every ray's result equals that of
+    the same ray in a trace of another length, and the oracle's."""
+    import wayland_amd as wl
+    print(f"case: {n} rays", flush=True)
+    sc = scenes.icosphere_scene(6, 3, seed=2)
+    accel = wl.Accel(gpu_ctx, sc)
+    rays = scenes.traversal_rays(n + 4096, seed=9)
+    h, occ = _hits(accel, rays[:n])
+    whole, occ_whole = _hits(accel, rays)
+    _same(h, whole[:n])
+    assert np.array_equal(occ, occ_whole[:n])
+    _same(h[::41], ob.OracleBVH(sc.triangles()).closest(rays[:n:41]))

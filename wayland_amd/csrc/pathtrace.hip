@@ -183,7 +183,7 @@ void k_extend(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs
             },
             store);
     else
-        trav_persistent<false, kPtBlock, STACK != 16, false, false, 0, 20, 0, 256,
+        trav_persistent<false, kPtBlock, STACK != 16, false, false, 0, 20, 0,
                         pt_top_nodes<STACK, false>() != 0>(
             S.nodes, S.tris, count, stack, load, store,
             reinterpret_cast<const WlBvh8Node *>(top), ntop);
@@ -213,7 +213,7 @@ void k_extend_first(PtParams P, PtScene S, PtBuffers B)
         trav_setup(r, o.x, o.y, o.z, d.x, d.y, d.z, P.epsilon, 1e30f);
     };
     auto store = [&](uint32_t i, const TravResult &h) { store_hit_nt(B.hits, i, h); };
-    trav_persistent<false, kPtBlock, STACK != 16, false, false, 0, 20, 0, 256,
+    trav_persistent<false, kPtBlock, STACK != 16, false, false, 0, 20, 0,
                     pt_top_nodes<STACK, false>() != 0>(
         S.nodes, S.tris, count, stack, load, store,
         reinterpret_cast<const WlBvh8Node *>(top), ntop);
@@ -933,7 +933,7 @@ void k_shadow(PtScene S, PtBuffers B, const PtReq *__restrict__ reqs)
             },
             add);
     else
-        trav_persistent<true, kPtBlock, STACK != 16, false, false, 2, 20, 0, 256,
+        trav_persistent<true, kPtBlock, STACK != 16, false, false, 2, 20, 0,
                         pt_top_nodes<STACK, false>() != 0>(
             S.nodes, S.tris, count, stack, load, add,
             reinterpret_cast<const WlBvh8Node *>(top), ntop);

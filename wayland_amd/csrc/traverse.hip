@@ -24,15 +24,20 @@ constexpr int kTraceBlock = 256;
 constexpr uint32_t kTopNodes = 73;
 
 // Chunk scheduling (trav_persistent's DYN = 2): chunks of this many rays,
-// taken at run time from one counter per XCD.  The static split it replaced
-// (interleaved chunks per wave) left the kernel waiting for its slowest
-// waves: 8.68-8.75 -> 9.32-9.41 Grays/s on 2^23 incoherent closest-hit rays.
-constexpr uint32_t kTraceChunk = 256;
+// taken at run time from one counter per XCD, each counter in a cache line of
+// its own and each chunk asked for one ahead.  2^23 rays, closest / any hit:
+// 64: 696 / 534 us, 96: 688 / 522, 128: 691 / 521, 256: 713 / 523, 512: 730 /
+// 524 (727 / 603 us with 256 and the eight counters in one line).  A launch
+// with fewer than 128 rays per resident wave takes 64, which fill one wave's
+// lanes: 100,003 rays 112 -> 65 us (16: 94, 32: 79, 128: 81 before the last
+// rays' both-steps rule of trav_persistent).
+constexpr uint32_t kTraceChunk = 128;
 
-// The chunk counters' values at launch, one per XCD.
+// The chunk counters' values at launch, one per XCD, and the launch's chunk.
 struct TraceSched
 {
     uint32_t base[8];
+    uint32_t chunk;
 };
 
 template <int STACK>
@@ -68,12 +73,12 @@ void k_trace_closest_p(
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
     trav_persistent<false, kTraceBlock, STACK != 16, false, true, 0, kRefillLanes, 2,
-                    kTraceChunk, top_nodes<STACK>() != 0>(
+                    top_nodes<STACK>() != 0>(
         nodes, tris, n, stack,
         [&](uint32_t i, TravRay &r) { load_ray(rays, i, r); },
         [&](uint32_t i, const TravResult &h) { store_hit_nt(hits, i, h); },
-        reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u, sched,
-        base.base[blockIdx.x % 8u]);
+        reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u,
+        sched + kSchedStride * (blockIdx.x % 8u), base.base[blockIdx.x % 8u], base.chunk);
 }
 
 template <int STACK>
@@ -87,15 +92,15 @@ void k_trace_any_p(const WlBvh8Node *__restrict__ nodes, const WlTriRecord *__re
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
     trav_persistent<true, kTraceBlock, STACK != 16, false, true, 0, kRefillLanes, 2,
-                    kTraceChunk, top_nodes<STACK>() != 0>(
+                    top_nodes<STACK>() != 0>(
         nodes, tris, n, stack,
         [&](uint32_t i, TravRay &r) { load_ray(rays, i, r); },
         [&](uint32_t i, const TravResult &h) {
             if (h.prim != WL_INVALID)
                 atomicOr(&bits[i >> 5], 1u << (i & 31u));
         },
-        reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u, sched,
-        base.base[blockIdx.x % 8u]);
+        reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u,
+        sched + kSchedStride * (blockIdx.x % 8u), base.base[blockIdx.x % 8u], base.chunk);
 }
 
 // Instrumented closest hit: one ray per lane, per-ray node/triangle counts.
@@ -152,24 +157,35 @@ static uint32_t persistent_grid(K kernel, uint32_t /*unused*/, int num_cus)
     return (uint32_t)(per_cu * std::max(1, num_cus));
 }
 
+// Rays per chunk of a launch of n rays on a GPU that holds `grid_cache`
+// workgroups at once.
+static uint32_t trace_chunk(uint32_t n, uint32_t grid_cache)
+{
+    const uint32_t waves = grid_cache * (kTraceBlock / 64);
+    return n / kTraceChunk < waves ? 64u : kTraceChunk;
+}
+
 // The counters' values for a launch over n rays, advanced past it.
-static TraceSched take_bases(wl_context_s::SchedBlock *sb, uint32_t n)
+static TraceSched take_bases(wl_context_s::SchedBlock *sb, uint32_t n, uint32_t chunk)
 {
     TraceSched t;
+    t.chunk = chunk;
     for (uint32_t x = 0; x < 8; ++x)
     {
         t.base[x] = sb->base[x];
-        sb->base[x] += dyn_xcd_chunks(n, x, kTraceChunk);
+        sb->base[x] += dyn_xcd_chunks(n, x, t.chunk);
     }
     return t;
 }
 
-// The persistent grid for n rays, rounded up to a multiple of 8 so that each
-// XCD's eighth of the rays has workgroups (chunk scheduling DYN = 2).
-static uint32_t xcd_grid(uint32_t grid_cache, uint32_t n)
+// The persistent grid for n rays in chunks of `chunk`, rounded up to a multiple
+// of 8 so that each XCD's eighth of the rays has workgroups (chunk scheduling
+// DYN = 2).
+static uint32_t xcd_grid(uint32_t grid_cache, uint32_t n, uint32_t chunk)
 {
+    const uint32_t per_block = chunk * (kTraceBlock / 64);
     const uint32_t g = (uint32_t)std::min<uint64_t>(
-        grid_cache, ((uint64_t)n + kTraceBlock - 1) / kTraceBlock);
+        grid_cache, ((uint64_t)n + per_block - 1) / per_block);
     return (g + 7u) & ~7u;
 }
 
@@ -184,13 +200,14 @@ static hipError_t closest_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t
         grid_cache = persistent_grid(k_trace_closest_p<STACK>, 0xFFFFFFFFu, a->ctx->num_cus);
         cus_cache = a->ctx->num_cus;
     }
-    const uint32_t grid = xcd_grid(grid_cache, n);
+    const uint32_t chunk = trace_chunk(n, grid_cache);
+    const uint32_t grid = xcd_grid(grid_cache, n, chunk);
     std::lock_guard<std::mutex> lock(a->ctx->sched_mu);
     wl_context_s::SchedBlock *sb = nullptr;
     const hipError_t e = sched_block(a->ctx, s, &sb);
     if (e != hipSuccess)
         return e;
-    const TraceSched base = take_bases(sb, n);
+    const TraceSched base = take_bases(sb, n, chunk);
     hipLaunchKernelGGL(k_trace_closest_p<STACK>, dim3(grid), dim3(kTraceBlock), 0, s,
                        a->d_nodes, a->d_tris, rays, n, hits,
                        std::min<uint32_t>(a->num_nodes, top_nodes<STACK>()), sb->dev, base);
@@ -208,13 +225,14 @@ static hipError_t any_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t n,
         grid_cache = persistent_grid(k_trace_any_p<STACK>, 0xFFFFFFFFu, a->ctx->num_cus);
         cus_cache = a->ctx->num_cus;
     }
-    const uint32_t grid = xcd_grid(grid_cache, n);
+    const uint32_t chunk = trace_chunk(n, grid_cache);
+    const uint32_t grid = xcd_grid(grid_cache, n, chunk);
     std::lock_guard<std::mutex> lock(a->ctx->sched_mu);
     wl_context_s::SchedBlock *sb = nullptr;
     const hipError_t e = sched_block(a->ctx, s, &sb);
     if (e != hipSuccess)
         return e;
-    const TraceSched base = take_bases(sb, n);
+    const TraceSched base = take_bases(sb, n, chunk);
     const uint32_t words = (n + 31) / 32;
     hipLaunchKernelGGL(k_zero_words, dim3(std::min<uint32_t>((words + 255) / 256, 4096)),
                        dim3(256), 0, s, bits, words);

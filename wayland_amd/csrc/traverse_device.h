@@ -43,6 +43,17 @@ namespace wl
 WL_HD float wl_u2f(uint32_t u) { return __builtin_bit_cast(float, u); }
 WL_HD uint32_t wl_f2u(float f) { return __builtin_bit_cast(uint32_t, f); }
 
+// Keeps the compiler from seeing through x: a multiplication written as shifts
+// and adds stays that (the 32-bit integer multiply is a quarter-rate
+// instruction).
+WL_HD uint32_t opaque(uint32_t x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(x));
+#endif
+    return x;
+}
+
 struct TravRay
 {
     float o[3];
@@ -319,7 +330,7 @@ WL_HD NodeHits node_visit(const WlBvh8Node *__restrict__ nodes, uint32_t node,
     x = (x | x << 12) & 0x000F000Fu;
     x = (x | x << 6) & 0x03030303u;
     x = (x | x << 3) & 0x11111111u;
-    h.trimask = ((x << 4) - x) & h.trivalid;
+    h.trimask = (opaque(x << 4) - x) & h.trivalid;
     // inner hits to key space: bit s -> bit s ^ k (xor of a 3-bit index =
     // swaps of single bits, pairs and nibbles)
     uint32_t m = hitmask & imask;
@@ -340,9 +351,11 @@ WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t i, const Tra
     const float4 *tp;
     if (WIDE)
         tp = reinterpret_cast<const float4 *>(tris + i);
-    else // 48 i as shifts: the full 32-bit multiply is a quarter-rate instruction
-        tp = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(tris) +
-                                              (((i << 1) + i) << 4));
+    else
+    {
+        const uint32_t i3 = opaque((i << 1) + i);
+        tp = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(tris) + (i3 << 4));
+    }
     const float4 w0 = tp[0], w1 = tp[1], w2 = tp[2];
     float t, b1, b2;
     // the best hit so far bounds t: closest hit keeps only t <= res.t (ties to

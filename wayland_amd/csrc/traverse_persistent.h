@@ -12,7 +12,9 @@
 // about 170 instructions, a triangle step about 120, whatever the number of
 // lanes in it), so a step waits until enough lanes need it: the triangle step
 // until kTriLanes hold a pending triangle, the node step until kNodeLanes can
-// take a node, unless nothing else can run.  Running both on every pass left
+// take a node, unless nothing else can run.  Once the wave's rays are used up
+// every pass runs both: the last rays' latency counts then, not the issue
+// slots.  Running both on every pass left
 // 9 lanes of 64 in the triangle step on the 2M-triangle soup, and 21 in the
 // node step on a 36-triangle box.  With the steps apart, 32-bit node offsets
 // and results handed out at the refill: 2^23 incoherent rays 842 -> 727 us
@@ -62,6 +64,15 @@ constexpr int kRefillLanes = 16;
 constexpr int kTriLanes = 16;
 constexpr int kNodeLanes = 24;
 
+// Number of lanes in m, kept in a scalar register (a compare of the 64-bit
+// count would go to the vector unit).
+__device__ __forceinline__ int lane_count(uint64_t m)
+{
+    int c = __popcll(m);
+    asm("" : "+s"(c));
+    return c;
+}
+
 __device__ __forceinline__ uint32_t lane_prefix(uint64_t m)
 {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
@@ -89,9 +100,9 @@ __device__ __forceinline__ uint32_t lane_prefix(uint64_t m)
 // coherent queues together.
 // top / ntop (optional): nodes [0, ntop) copied to LDS by the caller (see
 // node_visit).
-// DYN = 2: chunks of DCHUNK rays are handed out at run time instead, so a
+// DYN = 2: chunks of `chunk` rays are handed out at run time instead, so a
 // wave slowed by expensive rays takes fewer chunks.  One global counter per
-// XCD (`dyn`, 8 words): XCD x owns the x-th eighth of the rays, its waves
+// XCD (`dyn`, this XCD's): XCD x owns the x-th eighth of the rays, its waves
 // start on chunks 0 .. W-1 of that eighth (W waves per XCD; the grid is a
 // multiple of 8) and then take chunk W + (counter - base) each, base =
 // `dyn_base`, the counter's value at launch.  Every wave that had a chunk
@@ -99,15 +110,15 @@ __device__ __forceinline__ uint32_t lane_prefix(uint64_t m)
 // counter x by the eighth's chunk count: the host keeps the bases and nothing
 // is reset.
 template <bool ANY, int BLOCK, bool WIDE, bool ROOTED = false, bool XCDMAP = false,
-          uint32_t CHUNKS = 0, int REFILL = kRefillLanes, int DYN = 0,
-          uint32_t DCHUNK = 256, bool TOP = false, class Fetch, class Emit>
+          uint32_t CHUNKS = 0, int REFILL = kRefillLanes, int DYN = 0, bool TOP = false,
+          class Fetch, class Emit>
 __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ nodes,
                                                 const WlTriRecord *__restrict__ tris,
                                                 uint32_t n, uint32_t *stack,
                                                 Fetch fetch, Emit emit,
                                                 const WlBvh8Node *top = nullptr,
                                                 uint32_t ntop = 0, uint32_t *dyn = nullptr,
-                                                uint32_t dyn_base = 0)
+                                                uint32_t dyn_base = 0, uint32_t chunk = 0)
 {
     static_assert(BLOCK % 64 == 0, "whole waves only");
     constexpr uint32_t kNone = 0xFFFFFFFFu;
@@ -132,23 +143,20 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
     const uint32_t xhi = xlo + n8 < n ? xlo + n8 : n;
     const uint32_t wx = (blockIdx.x / 8u) * (BLOCK / 64) + wave_in_block;
     const uint32_t wavesx = (G / 8u) * (BLOCK / 64);
-    // the next chunk of the DYN schedule into [next, end)
-    auto take_chunk = [&](bool first) {
+    // DYN: chunk c of the XCD's eighth into [next, end); a wave that got one
+    // asks for its next at once (lane 0 holds the answer, `ahead`), so the
+    // atomic's latency passes behind the chunk's own rays
+    uint32_t ahead = 0;
+    auto take_chunk = [&](uint32_t c) {
         static_assert(DYN == 0 || DYN == 2, "DYN is 0 or 2");
-        uint32_t c = wx;
-        if (!first)
-        {
-            uint32_t k = 0;
-            if (__lane_id() == 0)
-                k = atomicAdd(dyn + xcd, 1u) - dyn_base;
-            c = wavesx + __builtin_amdgcn_readfirstlane(k);
-        }
-        const uint64_t s0 = xlo + (uint64_t)c * DCHUNK;
+        const uint64_t s0 = xlo + (uint64_t)c * chunk;
         next = (uint32_t)(s0 < xhi ? s0 : xhi);
-        end = (uint32_t)(s0 + DCHUNK < xhi ? s0 + DCHUNK : xhi);
+        end = (uint32_t)(s0 + chunk < xhi ? s0 + chunk : xhi);
+        if (next < end && __lane_id() == 0)
+            ahead = atomicAdd(dyn, 1u);
     };
     if constexpr (DYN != 0)
-        take_chunk(true);
+        take_chunk(wx);
     else
     {
         const uint64_t s0 = cidx * C;
@@ -163,7 +171,7 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
     for (;;)
     {
         const uint64_t busy = __ballot(!trav_done(st));
-        const uint32_t nidle = 64u - (uint32_t)__popcll(busy);
+        const uint32_t nidle = (uint32_t)lane_count(~busy);
         if ((next < end && nidle >= (uint32_t)REFILL) || busy == 0)
         {
             const bool idle = trav_done(st);
@@ -191,7 +199,7 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
             }
             next = next + nidle < end ? next + nidle : end;
             if (DYN != 0 && next >= end)
-                take_chunk(false);
+                take_chunk(wavesx + __builtin_amdgcn_readfirstlane(ahead) - dyn_base);
             else if (DYN == 0 && CHUNKS != 0 && next >= end)
             {
                 cidx += waves;
@@ -202,14 +210,15 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
         }
         // a lane with a pending triangle takes the triangle step next, any
         // other unfinished lane the node step
-        const int nt = __popcll(__ballot(st.trimask != 0));
-        const int nn = __popcll(__ballot(st.trimask == 0 && st.grp_mask != 0));
-        const bool tri = nt >= kTriLanes || (nt > 0 && nn < kNodeLanes);
+        const int nt = lane_count(__ballot(st.trimask != 0));
+        const int nn = lane_count(__ballot(st.trimask == 0 && st.grp_mask != 0));
+        const bool last = next >= end;
+        const bool tri = nt >= kTriLanes || (nt > 0 && (last || nn < kNodeLanes));
         if (tri && st.trimask != 0)
             trav_tri<ANY, false, WIDE>(tris, r, st);
         const bool can = st.trimask == 0 && st.grp_mask != 0;
-        const int nn2 = __popcll(__ballot(can));
-        if ((!tri || nn2 >= kNodeLanes) && can)
+        const int nn2 = lane_count(__ballot(can));
+        if ((!tri || last || nn2 >= kNodeLanes) && can)
             trav_node<BLOCK, TOP, WIDE>(nodes, r, st, stack, top, ntop);
     }
 }

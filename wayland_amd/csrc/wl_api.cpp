@@ -57,9 +57,9 @@ hipError_t sched_block(wl_context ctx, hipStream_t s, wl_context_s::SchedBlock *
         return hipSuccess;
     }
     wl_context_s::SchedBlock b;
-    hipError_t e = hipMalloc((void **)&b.dev, 256);
+    hipError_t e = hipMalloc((void **)&b.dev, 8 * 4 * wl::kSchedStride);
     if (e == hipSuccess)
-        e = hipMemset(b.dev, 0, 256);
+        e = hipMemset(b.dev, 0, 8 * 4 * wl::kSchedStride);
     if (e == hipSuccess) // the zeros land before any stream's next launch
         e = hipDeviceSynchronize();
     if (e != hipSuccess)

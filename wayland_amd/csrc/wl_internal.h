@@ -38,6 +38,11 @@ struct wl_context_s
 
 namespace wl
 {
+// Words from one XCD's chunk counter to the next: a cache line or more each.
+// With the eight in one line, every fetch moved the line between the XCDs'
+// L2s (about 100 ns per fetch).
+constexpr uint32_t kSchedStride = 64;
+
 void ctx_retain(wl_context ctx);
 void ctx_release(wl_context ctx);
 // The chunk counter block of stream s (allocated on first use); the caller

@@ -82,3 +82,20 @@ def test_ray_counts_around_the_chunk_sizes(gpu_ctx, n):
     _same(h, whole[:n])
     assert np.array_equal(occ, occ_whole[:n])
     _same(h[::41], ob.OracleBVH(sc.triangles()).closest(rays[:n:41]))
+
+
+@pytest.mark.parametrize("width", [1, 63, 255, 256, 257, 2047, 2048, 2049, 4100])
+@pytest.mark.parametrize("sort", [0, 1])
+def test_batch_sizes_around_the_queue_segments(gpu_ctx, width, sort):
+    """A batch of `width` paths against the same paths in batches of at most
+    64: the films are bit-identical, whatever queue segment a path is in."""
+    import torch
+    import wayland_amd as wl
+    print(f"case: {width} x 1, sort {sort}", flush=True)
+    sc = scenes.wavefront_scene(4, 2, width=width, height=1)
+    pt = wl.PathTracer(gpu_ctx, wl.Accel(gpu_ctx, sc), sc)
+    kw = dict(spp=1, max_depth=6, rr_depth=2, flags=wl.PT_SORT_BY_MATERIAL if sort else 0)
+    a, _ = pt.render(wl.pt_config(width, 1, **kw), stats=False)
+    b, _ = pt.render(wl.pt_config(width, 1, max_batch_paths=64, **kw), stats=False)
+    assert torch.equal(a, b)
+    assert (a[:, 0:3] != 0).any()

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(kExBlock) void k_example_pt(ExampleLaunch L)
                 TravRay r;
                 trav_setup(r, o.x, o.y, o.z, dir.x, dir.y, dir.z, tmin, 30.f);
                 uint32_t nn = 0, nt = 0;
-                const TravResult h = trav_run<false, false, kExBlock, true>(
+                const TravResult h = trav_run<kClosest, false, kExBlock, true>(
                     L.nodes, L.tris, r, true, stack, threadIdx.x, nn, nt);
                 if (h.prim == WL_INVALID)
                 {

@@ -32,6 +32,7 @@ static thread_local const char *g_fault_what = nullptr;
     } while (0)
 
 #include "traverse_device.h"
+#include "wl_pt.h"
 
 struct HostEmu
 {
@@ -89,10 +90,10 @@ uint64_t wlh_trace(void *p, const float *rays, uint32_t n, float *hits,
             uint32_t nn = 0, nt = 0;
             wl::TravResult res;
             if (any)
-                res = wl::trav_run<true, true, 1>(h->bvh.nodes.data(), h->bvh.tris.data(),
+                res = wl::trav_run<wl::kAny, true, 1>(h->bvh.nodes.data(), h->bvh.tris.data(),
                                                   tr, true, stack, 0, nn, nt);
             else
-                res = wl::trav_run<false, true, 1>(h->bvh.nodes.data(), h->bvh.tris.data(),
+                res = wl::trav_run<wl::kClosest, true, 1>(h->bvh.nodes.data(), h->bvh.tris.data(),
                                                    tr, true, stack, 0, nn, nt);
             float *o = hits + 4 * (size_t)i;
             o[0] = res.t;
@@ -243,6 +244,9 @@ uint64_t wlh_serve_check(const uint32_t *req4, uint32_t n, uint32_t capacity, ui
     }
     return bad;
 }
+
+// Entries of a queue segment of a batch of n paths (wl_pt.h).
+uint32_t wlh_pt_segment(uint64_t n) { return wl::pt_segment(n); }
 
 // The counter advance of the run-time chunk schedule (dyn_xcd_chunks).
 uint32_t wlh_dyn_chunks(uint32_t n, uint32_t xcd, uint32_t chunk)

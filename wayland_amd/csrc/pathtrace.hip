@@ -4,10 +4,12 @@
 // PathTracing.cu:40-139, __closesthit__radiance :181-289, __miss__radiance
 // :163-171, NEE :81-128, RR :130-138) as queue kernels:
 //
-//   [extend -> shade -> shadow] x max_depth -> accumulate
+//   first trace -> [shade -> trace] x max_depth -> accumulate
 //
-//   extend     closest-hit BVH8 traversal of the active ray queue.  The
-//              first pass of a single-scene batch traces path i's camera
+//   trace      BVH8 traversal: closest hits of the next bounce's rays and, in
+//              the same launch, any hits of this bounce's shadow rays, whose
+//              precomputed NEE contribution is added where unoccluded.  The
+//              first one of a single-scene batch traces path i's camera
 //              ray (TEA seed (pixel, frame), pinhole ray) computed in place,
 //              and the first shade pass recomputes that vertex's state and
 //              starts the path's radiance: nothing is written per path
@@ -17,15 +19,20 @@
 //              sample-pdf-eval / NEE light sample + BSDF eval / RR, in the
 //              reference's RNG draw order; appends the continuing paths and
 //              the shadow rays to compacted queues (wave64 ballot + mbcnt
-//              prefix, one atomic per queue per workgroup).
-//   shadow     any-hit traversal of the shadow queue; adds the precomputed
-//              NEE contribution of unoccluded rays.
+//              prefix, one atomic per workgroup).
 //   accumulate compensated (Kahan) FP32 film: sum + compensation per pixel.
 //
 // Radiance contributions reach a path in the reference's order (one per
 // bounce at most), so per-sample radiance matches a serial evaluation.
 // Every kernel loops over a device-side queue count with a fixed grid, so the
 // host enqueues a whole batch without synchronising.
+//
+// The queues are split into eight segments, one per XCD (workgroups with
+// blockIdx % 8 == x run on XCD x): a workgroup appends to its XCD's segment
+// and the next kernel's workgroups on that XCD read it, so the append counter
+// and the entries stay in one L2.  The first queue is the identity over the
+// batch's paths (entry i is path i, blocks of kPtBlock dealt to the XCDs in
+// turn) and is never written.
 #include "guide_device.h"
 #include "shading_device.h"
 #include "traverse_persistent.h"
@@ -37,14 +44,42 @@ namespace wl
 
 constexpr int kPtBlock = 256;
 
-// ---- workgroup-level append to two queues -----------------------------------
-// Every wave of the workgroup calls this in the same loop pass.  Per wave a
-// ballot and mbcnt prefix; per workgroup one atomic per queue, issued by one
-// thread.  All waves appending to one counter serialise at one L2 channel,
-// so a per-wave atomic makes the counter the bottleneck of the shade kernel;
-// a per-workgroup one divides that by the waves per workgroup.  The LDS
-// slots alternate between passes (pass parity), so two barriers per pass
-// suffice.
+// ---- queues -------------------------------------------------------------------
+// XCD x's queue lengths of one parity: low word the ray queue's segment, high
+// word the shadow queue's.
+__device__ __forceinline__ unsigned long long *queue_len(const PtBuffers &B, uint32_t xcd,
+                                                         int parity)
+{
+    return reinterpret_cast<unsigned long long *>(B.counters +
+                                                  kPtCounterStride * (4 * xcd + (uint32_t)parity));
+}
+// XCD x's chunk counter of the traversal (zero when a trace kernel starts).
+__device__ __forceinline__ uint32_t *queue_chunks(const PtBuffers &B, uint32_t xcd)
+{
+    return B.counters + kPtCounterStride * (4 * xcd + 2);
+}
+
+// The entries of the ray queue that this XCD's workgroups take, in blocks of
+// kPtBlock: block k of the walk is [at(k), at(k) + kPtBlock) clipped to limit.
+struct QueueWalk
+{
+    uint32_t base, step, limit;
+    __device__ __forceinline__ uint32_t at(uint32_t k) const { return base + k * step; }
+};
+__device__ __forceinline__ QueueWalk queue_walk(const PtBuffers &B, int parity, bool first)
+{
+    const uint32_t x = blockIdx.x % 8u;
+    if (first)
+        return QueueWalk{ x * kPtBlock, 8u * kPtBlock, B.counters[kPtFlatCount] };
+    const uint32_t lo = x * B.segcap;
+    return QueueWalk{ lo, kPtBlock, lo + (uint32_t)*queue_len(B, x, parity) };
+}
+
+// Workgroup-level append to the XCD's segments of two queues.  Every wave of
+// the workgroup calls this in the same loop pass.  Per wave a ballot and
+// mbcnt prefix; per workgroup one 64-bit atomic for both queues, issued by one
+// thread.  The LDS slots alternate between passes (pass parity), so two
+// barriers per pass suffice.
 struct BlockAppendLds
 {
     uint32_t cnt[2][2][kPtBlock / 64]; // [pass parity][queue][wave]
@@ -52,7 +87,7 @@ struct BlockAppendLds
 };
 
 __device__ __forceinline__ void block_append2(BlockAppendLds &L, uint32_t pass,
-                                              uint32_t *c0, bool p0, uint32_t *c1, bool p1,
+                                              unsigned long long *len, bool p0, bool p1,
                                               uint32_t &slot0, uint32_t &slot1)
 {
     const uint32_t par = pass & 1u;
@@ -72,8 +107,10 @@ __device__ __forceinline__ void block_append2(BlockAppendLds &L, uint32_t pass,
             t0 += L.cnt[par][0][w];
             t1 += L.cnt[par][1][w];
         }
-        L.base[par][0] = t0 ? atomicAdd(c0, t0) : 0u;
-        L.base[par][1] = t1 ? atomicAdd(c1, t1) : 0u;
+        const unsigned long long add = (unsigned long long)t1 << 32 | t0;
+        const unsigned long long old = add ? atomicAdd(len, add) : 0ull;
+        L.base[par][0] = (uint32_t)old;
+        L.base[par][1] = (uint32_t)(old >> 32);
     }
     __syncthreads();
     uint32_t o0 = L.base[par][0], o1 = L.base[par][1];
@@ -82,10 +119,8 @@ __device__ __forceinline__ void block_append2(BlockAppendLds &L, uint32_t pass,
         o0 += L.cnt[par][0][w];
         o1 += L.cnt[par][1][w];
     }
-    slot0 = o0 + __builtin_amdgcn_mbcnt_hi((uint32_t)(m0 >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m0, 0u));
-    slot1 = o1 + __builtin_amdgcn_mbcnt_hi((uint32_t)(m1 >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m1, 0u));
+    slot0 = o0 + lane_prefix(m0);
+    slot1 = o1 + lane_prefix(m1);
 }
 
 __device__ __forceinline__ float4 f4(V3 v, float w) { return make_float4(v.x, v.y, v.z, w); }
@@ -107,8 +142,15 @@ __device__ __forceinline__ void camera_ray(const PtParams &P, uint32_t p, V3 &o,
     o = ld3(P.cam.pos);
 }
 
-// Start of a single-scene batch: the first queue's length and the material
-// bins.  No per-path state is written: the first extend pass computes each
+// Clears the queue lengths and chunk counters and sets the first queue's length.
+__device__ __forceinline__ void start_counters(const PtBuffers &B, uint32_t npaths)
+{
+    for (uint32_t i = threadIdx.x; i < kPtCounters; i += blockDim.x)
+        B.counters[i] = i == kPtFlatCount ? npaths : 0u;
+}
+
+// Start of a single-scene batch: the queue counters and the material bins.
+// No per-path state is written: the first trace computes each
 // path's camera ray with camera_ray, and the first shade pass recomputes the
 // first vertex's state (origin, direction and seed, throughput 1, depth 0,
 // lastTraceTerm 1, lastPdf 1) and writes the path's radiance (and, when
@@ -116,8 +158,7 @@ __device__ __forceinline__ void camera_ray(const PtParams &P, uint32_t p, V3 &o,
 // or radiance write and read before its first traversal.
 __global__ void k_batch_start(PtParams P, PtBuffers B)
 {
-    if (threadIdx.x == 0)
-        B.counters[0] = P.npix * P.nsamples;
+    start_counters(B, P.npix * P.nsamples);
     for (uint32_t b = threadIdx.x; b < P.sort_bins; b += blockDim.x)
         B.sort_bins[b] = 0;
 }
@@ -146,47 +187,25 @@ __device__ __forceinline__ uint32_t pt_load_top(uint4 *top, const PtScene &S)
     return ntop;
 }
 
-// ---- extend: closest hit for the active queue -----------------------------
-template <int STACK, bool MULTI>
-__global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(STACK == 16 ? 6 : 5)))
-void k_extend(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs, float eps)
+// ---- trace: closest hits of the ray queue, any hits of the shadow queue -----
+// Rays per chunk (traverse_persistent.h): 64 fill one wave's lanes, more share
+// the counter's latency once every wave has plenty.
+__device__ __forceinline__ uint32_t queue_chunk(uint32_t n_xcd)
 {
-    __shared__ uint32_t stack[STACK * kPtBlock];
-    __shared__ uint4 top[8 * (pt_top_nodes<STACK, MULTI>() ? pt_top_nodes<STACK, MULTI>() : 1)];
-    const uint32_t ntop = pt_load_top<STACK, MULTI>(top, S);
-    const uint32_t count = B.counters[parity];
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-    {
-        B.counters[parity ^ 1] = 0; // next queue
-        B.counters[2] = 0;          // shadow queue
-        B.stats[0] += count;        // extension rays (single writer)
-    }
-    const wl_ray *rays = parity ? B.rays1 : B.rays0;
-    const uint32_t *qreq = parity ? B.qreq1 : B.qreq0; // multi-request batches
-    // the queues carry the path's lastPdf and seed in the rays' w words (the
-    // shade pass reads its state back from the ray): every extension ray is
-    // traced on [epsilon, 1e30], epsilon the batch's or the ray's request's
-    auto load_eps = [&](uint32_t i, TravRay &r, float e) {
-        const f4v *rp = reinterpret_cast<const f4v *>(rays + i);
-        const f4v a = __builtin_nontemporal_load(rp), b = __builtin_nontemporal_load(rp + 1);
-        trav_setup(r, a.x, a.y, a.z, b.x, b.y, b.z, e, 1e30f);
+    const uint32_t wavesx = (gridDim.x / 8u) * (kPtBlock / 64);
+    return n_xcd / 128u < wavesx ? 64u : 128u;
+}
+
+// The first queue's chunks: the XCD's blocks of kPtBlock entries, in pieces.
+__device__ __forceinline__ auto first_chunks(uint32_t n)
+{
+    const uint32_t chunk = queue_chunk(n / 8u), per = kPtBlock / chunk;
+    const uint32_t x = blockIdx.x % 8u;
+    return [=](uint32_t c, uint32_t &next, uint32_t &end) {
+        const uint64_t s0 = ((uint64_t)(c / per) * 8u + x) * kPtBlock + (c % per) * chunk;
+        next = (uint32_t)(s0 < n ? s0 : n);
+        end = (uint32_t)(s0 + chunk < n ? s0 + chunk : n);
     };
-    auto load = [&](uint32_t i, TravRay &r) { load_eps(i, r, eps); };
-    auto store = [&](uint32_t i, const TravResult &h) { store_hit_nt(B.hits, i, h); };
-    if constexpr (MULTI) // S.nodes / S.tris: the arena of the requests' BVHs
-        trav_persistent<false, kPtBlock, STACK != 16, true, false, 8, 20>(
-            S.nodes, S.tris, count, stack,
-            [&](uint32_t i, TravRay &r, uint32_t &root) {
-                const PtReq &rq = reqs[qreq[i]];
-                root = rq.root;
-                load_eps(i, r, rq.P.epsilon);
-            },
-            store);
-    else
-        trav_persistent<false, kPtBlock, STACK != 16, false, false, 0, 20, 0,
-                        pt_top_nodes<STACK, false>() != 0>(
-            S.nodes, S.tris, count, stack, load, store,
-            reinterpret_cast<const WlBvh8Node *>(top), ntop);
 }
 
 // The first bounce of a single-scene batch: queue entry i is path i, and its
@@ -194,29 +213,133 @@ void k_extend(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs
 // not read from a ray queue: nothing is written before the first traversal.
 template <int STACK>
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(5)))
-void k_extend_first(PtParams P, PtScene S, PtBuffers B)
+void k_trace_first(PtParams P, PtScene S, PtBuffers B)
 {
     __shared__ uint32_t stack[STACK * kPtBlock];
     __shared__ uint4 top[8 * (pt_top_nodes<STACK, false>() ? pt_top_nodes<STACK, false>() : 1)];
     const uint32_t ntop = pt_load_top<STACK, false>(top, S);
     const uint32_t count = P.npix * P.nsamples;
     if (blockIdx.x == 0 && threadIdx.x == 0)
-    {
-        B.counters[1] = 0; // next queue
-        B.counters[2] = 0; // shadow queue
         B.stats[0] += count;
+    trav_persistent<kClosest, kPtBlock, STACK != 16, pt_top_nodes<STACK, false>() != 0>(
+        S.nodes, S.tris, stack, first_chunks(count),
+        [&](uint32_t i, TravRay &r, uint32_t &) {
+            V3 o, d;
+            uint32_t seed;
+            camera_ray(P, i, o, d, seed);
+            trav_setup(r, o.x, o.y, o.z, d.x, d.y, d.z, P.epsilon, 1e30f);
+        },
+        [&](uint32_t i, const TravRay &, const TravResult &h) { store_hit_nt(B.hits, i, h); },
+        reinterpret_cast<const WlBvh8Node *>(top), ntop, queue_chunks(B, blockIdx.x % 8u), 0u);
+}
+
+// The two queues of a bounce are independent (a shadow ray adds to its path's
+// radiance, which the closest hits do not touch), so one launch traces both:
+// each XCD's chunks are those of its ray segment, then those of its shadow
+// segment.  The shadow rays fill the waves that the last closest hits leave
+// idle, and a bounce costs one launch less.  The chunks handed out at run time
+// replace equal ranges per wave, which waited for the most expensive one (the
+// caustic's shadow kernel took 87 us on average for what its closest hits did
+// in 64).  With the per-XCD queues: 1024^2 caustic pass 3.01 -> 2.05 ms, two
+// 1024^2 Cornell frames of 25 bounces 3.33 -> 2.53 ms, 517 x 389 x 3 textured
+// 1.35 -> 0.87 ms, 1080p x 64 spp 40.2 -> 36.0 ms, 64 serving requests 393 (at
+// equal ranges before any of this) -> 309 ms.
+// first: the multi-request raygen's queue (all rays, no shadow rays).
+template <int STACK, bool MULTI>
+__global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(STACK == 16 ? 6 : 5)))
+void k_trace(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs, float eps,
+             int first)
+{
+    __shared__ uint32_t stack[STACK * kPtBlock];
+    __shared__ uint4 top[8 * (pt_top_nodes<STACK, MULTI>() ? pt_top_nodes<STACK, MULTI>() : 1)];
+    const uint32_t ntop = pt_load_top<STACK, MULTI>(top, S);
+    const uint32_t x = blockIdx.x % 8u;
+    const wl_ray *rays = parity ? B.rays1 : B.rays0;
+    const uint32_t *qreq = parity ? B.qreq1 : B.qreq0; // multi-request batches
+    const unsigned long long len = *queue_len(B, x, parity);
+    const uint32_t flat = first ? B.counters[kPtFlatCount] : 0u;
+    const uint32_t nrays = (uint32_t)len, nshadow = (uint32_t)(len >> 32);
+    if (blockIdx.x < 8u && threadIdx.x == 0)
+    {
+        *queue_len(B, x, parity ^ 1) = 0ull; // the next shade pass appends there
+        const unsigned long long n0 = first ? (x == 0 ? flat : 0u) : nrays;
+        if (n0)
+            atomicAdd(&B.stats[0], n0); // extension rays
+        if (nshadow)
+            atomicAdd(&B.stats[1], (unsigned long long)nshadow);
     }
-    auto load = [&](uint32_t i, TravRay &r) {
-        V3 o, d;
-        uint32_t seed;
-        camera_ray(P, i, o, d, seed);
-        trav_setup(r, o.x, o.y, o.z, d.x, d.y, d.z, P.epsilon, 1e30f);
+    const auto flat_range = first_chunks(flat);
+    const uint32_t lo = x * B.segcap;
+    const uint32_t chunk = queue_chunk(nrays + nshadow);
+    const uint32_t ray_chunks = (nrays + chunk - 1u) / chunk;
+    bool shadow = false; // the kind of the wave's current chunk
+    auto range = [&](uint32_t c, uint32_t &next, uint32_t &end) {
+        if (first)
+        {
+            flat_range(c, next, end);
+            return;
+        }
+        shadow = c >= ray_chunks;
+        const uint32_t n = shadow ? nshadow : nrays;
+        const uint64_t s0 = (uint64_t)(shadow ? c - ray_chunks : c) * chunk;
+        next = lo + (uint32_t)(s0 < n ? s0 : n);
+        end = lo + (uint32_t)(s0 + chunk < n ? s0 + chunk : n);
     };
-    auto store = [&](uint32_t i, const TravResult &h) { store_hit_nt(B.hits, i, h); };
-    trav_persistent<false, kPtBlock, STACK != 16, false, false, 0, 20, 0,
-                    pt_top_nodes<STACK, false>() != 0>(
-        S.nodes, S.tris, count, stack, load, store,
-        reinterpret_cast<const WlBvh8Node *>(top), ntop);
+    auto fetch = [&](uint32_t i, TravRay &r, uint32_t &root) {
+        // the queues carry the path's lastPdf and seed in the rays' w words
+        // (the shade pass reads its state back from the ray): every extension
+        // ray is traced on [epsilon, 1e30], epsilon the batch's or the ray's
+        // request's
+        const f4v *rp = reinterpret_cast<const f4v *>((shadow ? B.srays : rays) + i);
+        const f4v a = __builtin_nontemporal_load(rp), b = __builtin_nontemporal_load(rp + 1);
+        float tmin = a.w, tmax = b.w;
+        if (!shadow)
+        {
+            tmin = eps;
+            tmax = 1e30f;
+        }
+        if constexpr (MULTI) // S.nodes / S.tris: the arena of the requests' BVHs
+        {
+            if (shadow)
+                root = B.sreq[i];
+            else
+            {
+                const PtReq &rq = reqs[qreq[i]];
+                root = rq.root;
+                tmin = rq.P.epsilon;
+            }
+        }
+        trav_setup(r, a.x, a.y, a.z, b.x, b.y, b.z, tmin, tmax);
+        r.code |= shadow ? kAnyRay : 0u;
+    };
+    auto emit = [&](uint32_t i, const TravRay &r, const TravResult &h) {
+        if (!(r.code & kAnyRay))
+        {
+            store_hit_nt(B.hits, i, h);
+            return;
+        }
+        if (h.prim != WL_INVALID)
+            return;
+        // unoccluded: add the NEE contribution (one shadow ray per path)
+        const uint32_t path = B.spath[i];
+        const float4 c = B.scontrib[i];
+        float4 rr = B.rad[path];
+        rr.x = rr.x + c.x;
+        rr.y = rr.y + c.y;
+        rr.z = rr.z + c.z;
+        B.rad[path] = rr;
+        if (c.w != 0.0f) // the path records guide training radiance
+        {
+            float4 ga = B.gacc[path];
+            ga.x += c.x;
+            ga.y += c.y;
+            ga.z += c.z;
+            B.gacc[path] = ga;
+        }
+    };
+    trav_persistent<kMixed, kPtBlock, STACK != 16, pt_top_nodes<STACK, MULTI>() != 0>(
+        S.nodes, S.tris, stack, range, fetch, emit, reinterpret_cast<const WlBvh8Node *>(top),
+        ntop, queue_chunks(B, x), 0u);
 }
 
 // ---- material sort of the shade queue ------------------------------------------
@@ -235,16 +358,19 @@ __device__ __forceinline__ uint32_t sort_key(const PtScene &S, uint32_t prim, ui
 }
 
 __global__ __launch_bounds__(kPtBlock) void k_sort_count(PtParams P, PtScene S, PtBuffers B,
-                                                         int parity)
+                                                         int parity, int first)
 {
     __shared__ uint32_t hist[kSortMaxBins];
     const uint32_t nb = P.sort_bins;
     for (uint32_t b = threadIdx.x; b < nb; b += kPtBlock)
         hist[b] = 0;
     __syncthreads();
-    const uint32_t count = B.counters[parity];
-    for (uint32_t i = blockIdx.x * kPtBlock + threadIdx.x; i < count; i += gridDim.x * kPtBlock)
+    const QueueWalk q = queue_walk(B, parity, first != 0);
+    for (uint32_t k = blockIdx.x / 8u; q.at(k) < q.limit; k += gridDim.x / 8u)
     {
+        const uint32_t i = q.at(k) + threadIdx.x;
+        if (i >= q.limit)
+            break;
         const uint32_t key =
             sort_key(S, __float_as_uint(reinterpret_cast<const float4 *>(B.hits)[i].y), nb);
         B.sort_keys[i] = key;
@@ -289,20 +415,21 @@ __global__ void k_sort_scan(PtParams P, PtBuffers B)
     }
 }
 
-__global__ __launch_bounds__(kPtBlock) void k_sort_scatter(PtParams P, PtBuffers B, int parity)
+__global__ __launch_bounds__(kPtBlock) void k_sort_scatter(PtParams P, PtBuffers B, int parity,
+                                                           int first)
 {
     __shared__ uint32_t hist[kSortMaxBins];
     __shared__ uint32_t base[kSortMaxBins];
     const uint32_t nb = P.sort_bins;
-    const uint32_t count = B.counters[parity];
-    for (uint32_t start = blockIdx.x * kPtBlock; start < count; start += gridDim.x * kPtBlock)
+    const QueueWalk q = queue_walk(B, parity, first != 0);
+    for (uint32_t k = blockIdx.x / 8u; q.at(k) < q.limit; k += gridDim.x / 8u)
     {
         for (uint32_t b = threadIdx.x; b < nb; b += kPtBlock)
             hist[b] = 0;
         __syncthreads();
-        const uint32_t i = start + threadIdx.x;
+        const uint32_t i = q.at(k) + threadIdx.x;
         uint32_t key = 0, local = 0;
-        if (i < count)
+        if (i < q.limit)
         {
             key = B.sort_keys[i];
             local = atomicAdd(&hist[key], 1u);
@@ -312,7 +439,7 @@ __global__ __launch_bounds__(kPtBlock) void k_sort_scatter(PtParams P, PtBuffers
             if (hist[b])
                 base[b] = atomicAdd(&B.sort_bins[kSortMaxBins + b], hist[b]);
         __syncthreads();
-        if (i < count)
+        if (i < q.limit)
             B.sort_perm[base[key] + local] = i;
         __syncthreads();
     }
@@ -397,12 +524,10 @@ void k_guide_infer_pt(PtParams P, PtScene S, PtBuffers B, int parity)
     guide_stage<kPtBlock, kGuideFwdVecs>(sA, fwd);
     guide_stage_biases<kPtBlock>(sb, P.gparams);
     __syncthreads();
-    const uint32_t count = B.counters[parity];
+    const QueueWalk qw = queue_walk(B, parity, SEL != 2);
     const uint32_t *qin = parity ? B.qpath1 : B.qpath0;
     const wl_ray *rays = parity ? B.rays1 : B.rays0;
     const int lane = threadIdx.x & 63, g = lane >> 4;
-    const uint32_t nwaves = gridDim.x * (kPtBlock / 64);
-    const uint32_t wave = blockIdx.x * (kPtBlock / 64) + threadIdx.x / 64;
     // one tile: ring entries [head, head + n), n <= 16 (wave-uniform)
     auto run_tile = [&](uint32_t head, uint32_t n) {
         const uint32_t k = (uint32_t)(lane & 15);
@@ -448,11 +573,12 @@ void k_guide_infer_pt(PtParams P, PtScene S, PtBuffers B, int parity)
         guide_decode_lanes(o, g, B.gout + kGuideDecoded * (size_t)i, valid);
     };
     uint32_t head = 0, tail = 0; // ring positions, wave-uniform
-    for (uint32_t base = wave * 64u; base < count; base += nwaves * 64u)
+    // wave w of a workgroup takes the 64 entries 64 w of each of its blocks
+    for (uint32_t b = blockIdx.x / 8u; qw.at(b) < qw.limit; b += gridDim.x / 8u)
     {
-        const uint32_t i = base + (uint32_t)lane;
+        const uint32_t i = qw.at(b) + threadIdx.x;
         bool want = false;
-        if (i < count)
+        if (i < qw.limit)
         {
             const uint32_t prim = reinterpret_cast<const uint32_t *>(B.hits)[4 * (size_t)i + 1];
             want = guide_wanted<SEL>(P, S, B, qin, prim, i);
@@ -493,18 +619,33 @@ __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(3)))
 void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__restrict__ reqs,
              int first)
 {
-    const uint32_t count = B.counters[parity];
+    QueueWalk q = queue_walk(B, parity, first != 0);
+    if (!MULTI && P0.sort_bins)
+    {
+        // the sorted order of the whole queue, dealt in blocks as the first's
+        uint32_t total = B.counters[kPtFlatCount];
+        if (!first)
+        {
+            total = 0;
+            for (uint32_t x = 0; x < 8u; ++x)
+                total += (uint32_t)*queue_len(B, x, parity);
+        }
+        q = QueueWalk{ (blockIdx.x % 8u) * kPtBlock, 8u * kPtBlock, total };
+    }
+    if (blockIdx.x < 8u && threadIdx.x == 0)
+        *queue_chunks(B, blockIdx.x) = 0u; // the next trace counts from zero
+    const uint32_t seg = (blockIdx.x % 8u) * B.segcap;
     const uint32_t *qin = parity ? B.qpath1 : B.qpath0;
     uint32_t *qout = parity ? B.qpath0 : B.qpath1;
     wl_ray *rout = parity ? B.rays0 : B.rays1;
     __shared__ BlockAppendLds app;
     uint32_t pass = 0;
-    // every thread of the workgroup runs the same passes (base is per
+    // every thread of the workgroup runs the same passes (k is per
     // workgroup), as the workgroup barriers of the append require
-    for (uint32_t base = blockIdx.x * kPtBlock; base < count; base += gridDim.x * kPtBlock)
+    for (uint32_t k = blockIdx.x / 8u; q.at(k) < q.limit; k += gridDim.x / 8u)
     {
-        const uint32_t j = base + threadIdx.x;
-        const bool in_range = j < count;
+        const uint32_t j = q.at(k) + threadIdx.x;
+        const bool in_range = j < q.limit;
         // material-sorted order: the j-th entry of the sorted queue
         const uint32_t i = (!MULTI && P0.sort_bins && in_range) ? B.sort_perm[j] : j;
         bool cont = false, shadow = false, shadow_gacc = false;
@@ -872,8 +1013,10 @@ void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__re
         }
         // ---- compaction (whole wave participates)
         uint32_t slot, sslot;
-        block_append2(app, pass++, &B.counters[parity ^ 1], cont, &B.counters[2], shadow, slot,
+        block_append2(app, pass++, queue_len(B, blockIdx.x % 8u, parity ^ 1), cont, shadow, slot,
                       sslot);
+        slot += seg;
+        sslot += seg;
         if (cont)
         {
             qout[slot] = path;
@@ -892,58 +1035,13 @@ void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__re
     }
 }
 
-// ---- shadow: any hit; unoccluded rays add their NEE contribution ----------
-template <int STACK, bool MULTI>
-__global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(STACK == 16 ? 6 : 5)))
-void k_shadow(PtScene S, PtBuffers B, const PtReq *__restrict__ reqs)
-{
-    __shared__ uint32_t stack[STACK * kPtBlock];
-    __shared__ uint4 top[8 * (pt_top_nodes<STACK, MULTI>() ? pt_top_nodes<STACK, MULTI>() : 1)];
-    const uint32_t ntop = pt_load_top<STACK, MULTI>(top, S);
-    const uint32_t count = B.counters[2];
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        B.stats[1] += count;
-    auto load = [&](uint32_t i, TravRay &r) { load_ray_nt(B.srays, i, r); };
-    auto add = [&](uint32_t i, const TravResult &h) {
-        if (h.prim != WL_INVALID)
-            return;
-        // unoccluded: add the NEE contribution (one shadow ray per path)
-        const uint32_t path = B.spath[i];
-        const float4 c = B.scontrib[i];
-        float4 rr = B.rad[path];
-        rr.x = rr.x + c.x;
-        rr.y = rr.y + c.y;
-        rr.z = rr.z + c.z;
-        B.rad[path] = rr;
-        if (c.w != 0.0f) // the path records guide training radiance
-        {
-            float4 ga = B.gacc[path];
-            ga.x += c.x;
-            ga.y += c.y;
-            ga.z += c.z;
-            B.gacc[path] = ga;
-        }
-    };
-    if constexpr (MULTI) // S.nodes / S.tris: the arena of the requests' BVHs
-        trav_persistent<true, kPtBlock, STACK != 16, true, false, 8, 20>(
-            S.nodes, S.tris, count, stack,
-            [&](uint32_t i, TravRay &r, uint32_t &root) {
-                root = B.sreq[i];
-                load(i, r);
-            },
-            add);
-    else
-        trav_persistent<true, kPtBlock, STACK != 16, false, false, 2, 20, 0,
-                        pt_top_nodes<STACK, false>() != 0>(
-            S.nodes, S.tris, count, stack, load, add,
-            reinterpret_cast<const WlBvh8Node *>(top), ntop);
-}
-
 // ---- batched serving: raygen and film update of a multi-request megabatch ----
-__global__ void k_batch_begin(PtMultiLaunch L)
+__global__ void k_batch_begin(PtMultiLaunch L, PtBuffers B)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        *L.header = L.batches[*L.batch_index];
+    const PtBatchHeader h = L.batches[*L.batch_index];
+    if (threadIdx.x == 0)
+        *L.header = h;
+    start_counters(B, h.paths);
 }
 
 __global__ void k_batch_end(PtMultiLaunch L)
@@ -988,8 +1086,6 @@ __global__ __launch_bounds__(kPtBlock) void k_raygen_multi(PtMultiLaunch L, PtBu
         B.rays0[p] = wl_ray{ o.x, o.y, o.z, 1.0f, d.x, d.y, d.z, __uint_as_float(seed) };
         B.qreq0[p] = it.req;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        B.counters[0] = npaths;
 }
 
 // Kahan update of each item's film, samples in ascending order (the order
@@ -1195,7 +1291,25 @@ __global__ void k_resolve(const float *film, uint32_t npix, uint32_t nsamples, f
 }
 
 // ---- host side: one batch ---------------------------------------------------
-hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B,
+// Workgroups of `kernel` that fit a CU at once.
+template <class K>
+static int blocks_per_cu(K kernel)
+{
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kPtBlock, 0) != hipSuccess ||
+        n < 1)
+        n = 4;
+    return n;
+}
+
+// A grid of at most `blocks` workgroups and per_cu per CU, a multiple of 8.
+static uint32_t grid8(uint32_t blocks, int num_cus, int per_cu)
+{
+    const uint32_t fit = (uint32_t)std::max(1, num_cus) * (uint32_t)per_cu;
+    return (std::min<uint32_t>(blocks, fit) + 7u) & ~7u;
+}
+
+hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B0,
                         int num_cus, hipStream_t st)
 {
     const uint32_t npaths = P.npix * P.nsamples;
@@ -1203,57 +1317,48 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B,
     // a BVH at most 16 deep needs at most 15 stack entries per lane; those
     // kernels also address nodes and triangles with 32-bit offsets
     const bool shallow = S.bvh_depth <= 16 && wl_bvh8_narrow(S.num_nodes, S.num_tris);
-    // persistent traversal grids: the workgroups that fit the GPU at once
+    // persistent traversal grids: the workgroups that fit the GPU at once.  All
+    // grids are multiples of 8 (each XCD its share).
     static int occ16 = 0, occ32 = 0, occf16 = 0, occf32 = 0;
     if (!occ16)
     {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occf16, k_extend_first<16>, kPtBlock,
-                                                         0) != hipSuccess ||
-            occf16 < 1)
-            occf16 = 4;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &occf32, k_extend_first<WL_BVH8_STACK_DEPTH>, kPtBlock, 0) != hipSuccess ||
-            occf32 < 1)
-            occf32 = 4;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ16, k_extend<16, false>, kPtBlock,
-                                                         0) != hipSuccess ||
-            occ16 < 1)
-            occ16 = 4;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &occ32, k_extend<WL_BVH8_STACK_DEPTH, false>, kPtBlock, 0) != hipSuccess ||
-            occ32 < 1)
-            occ32 = 4;
+        occf16 = blocks_per_cu(k_trace_first<16>);
+        occf32 = blocks_per_cu(k_trace_first<WL_BVH8_STACK_DEPTH>);
+        occ32 = blocks_per_cu(k_trace<WL_BVH8_STACK_DEPTH, false>);
+        occ16 = blocks_per_cu(k_trace<16, false>);
     }
-    const uint32_t g_trav =
-        std::min<uint32_t>(blocks_all, (uint32_t)num_cus * (uint32_t)(shallow ? occ16 : occ32));
-    const uint32_t g_first =
-        std::min<uint32_t>(blocks_all, (uint32_t)num_cus * (uint32_t)(shallow ? occf16 : occf32));
-    const uint32_t g_shade = std::min<uint32_t>(blocks_all, (uint32_t)num_cus * 8);
-    const uint32_t g_sort = std::min<uint32_t>(blocks_all, (uint32_t)num_cus * 4);
-    // guide inference: 64 queries per workgroup pass, up to 4 workgroups per CU
-    const uint32_t g_guide =
-        std::max<uint32_t>(1, std::min<uint32_t>((npaths + 63) / 64, (uint32_t)num_cus * 4));
+    const uint32_t g_trav = grid8(4 * blocks_all, num_cus, shallow ? occ16 : occ32);
+    const uint32_t g_first = grid8(4 * blocks_all, num_cus, shallow ? occf16 : occf32);
+    const uint32_t g_shade = grid8(blocks_all, num_cus, 8);
+    const uint32_t g_sort = grid8(blocks_all, num_cus, 4);
+    // guide inference: up to 4 workgroups per CU
+    const uint32_t g_guide = grid8(blocks_all, num_cus, 4);
+    PtBuffers B = B0;
+    B.segcap = pt_segment(npaths);
+    auto trace = [&](int parity) {
+        if (shallow)
+            hipLaunchKernelGGL((k_trace<16, false>), dim3(g_trav), dim3(kPtBlock), 0, st, S, B,
+                               parity, nullptr, P.epsilon, 0);
+        else
+            hipLaunchKernelGGL((k_trace<WL_BVH8_STACK_DEPTH, false>), dim3(g_trav),
+                               dim3(kPtBlock), 0, st, S, B, parity, nullptr, P.epsilon, 0);
+    };
     hipLaunchKernelGGL(k_batch_start, dim3(1), dim3(kPtBlock), 0, st, P, B);
+    if (shallow)
+        hipLaunchKernelGGL((k_trace_first<16>), dim3(g_first), dim3(kPtBlock), 0, st, P, S, B);
+    else
+        hipLaunchKernelGGL((k_trace_first<WL_BVH8_STACK_DEPTH>), dim3(g_first), dim3(kPtBlock), 0,
+                           st, P, S, B);
     for (uint32_t b = 0; b < P.max_depth; ++b)
     {
-        const int parity = (int)(b & 1u);
-        if (b == 0 && shallow)
-            hipLaunchKernelGGL((k_extend_first<16>), dim3(g_first), dim3(kPtBlock), 0, st, P, S,
-                               B);
-        else if (b == 0)
-            hipLaunchKernelGGL((k_extend_first<WL_BVH8_STACK_DEPTH>), dim3(g_first),
-                               dim3(kPtBlock), 0, st, P, S, B);
-        else if (shallow)
-            hipLaunchKernelGGL((k_extend<16, false>), dim3(g_trav), dim3(kPtBlock), 0, st, S, B,
-                               parity, nullptr, P.epsilon);
-        else
-            hipLaunchKernelGGL((k_extend<WL_BVH8_STACK_DEPTH, false>), dim3(g_trav),
-                               dim3(kPtBlock), 0, st, S, B, parity, nullptr, P.epsilon);
+        const int parity = (int)(b & 1u), first = b == 0 ? 1 : 0;
         if (P.sort_bins)
         {
-            hipLaunchKernelGGL(k_sort_count, dim3(g_sort), dim3(kPtBlock), 0, st, P, S, B, parity);
+            hipLaunchKernelGGL(k_sort_count, dim3(g_sort), dim3(kPtBlock), 0, st, P, S, B, parity,
+                               first);
             hipLaunchKernelGGL(k_sort_scan, dim3(1), dim3(kPtBlock), 0, st, P, B);
-            hipLaunchKernelGGL(k_sort_scatter, dim3(g_sort), dim3(kPtBlock), 0, st, P, B, parity);
+            hipLaunchKernelGGL(k_sort_scatter, dim3(g_sort), dim3(kPtBlock), 0, st, P, B, parity,
+                               first);
         }
         // guided sampling on the first gbounces bounces (0 = all)
         const bool gsample = (P.gmode & 1u) && (P.gbounces == 0 || b < P.gbounces);
@@ -1268,26 +1373,21 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B,
                                    S, B, parity);
             if (gtrain)
                 hipLaunchKernelGGL((k_shade<true, true, false>), dim3(g_shade), dim3(kPtBlock), 0,
-                                   st, P, S, B, parity, nullptr, b == 0 ? 1 : 0);
+                                   st, P, S, B, parity, nullptr, first);
             else
                 hipLaunchKernelGGL((k_shade<true, false, false>), dim3(g_shade), dim3(kPtBlock),
-                                   0, st, P, S, B, parity, nullptr, b == 0 ? 1 : 0);
+                                   0, st, P, S, B, parity, nullptr, first);
         }
         else if (gtrain)
             hipLaunchKernelGGL((k_shade<false, true, false>), dim3(g_shade), dim3(kPtBlock), 0, st,
-                               P, S, B, parity, nullptr, b == 0 ? 1 : 0);
+                               P, S, B, parity, nullptr, first);
         else if (B.trace)
             hipLaunchKernelGGL((k_shade<false, false, false, true>), dim3(g_shade),
-                               dim3(kPtBlock), 0, st, P, S, B, parity, nullptr, b == 0 ? 1 : 0);
+                               dim3(kPtBlock), 0, st, P, S, B, parity, nullptr, first);
         else
             hipLaunchKernelGGL((k_shade<false, false, false>), dim3(g_shade), dim3(kPtBlock), 0,
-                               st, P, S, B, parity, nullptr, b == 0 ? 1 : 0);
-        if (shallow)
-            hipLaunchKernelGGL((k_shadow<16, false>), dim3(g_trav), dim3(kPtBlock), 0, st, S, B,
-                               nullptr);
-        else
-            hipLaunchKernelGGL((k_shadow<WL_BVH8_STACK_DEPTH, false>), dim3(g_trav),
-                               dim3(kPtBlock), 0, st, S, B, nullptr);
+                               st, P, S, B, parity, nullptr, first);
+        trace(parity ^ 1); // the next bounce's rays, this bounce's shadow rays
     }
     return hipGetLastError();
 }
@@ -1296,17 +1396,10 @@ static int g_multi_occ16 = 0, g_multi_occ32 = 0;
 
 void pt_multi_init()
 {
-    int &occ16 = g_multi_occ16, &occ32 = g_multi_occ32;
-    if (!occ16)
+    if (!g_multi_occ16)
     {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ16, k_extend<16, true>, kPtBlock,
-                                                         0) != hipSuccess ||
-            occ16 < 1)
-            occ16 = 4;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &occ32, k_extend<WL_BVH8_STACK_DEPTH, true>, kPtBlock, 0) != hipSuccess ||
-            occ32 < 1)
-            occ32 = 4;
+        g_multi_occ32 = blocks_per_cu(k_trace<WL_BVH8_STACK_DEPTH, true>);
+        g_multi_occ16 = blocks_per_cu(k_trace<16, true>);
     }
 }
 
@@ -1316,40 +1409,39 @@ hipError_t pt_clock_stamp(unsigned long long *dst, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t pt_run_multi(const PtMultiLaunch &L, const PtBuffers &B, int num_cus, hipStream_t st)
+hipError_t pt_run_multi(const PtMultiLaunch &L, const PtBuffers &B0, int num_cus, hipStream_t st)
 {
     pt_multi_init();
-    const int occ16 = g_multi_occ16, occ32 = g_multi_occ32;
     const uint32_t blocks_all = (L.capacity + kPtBlock - 1) / kPtBlock;
-    const uint32_t cus = (uint32_t)std::max(1, num_cus);
-    const uint32_t g_gen = std::min<uint32_t>(blocks_all, cus * 8);
-    const uint32_t g_trav = std::min<uint32_t>(blocks_all, cus * (uint32_t)(L.stack16 ? occ16 : occ32));
+    const uint32_t g_gen = grid8(blocks_all, num_cus, 8);
+    const uint32_t g_trav =
+        grid8(4 * blocks_all, num_cus, L.stack16 ? g_multi_occ16 : g_multi_occ32);
     const uint32_t g_shade =
-        std::min<uint32_t>(blocks_all, cus * std::max<uint32_t>(1, L.shade_blocks_per_cu));
+        grid8(blocks_all, num_cus, (int)std::max<uint32_t>(1, L.shade_blocks_per_cu));
     const PtParams P0{};
     const PtScene S0{};
     PtScene SA{}; // traversal: the node/triangle arena of the requests' BVHs
     SA.nodes = L.nodes;
     SA.tris = L.tris;
-    hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(64), 0, st, L);
+    PtBuffers B = B0;
+    B.segcap = pt_segment(L.capacity);
+    auto trace = [&](int parity, int first) {
+        if (L.stack16)
+            hipLaunchKernelGGL((k_trace<16, true>), dim3(g_trav), dim3(kPtBlock), 0, st, SA, B,
+                               parity, L.reqs, 0.0f, first);
+        else
+            hipLaunchKernelGGL((k_trace<WL_BVH8_STACK_DEPTH, true>), dim3(g_trav),
+                               dim3(kPtBlock), 0, st, SA, B, parity, L.reqs, 0.0f, first);
+    };
+    hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(kPtBlock), 0, st, L, B);
     hipLaunchKernelGGL(k_raygen_multi, dim3(g_gen), dim3(kPtBlock), 0, st, L, B);
+    trace(0, 1);
     for (uint32_t b = 0; b < L.max_depth; ++b)
     {
         const int parity = (int)(b & 1u);
-        if (L.stack16)
-            hipLaunchKernelGGL((k_extend<16, true>), dim3(g_trav), dim3(kPtBlock), 0, st, SA, B,
-                               parity, L.reqs, 0.0f);
-        else
-            hipLaunchKernelGGL((k_extend<WL_BVH8_STACK_DEPTH, true>), dim3(g_trav),
-                               dim3(kPtBlock), 0, st, SA, B, parity, L.reqs, 0.0f);
         hipLaunchKernelGGL((k_shade<false, false, true>), dim3(g_shade), dim3(kPtBlock), 0, st,
                            P0, S0, B, parity, L.reqs, b == 0 ? 1 : 0);
-        if (L.stack16)
-            hipLaunchKernelGGL((k_shadow<16, true>), dim3(g_trav), dim3(kPtBlock), 0, st, SA, B,
-                               L.reqs);
-        else
-            hipLaunchKernelGGL((k_shadow<WL_BVH8_STACK_DEPTH, true>), dim3(g_trav),
-                               dim3(kPtBlock), 0, st, SA, B, L.reqs);
+        trace(parity ^ 1, 0);
     }
     hipLaunchKernelGGL(k_accumulate_multi, dim3(g_gen), dim3(kPtBlock), 0, st, L, B);
     hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, L);
@@ -1383,7 +1475,7 @@ hipError_t pt_arena_copy_nodes(WlBvh8Node *dst, const WlBvh8Node *src, uint32_t 
 hipError_t pt_guide_infer_queue(const PtParams &P, const PtScene &S, const PtBuffers &B,
                                 uint32_t n, int num_cus, hipStream_t st)
 {
-    const uint32_t g = std::max<uint32_t>(1, std::min<uint32_t>((n + 63) / 64, (uint32_t)num_cus * 4));
+    const uint32_t g = grid8((n + kPtBlock - 1) / kPtBlock, num_cus, 4);
     hipLaunchKernelGGL(k_guide_infer_pt<0>, dim3(g), dim3(kPtBlock), 0, st, P, S, B, 0);
     return hipGetLastError();
 }

@@ -23,8 +23,7 @@ constexpr int kTraceBlock = 256;
 // BVHs have no room for it.
 constexpr uint32_t kTopNodes = 73;
 
-// Chunk scheduling (trav_persistent's DYN = 2): chunks of this many rays,
-// taken at run time from one counter per XCD, each counter in a cache line of
+// Chunks of this many rays (traverse_persistent.h), taken at run time from one counter per XCD, each counter in a cache line of
 // its own and each chunk asked for one ahead.  2^23 rays, closest / any hit:
 // 64: 696 / 534 us, 96: 688 / 522, 128: 691 / 521, 256: 713 / 523, 512: 730 /
 // 524 (727 / 603 us with 256 and the eight counters in one line).  A launch
@@ -53,9 +52,18 @@ __device__ __forceinline__ void load_top(uint4 *top, const WlBvh8Node *__restric
     __syncthreads();
 }
 
-__device__ __forceinline__ void load_ray(const wl_ray *__restrict__ rays, uint32_t i, TravRay &r)
+// The raw traces' chunks: XCD x owns the x-th eighth of the n rays (see
+// dyn_xcd_chunks), whose rays and hits then go through one L2.
+__device__ __forceinline__ auto eighth_chunks(uint32_t n, uint32_t chunk)
 {
-    load_ray_nt(rays, i, r);
+    const uint32_t n8 = (n + 7u) / 8u, xcd = blockIdx.x % 8u;
+    const uint32_t lo = xcd * n8 < n ? xcd * n8 : n;
+    const uint32_t hi = lo + n8 < n ? lo + n8 : n;
+    return [=](uint32_t c, uint32_t &next, uint32_t &end) {
+        const uint64_t s0 = lo + (uint64_t)c * chunk;
+        next = (uint32_t)(s0 < hi ? s0 : hi);
+        end = (uint32_t)(s0 + chunk < hi ? s0 + chunk : hi);
+    };
 }
 
 // ntop: nodes copied to LDS, min(node count, top_nodes<STACK>()); sched /
@@ -72,13 +80,12 @@ void k_trace_closest_p(
     __shared__ uint4 top[8 * (top_nodes<STACK>() ? top_nodes<STACK>() : 1)];
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
-    trav_persistent<false, kTraceBlock, STACK != 16, false, true, 0, kRefillLanes, 2,
-                    top_nodes<STACK>() != 0>(
-        nodes, tris, n, stack,
-        [&](uint32_t i, TravRay &r) { load_ray(rays, i, r); },
-        [&](uint32_t i, const TravResult &h) { store_hit_nt(hits, i, h); },
+    trav_persistent<kClosest, kTraceBlock, STACK != 16, top_nodes<STACK>() != 0>(
+        nodes, tris, stack, eighth_chunks(n, base.chunk),
+        [&](uint32_t i, TravRay &r, uint32_t &) { load_ray_nt(rays, i, r); },
+        [&](uint32_t i, const TravRay &, const TravResult &h) { store_hit_nt(hits, i, h); },
         reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u,
-        sched + kSchedStride * (blockIdx.x % 8u), base.base[blockIdx.x % 8u], base.chunk);
+        sched + kSchedStride * (blockIdx.x % 8u), base.base[blockIdx.x % 8u]);
 }
 
 template <int STACK>
@@ -91,16 +98,15 @@ void k_trace_any_p(const WlBvh8Node *__restrict__ nodes, const WlTriRecord *__re
     __shared__ uint4 top[8 * (top_nodes<STACK>() ? top_nodes<STACK>() : 1)];
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
-    trav_persistent<true, kTraceBlock, STACK != 16, false, true, 0, kRefillLanes, 2,
-                    top_nodes<STACK>() != 0>(
-        nodes, tris, n, stack,
-        [&](uint32_t i, TravRay &r) { load_ray(rays, i, r); },
-        [&](uint32_t i, const TravResult &h) {
+    trav_persistent<kAny, kTraceBlock, STACK != 16, top_nodes<STACK>() != 0>(
+        nodes, tris, stack, eighth_chunks(n, base.chunk),
+        [&](uint32_t i, TravRay &r, uint32_t &) { load_ray_nt(rays, i, r); },
+        [&](uint32_t i, const TravRay &, const TravResult &h) {
             if (h.prim != WL_INVALID)
                 atomicOr(&bits[i >> 5], 1u << (i & 31u));
         },
         reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u,
-        sched + kSchedStride * (blockIdx.x % 8u), base.base[blockIdx.x % 8u], base.chunk);
+        sched + kSchedStride * (blockIdx.x % 8u), base.base[blockIdx.x % 8u]);
 }
 
 // Instrumented closest hit: one ray per lane, per-ray node/triangle counts.
@@ -115,11 +121,11 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_closest_counted(
     const bool active = rid < n;
     TravRay r;
     if (active)
-        load_ray(rays, rid, r);
+        load_ray_nt(rays, rid, r);
     else
         trav_setup(r, 0, 0, 0, 1, 0, 0, 0, 0);
     uint32_t nn = 0, nt = 0;
-    TravResult h = trav_run<false, true, kTraceBlock>(nodes, tris, r, active, stack,
+    TravResult h = trav_run<kClosest, true, kTraceBlock>(nodes, tris, r, active, stack,
                                                      threadIdx.x, nn, nt);
     if (active)
     {
@@ -179,8 +185,7 @@ static TraceSched take_bases(wl_context_s::SchedBlock *sb, uint32_t n, uint32_t 
 }
 
 // The persistent grid for n rays in chunks of `chunk`, rounded up to a multiple
-// of 8 so that each XCD's eighth of the rays has workgroups (chunk scheduling
-// DYN = 2).
+// of 8 so that each XCD's eighth of the rays has workgroups.
 static uint32_t xcd_grid(uint32_t grid_cache, uint32_t n, uint32_t chunk)
 {
     const uint32_t per_block = chunk * (kTraceBlock / 64);

@@ -63,7 +63,8 @@ struct TravRay
     // bits 0-2: visit key, bit k clear for d_k < 0 (slots in increasing
     // slot ^ key order are near first); bits 4-6: bit 4 + k set for d_k < 0
     // (16 x bit = the byte offset of the near plane in its lo / hi pair);
-    // bits 8, 9: the largest component is x, y (else z); bit 31: it is < 0
+    // bits 8, 9: the largest component is x, y (else z); bit 31: it is < 0;
+    // bit 10: kAnyRay
     uint32_t code;
 };
 
@@ -342,9 +343,19 @@ WL_HD NodeHits node_visit(const WlBvh8Node *__restrict__ nodes, uint32_t node,
     return h;
 }
 
+// Which rays a traversal takes: closest hit, any hit, or both kinds, the
+// any-hit rays marked with kAnyRay in TravRay::code.
+enum
+{
+    kClosest = 0,
+    kAny = 1,
+    kMixed = 2
+};
+constexpr uint32_t kAnyRay = 1u << 10;
+
 // Test triangle record i; keeps the closest hit (ties to the smaller
 // primitive id).  Returns true for an accepted hit.
-template <bool ANY, bool AUX, bool WIDE>
+template <int RAYS, bool AUX, bool WIDE>
 WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t i, const TravRay &r,
                      TravState &st)
 {
@@ -363,7 +374,7 @@ WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t i, const Tra
     if (tri_test(r, w0, w1, w2, st.res.t, t, b1, b2))
     {
         const uint32_t prim = wl_f2u(w2.y);
-        if (ANY || t < st.res.t || (t == st.res.t && prim < st.res.prim))
+        if (RAYS == kAny || t < st.res.t || (t == st.res.t && prim < st.res.prim))
         {
             st.res.t = t;
             st.res.prim = prim;
@@ -380,10 +391,9 @@ WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t i, const Tra
     return false;
 }
 
-// Chunks of XCD xcd's eighth of n rays under the run-time chunk schedule of
-// the persistent trace kernels (traverse_persistent.h, DYN = 2): eighth x is
-// [x * ceil(n / 8), (x + 1) * ceil(n / 8)) clipped to n, and a launch
-// advances XCD x's counter by exactly this many.
+// The raw traces' chunks (traverse_persistent.h): XCD xcd's eighth of n rays is
+// [xcd * ceil(n / 8), (xcd + 1) * ceil(n / 8)) clipped to n, in this many
+// chunks, which is what a launch advances the XCD's counter by.
 WL_HD uint32_t dyn_xcd_chunks(uint32_t n, uint32_t xcd, uint32_t chunk)
 {
     const uint32_t n8 = (n + 7u) / 8u;
@@ -438,14 +448,15 @@ WL_HD bool trav_node(const WlBvh8Node *__restrict__ nodes, const TravRay &r, Tra
 }
 
 // One pending triangle (there must be one).  A hit of an any-hit ray ends it.
-template <bool ANY, bool AUX = false, bool WIDE = true>
+template <int RAYS, bool AUX = false, bool WIDE = true>
 WL_HD bool trav_tri(const WlTriRecord *__restrict__ tris, const TravRay &r, TravState &st)
 {
     const uint32_t b = __builtin_ctz(st.trimask);
     st.trimask &= st.trimask - 1u;
     const uint32_t i = st.tri_base + (uint32_t)__builtin_popcount(st.trivalid & ((1u << b) - 1u));
     WL_TRAV_CHECK(i < wl_trav_tris_bound, "triangle index");
-    if (tri_visit<ANY, AUX, WIDE>(tris, i, r, st) && ANY)
+    if (tri_visit<RAYS, AUX, WIDE>(tris, i, r, st) &&
+        (RAYS == kAny || (RAYS == kMixed && (r.code & kAnyRay))))
     {
         st.trimask = 0;
         st.grp_mask = 0;
@@ -460,7 +471,7 @@ WL_HD void trav_finish(TravResult &res)
 }
 
 // Traverse one ray to completion.  lane: the ray's first entry of the stack.
-template <bool ANY, bool COUNT, int BLOCK, bool AUX = false>
+template <int RAYS, bool COUNT, int BLOCK, bool AUX = false>
 WL_HD TravResult trav_run(const WlBvh8Node *__restrict__ nodes,
                           const WlTriRecord *__restrict__ tris, const TravRay &r, bool active,
                           uint32_t *lds_stack, uint32_t lane, uint32_t &n_nodes,
@@ -478,7 +489,7 @@ WL_HD TravResult trav_run(const WlBvh8Node *__restrict__ nodes,
         {
             if (COUNT)
                 ++n_tris;
-            if (trav_tri<ANY, AUX>(tris, r, st))
+            if (trav_tri<RAYS, AUX>(tris, r, st))
                 break;
         }
     }

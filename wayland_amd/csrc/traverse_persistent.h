@@ -21,12 +21,12 @@
 // (closest hit) and 679 -> 603 us (any hit), the 1080p wavefront render
 // 46.2 -> 40.9 ms, the 256 small serving requests 13.2 -> 11.5 ms.
 //
-// Each wave owns ceil(n / waves) rays (one range, or interleaved chunks) and
-// refills from a wave-uniform register, so no atomics are needed.  The
-// remapped index lb is a permutation of the workgroup indices and the chunks
-// of all waves tile [0, n), so every ray is owned by exactly one wave.  A
-// wave leaves the loop when its rays are used up and none of its lanes holds
-// a ray, so the grid always drains.
+// The rays of a launch come in chunks, a list of them per XCD: the hardware
+// deals workgroups round-robin to the 8 XCDs, each with its own L2, so XCD x's
+// workgroups are those with blockIdx % 8 == x.  An XCD's W waves start on its
+// chunks 0 .. W-1 and then each takes chunk W + k, k counted by one global
+// counter per XCD.  A wave leaves the loop when it got a chunk past its XCD's
+// last and none of its lanes holds a ray, so the grid always drains.
 #pragma once
 #include "../../include/wayland_hip.h"
 #include "traverse_device.h"
@@ -53,10 +53,7 @@ __device__ __forceinline__ void store_hit_nt(wl_hit *__restrict__ hits, uint32_t
     __builtin_nontemporal_store(v, reinterpret_cast<f4v *>(hits) + i);
 }
 
-// Default refill threshold: a wave refills once at least this many of its
-// lanes are idle (REFILL below overrides it per kernel; measured best: 16 for
-// 2^23 incoherent closest-hit and any-hit rays, 8 to 16 within noise for
-// closest hit; 16 to 28 equal for the path tracer's queues, which use 20).
+// A wave refills once at least this many of its lanes are idle.
 constexpr int kRefillLanes = 16;
 
 // Lanes that must wait for a step before a wave runs it while the other step
@@ -79,90 +76,41 @@ __device__ __forceinline__ uint32_t lane_prefix(uint64_t m)
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// fetch(i, TravRay&) sets up ray i (i < n); emit(i, const TravResult&)
-// consumes its result.  BLOCK must be a multiple of 64.  With ROOTED the
-// rays of one launch may belong to different BVHs stored back to back in one
-// node and triangle array (child and triangle indices rebased): fetch(i,
-// TravRay&, uint32_t &root) also gives the index of the ray's root node.
-// XCDMAP: the hardware deals workgroups round-robin to the 8 XCDs, each with
-// its own L2; the wave's ray range is taken from a remapped workgroup index so
-// that XCD x works on one contiguous eighth of the rays and their hits.  On
-// 2^23 incoherent rays this is 1-3 % faster for closest hit and 4 % for
-// any-hit; the path tracer's queues gain nothing from it and keep the plain
-// order.
-// CHUNKS > 0: instead of one contiguous range, wave w takes chunks w,
-// w + waves, w + 2 waves, ... of about 1/CHUNKS of its share each (at least
-// 64 rays), so waves whose share is expensive (a stretch of a multi-scene
-// queue that hits the largest BVH) get cheaper chunks too.  It suits queues
-// whose cost varies along the queue (measured best: 4 for 2^23 incoherent
-// rays, 8 for multi-request queues, 2 for the path tracer's shadow rays); the
-// path tracer's extension rays keep contiguous ranges, which keep its
-// coherent queues together.
-// top / ntop (optional): nodes [0, ntop) copied to LDS by the caller (see
+// range(c, next, end): the ray indices [next, end) of the XCD's chunk c, empty
+// past its last chunk; c and the results are wave-uniform.  fetch(i, TravRay&,
+// root) sets up ray i (root: the index of its first node, 0 unless several
+// BVHs share the node array); emit(i, const TravRay&, const TravResult&)
+// consumes its result.  RAYS: kClosest, kAny, or kMixed, where fetch marks
+// any-hit rays with kAnyRay in TravRay::code.  BLOCK must be a multiple of 64
+// and the grid a multiple of 8.
+// top / ntop (with TOP): nodes [0, ntop) copied to LDS by the caller (see
 // node_visit).
-// DYN = 2: chunks of `chunk` rays are handed out at run time instead, so a
-// wave slowed by expensive rays takes fewer chunks.  One global counter per
-// XCD (`dyn`, this XCD's): XCD x owns the x-th eighth of the rays, its waves
-// start on chunks 0 .. W-1 of that eighth (W waves per XCD; the grid is a
-// multiple of 8) and then take chunk W + (counter - base) each, base =
-// `dyn_base`, the counter's value at launch.  Every wave that had a chunk
-// makes exactly one fetch past the eighth's last chunk, so a launch advances
-// counter x by the eighth's chunk count: the host keeps the bases and nothing
-// is reset.
-template <bool ANY, int BLOCK, bool WIDE, bool ROOTED = false, bool XCDMAP = false,
-          uint32_t CHUNKS = 0, int REFILL = kRefillLanes, int DYN = 0, bool TOP = false,
-          class Fetch, class Emit>
+// dyn: this XCD's chunk counter, dyn_base its value at launch.  Every wave
+// that had a chunk makes exactly one fetch past the XCD's last, so a launch
+// advances the counter by the XCD's number of chunks.
+template <int RAYS, int BLOCK, bool WIDE, bool TOP, class Range, class Fetch, class Emit>
 __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ nodes,
                                                 const WlTriRecord *__restrict__ tris,
-                                                uint32_t n, uint32_t *stack,
-                                                Fetch fetch, Emit emit,
-                                                const WlBvh8Node *top = nullptr,
-                                                uint32_t ntop = 0, uint32_t *dyn = nullptr,
-                                                uint32_t dyn_base = 0, uint32_t chunk = 0)
+                                                uint32_t *stack, Range range, Fetch fetch,
+                                                Emit emit, const WlBvh8Node *top, uint32_t ntop,
+                                                uint32_t *dyn, uint32_t dyn_base)
 {
     static_assert(BLOCK % 64 == 0, "whole waves only");
     constexpr uint32_t kNone = 0xFFFFFFFFu;
-    const uint32_t wave_in_block = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const uint32_t waves = gridDim.x * (BLOCK / 64);
-    const uint32_t G = gridDim.x;
-    const uint32_t lb = (XCDMAP && G % 8u == 0u) ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u
-                                                 : blockIdx.x;
-    const uint32_t wave = lb * (BLOCK / 64) + wave_in_block;
-    // the wave's current range [next, end) of chunk cidx (wave-uniform)
-    const uint32_t share = (uint32_t)(((uint64_t)n + waves - 1) / waves);
-    const uint32_t C = CHUNKS == 0 ? share
-                       : share / CHUNKS > 64u ? (share + CHUNKS - 1) / CHUNKS
-                                              : 64u;
-    uint64_t cidx = wave;
-    uint32_t next, end;
-    // DYN: this wave's XCD, its eighth [xlo, xhi) of the rays and its index
-    // among the XCD's waves
-    const uint32_t xcd = blockIdx.x % 8u;
-    const uint32_t n8 = (n + 7u) / 8u;
-    const uint32_t xlo = xcd * n8 < n ? xcd * n8 : n;
-    const uint32_t xhi = xlo + n8 < n ? xlo + n8 : n;
-    const uint32_t wx = (blockIdx.x / 8u) * (BLOCK / 64) + wave_in_block;
-    const uint32_t wavesx = (G / 8u) * (BLOCK / 64);
-    // DYN: chunk c of the XCD's eighth into [next, end); a wave that got one
-    // asks for its next at once (lane 0 holds the answer, `ahead`), so the
-    // atomic's latency passes behind the chunk's own rays
-    uint32_t ahead = 0;
+    // this wave among its XCD's
+    const uint32_t wx = (blockIdx.x / 8u) * (BLOCK / 64) +
+                        __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t wavesx = (gridDim.x / 8u) * (BLOCK / 64);
+    // chunk c into [next, end); a wave that got one asks for its next at once
+    // (lane 0 holds the answer, `ahead`), so the atomic's latency passes behind
+    // the chunk's own rays
+    uint32_t next, end, ahead = 0;
     auto take_chunk = [&](uint32_t c) {
-        static_assert(DYN == 0 || DYN == 2, "DYN is 0 or 2");
-        const uint64_t s0 = xlo + (uint64_t)c * chunk;
-        next = (uint32_t)(s0 < xhi ? s0 : xhi);
-        end = (uint32_t)(s0 + chunk < xhi ? s0 + chunk : xhi);
+        range(c, next, end);
         if (next < end && __lane_id() == 0)
             ahead = atomicAdd(dyn, 1u);
     };
-    if constexpr (DYN != 0)
-        take_chunk(wx);
-    else
-    {
-        const uint64_t s0 = cidx * C;
-        next = (uint32_t)(s0 < n ? s0 : n);
-        end = (uint32_t)(s0 + C < n ? s0 + C : n);
-    }
+    take_chunk(wx);
     TravRay r;
     trav_setup(r, 0, 0, 0, 1, 0, 0, 0, 0);
     TravState st;
@@ -172,13 +120,13 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
     {
         const uint64_t busy = __ballot(!trav_done(st));
         const uint32_t nidle = (uint32_t)lane_count(~busy);
-        if ((next < end && nidle >= (uint32_t)REFILL) || busy == 0)
+        if ((next < end && nidle >= (uint32_t)kRefillLanes) || busy == 0)
         {
             const bool idle = trav_done(st);
             if (idle && rid != kNone)
             {
                 trav_finish(st.res);
-                emit(rid, st.res);
+                emit(rid, r, st.res);
                 rid = kNone;
             }
             if (next >= end)
@@ -190,23 +138,13 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
                 {
                     rid = k;
                     uint32_t root = 0;
-                    if constexpr (ROOTED)
-                        fetch(rid, r, root);
-                    else
-                        fetch(rid, r);
+                    fetch(rid, r, root);
                     trav_init(st, r, true, threadIdx.x, root);
                 }
             }
             next = next + nidle < end ? next + nidle : end;
-            if (DYN != 0 && next >= end)
+            if (next >= end)
                 take_chunk(wavesx + __builtin_amdgcn_readfirstlane(ahead) - dyn_base);
-            else if (DYN == 0 && CHUNKS != 0 && next >= end)
-            {
-                cidx += waves;
-                const uint64_t s0 = cidx * C;
-                next = (uint32_t)(s0 < n ? s0 : n);
-                end = (uint32_t)(s0 + C < n ? s0 + C : n);
-            }
         }
         // a lane with a pending triangle takes the triangle step next, any
         // other unfinished lane the node step
@@ -215,7 +153,7 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
         const bool last = next >= end;
         const bool tri = nt >= kTriLanes || (nt > 0 && (last || nn < kNodeLanes));
         if (tri && st.trimask != 0)
-            trav_tri<ANY, false, WIDE>(tris, r, st);
+            trav_tri<RAYS, false, WIDE>(tris, r, st);
         const bool can = st.trimask == 0 && st.grp_mask != 0;
         const int nn2 = lane_count(__ballot(can));
         if ((!tri || last || nn2 >= kNodeLanes) && can)

@@ -82,6 +82,21 @@ struct PtParams
 };
 
 // Path state (structure of float4 arrays, one entry per path) and queues.
+// Counters of a batch: for XCD x the 64-bit lengths of its segments of the two
+// ray queues (parity 0, 1; low word rays, high word shadow rays) and its chunk
+// counter, each in a cache line of its own: word kPtCounterStride * (4 x + 0, 1,
+// 2).  kPtFlatCount: the length of the first queue, which has no segments.
+constexpr uint32_t kPtCounterStride = 32;
+constexpr uint32_t kPtCounters = 8 * 4 * kPtCounterStride;
+constexpr uint32_t kPtFlatCount = 3 * kPtCounterStride;
+
+// Entries of one of the eight queue segments of a batch of n paths: the shade
+// pass takes an XCD's entries in workgroups of 256, and every entry appends at
+// most one to each queue.
+constexpr uint32_t pt_segment(uint64_t n) { return (uint32_t)(((n + 255) / 256 + 7) / 8 * 256); }
+// Entries of a whole queue of a batch of n paths.
+constexpr size_t pt_queue_entries(uint64_t n) { return 8 * (size_t)pt_segment(n); }
+
 struct PtBuffers
 {
     float4 *thr;      // throughput, w = depth (bits 0-15), guided vertices (16-31)
@@ -98,7 +113,8 @@ struct PtBuffers
     uint32_t *qreq0, *qreq1, *sreq; // multi-request batches: request of each
                                     // ray queue slot / BVH root (node arena
                                     // index) of each shadow queue slot
-    uint32_t *counters;       // [0], [1] active queues, [2] shadow queue
+    uint32_t *counters;       // kPtCounters words: queue lengths, chunk counters
+    uint32_t segcap;          // entries of a queue segment (set per batch)
     unsigned long long *stats; // [0] extension rays, [1] shadow rays
     // learned guiding (only with PtParams::gmode != 0)
     float *gout;      // decoded mixture, 48 floats per queue slot

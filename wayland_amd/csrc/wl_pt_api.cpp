@@ -29,23 +29,24 @@ PtBuffers pt_carve(void *base, size_t cap, uint32_t *counters, unsigned long lon
         p += (bytes + 255) & ~(size_t)255;
         return (void *)q;
     };
+    const size_t q = pt_queue_entries(cap);
     B.thr = (float4 *)take(16 * cap);
     B.ltt = (float4 *)take(16 * cap);
     B.rad = (float4 *)take(16 * cap);
-    B.rays0 = (wl_ray *)take(32 * cap);
-    B.rays1 = (wl_ray *)take(32 * cap);
-    B.qpath0 = (uint32_t *)take(4 * cap);
-    B.qpath1 = (uint32_t *)take(4 * cap);
-    B.hits = (wl_hit *)take(16 * cap);
-    B.srays = (wl_ray *)take(32 * cap);
-    B.spath = (uint32_t *)take(4 * cap);
-    B.scontrib = (float4 *)take(16 * cap);
-    B.sort_keys = (uint32_t *)take(4 * cap);
-    B.sort_perm = (uint32_t *)take(4 * cap);
+    B.rays0 = (wl_ray *)take(32 * q);
+    B.rays1 = (wl_ray *)take(32 * q);
+    B.qpath0 = (uint32_t *)take(4 * q);
+    B.qpath1 = (uint32_t *)take(4 * q);
+    B.hits = (wl_hit *)take(16 * q);
+    B.srays = (wl_ray *)take(32 * q);
+    B.spath = (uint32_t *)take(4 * q);
+    B.scontrib = (float4 *)take(16 * q);
+    B.sort_keys = (uint32_t *)take(4 * q);
+    B.sort_perm = (uint32_t *)take(4 * q);
     B.sort_bins = (uint32_t *)take(4 * 2048);
-    B.qreq0 = (uint32_t *)take(4 * cap);
-    B.qreq1 = (uint32_t *)take(4 * cap);
-    B.sreq = (uint32_t *)take(4 * cap);
+    B.qreq0 = (uint32_t *)take(4 * q);
+    B.qreq1 = (uint32_t *)take(4 * q);
+    B.sreq = (uint32_t *)take(4 * q);
     B.counters = counters;
     B.stats = stats;
     return B;
@@ -54,7 +55,8 @@ PtBuffers pt_carve(void *base, size_t cap, uint32_t *counters, unsigned long lon
 size_t pt_batch_bytes(size_t cap)
 {
     auto r = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    return r(16 * cap) * 3 + r(32 * cap) * 3 + r(4 * cap) * 8 + r(16 * cap) * 2 + r(4 * 2048);
+    const size_t q = pt_queue_entries(cap);
+    return r(16 * cap) * 3 + r(32 * q) * 3 + r(4 * q) * 8 + r(16 * q) * 2 + r(4 * 2048);
 }
 
 PtScene pt_scene_view(wl_scene s)
@@ -122,7 +124,7 @@ wl::PtBuffers carve(wl_scene s)
     {
         char *g = (char *)s->d_gbatch;
         B.gout = (float *)g;
-        g += (192 * cap + 255) & ~(size_t)255;
+        g += (192 * wl::pt_queue_entries(cap) + 255) & ~(size_t)255;
         B.gacc = (float4 *)g;
         g += (16 * cap + 255) & ~(size_t)255;
         B.grec = (float *)g;
@@ -140,7 +142,7 @@ size_t batch_bytes(size_t cap) { return wl::pt_batch_bytes(cap); }
 size_t guide_batch_bytes(size_t cap)
 {
     auto r = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    return r(192 * cap) + r(16 * cap) + r(64 * cap);
+    return r(192 * wl::pt_queue_entries(cap)) + r(16 * cap) + r(64 * cap);
 }
 
 wl_status ensure_capacity(wl_scene s, uint32_t paths)
@@ -183,7 +185,7 @@ wl_status ensure_lane2(wl_scene s, uint32_t paths)
     if (!s->ev_join)
         WL_HIP_CHECK(hipEventCreateWithFlags(&s->ev_join, hipEventDisableTiming));
     if (!s->d_counters2)
-        WL_HIP_CHECK(hipMalloc((void **)&s->d_counters2, 64));
+        WL_HIP_CHECK(hipMalloc((void **)&s->d_counters2, 4 * wl::kPtCounters));
     if (!s->d_stats2)
         WL_HIP_CHECK(hipMalloc((void **)&s->d_stats2, 64));
     if (paths <= s->capacity2)
@@ -393,7 +395,7 @@ wl_status wl_scene_create(wl_context ctx, wl_accel accel,
     up((void **)&s->d_materials, mats.data(), mats.size() * sizeof(wl_disney_material));
     up(&s->d_lights, hl.data(), hl.size() * sizeof(wl::PtLight));
     if (e == hipSuccess)
-        e = hipMalloc((void **)&s->d_counters, 64);
+        e = hipMalloc((void **)&s->d_counters, 4 * wl::kPtCounters);
     if (e == hipSuccess)
         e = hipMalloc((void **)&s->d_stats, 64);
     if (e != hipSuccess)
@@ -829,9 +831,10 @@ wl_status wl_guide_infer_hits(wl_scene s, const wl_ray *rays, const wl_hit *hits
     wl::PtBuffers B{};
     B.rays0 = const_cast<wl_ray *>(rays);
     B.hits = const_cast<wl_hit *>(hits);
-    B.counters = s->d_counters; // the kernel reads the queue length from here
+    B.counters = s->d_counters; // the kernel reads the first queue's length from here
     B.gout = decoded;
-    WL_HIP_CHECK(hipMemcpyAsync(s->d_counters, &n, sizeof n, hipMemcpyHostToDevice, hs));
+    WL_HIP_CHECK(hipMemcpyAsync(s->d_counters + wl::kPtFlatCount, &n, sizeof n,
+                                hipMemcpyHostToDevice, hs));
     WL_HIP_CHECK(wl::pt_guide_infer_queue(P, scene_view(s), B, n, s->ctx->num_cus, hs));
     WL_HIP_CHECK(hipStreamSynchronize(hs)); // n is read from host memory
     return WL_SUCCESS;

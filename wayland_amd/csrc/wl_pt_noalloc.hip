@@ -20,13 +20,15 @@
 namespace
 {
 constexpr uint32_t kMaxPaths = WL_PT_NOALLOC_MAX_BATCH_PATHS;
-// header: queue counters at byte 0 (16 words), path / ray statistics at 128
-constexpr size_t kHeaderBytes = 256;
+// header: queue counters at byte 0, path / ray statistics behind them
+constexpr size_t kStatsAt = 4 * wl::kPtCounters;
+constexpr size_t kHeaderBytes = kStatsAt + 256;
+constexpr size_t kQueue = wl::pt_queue_entries(kMaxPaths);
 constexpr size_t r256(size_t b) { return (b + 255) & ~(size_t)255; }
 // the carve of wl::pt_carve for kMaxPaths paths (checked against
 // wl::pt_batch_bytes at set-up)
-constexpr size_t kBatchBytes = r256(16ull * kMaxPaths) * 3 + r256(32ull * kMaxPaths) * 3 +
-                               r256(4ull * kMaxPaths) * 8 + r256(16ull * kMaxPaths) * 2 +
+constexpr size_t kBatchBytes = r256(16ull * kMaxPaths) * 3 + r256(32ull * kQueue) * 3 +
+                               r256(4ull * kQueue) * 8 + r256(16ull * kQueue) * 2 +
                                r256(4ull * 2048);
 constexpr size_t kScratchBytes = kHeaderBytes + kBatchBytes;
 constexpr int kMaxDevices = 64;
@@ -41,8 +43,7 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 // be captured into a graph).
 __global__ void k_noalloc_clear(uint32_t *header)
 {
-    const uint32_t i = threadIdx.x;
-    if (i < kHeaderBytes / 4)
+    for (uint32_t i = threadIdx.x; i < kHeaderBytes / 4; i += blockDim.x)
         header[i] = 0u;
 }
 
@@ -102,8 +103,8 @@ extern "C" wl_status wl_pt_render_noalloc(wl_scene s, const wl_pt_config *c, flo
     const uint32_t ns = std::max<uint32_t>(1, std::min<uint32_t>(c->spp, cap / tile));
     char *b = (char *)base;
     uint32_t *counters = (uint32_t *)b;
-    unsigned long long *stats = (unsigned long long *)(b + 128);
-    hipLaunchKernelGGL(k_noalloc_clear, dim3(1), dim3(kHeaderBytes / 4), 0, hs, counters);
+    unsigned long long *stats = (unsigned long long *)(b + kStatsAt);
+    hipLaunchKernelGGL(k_noalloc_clear, dim3(1), dim3(256), 0, hs, counters);
     const wl::PtBuffers B = wl::pt_carve(b + kHeaderBytes, (size_t)tile * ns, counters, stats);
     const wl::PtScene S = wl::pt_scene_view(s);
     for (uint32_t s0 = 0; s0 < c->spp; s0 += ns)

@@ -542,7 +542,7 @@ wl_status create_server(wl_context ctx, const wl_serve_config &c, wl_server *out
     wl::ctx_retain(ctx);
     hipError_t e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
     if (e == hipSuccess)
-        e = hipMalloc((void **)&s->d_counters, 64);
+        e = hipMalloc((void **)&s->d_counters, 4 * wl::kPtCounters);
     if (e == hipSuccess)
         e = hipMalloc((void **)&s->d_stats, 64);
     if (e == hipSuccess)

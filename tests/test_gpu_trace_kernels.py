@@ -99,3 +99,34 @@ def test_batch_sizes_around_the_queue_segments(gpu_ctx, width, sort):
     b, _ = pt.render(wl.pt_config(width, 1, max_batch_paths=64, **kw), stats=False)
     assert torch.equal(a, b)
     assert (a[:, 0:3] != 0).any()
+
+
+@pytest.mark.parametrize("strategy", [0, 1, 2])
+def test_plain_materials_keep_every_bit(gpu_ctx, strategy):
+    """Materials without transmission, clearcoat, sheen, tint or subsurface are
+    shaded without those terms.  The same materials with a clearcoat gloss
+    outside [0, 1] (which a clearcoat of 0 multiplies away) take the general
+    expressions: the films are bit-identical, at the ends of the accepted
+    ranges too, and beside glass."""
+    import torch
+    import wayland_amd as wl
+    films = []
+    for gloss in (1.0, 1.5):
+        sc = scenes.wavefront_scene(12, 3, width=160, height=120)
+        rng = np.random.default_rng(4)
+        k = 0
+        for m in sc.meshes:
+            if m.light_L is not None:
+                continue
+            m.material = scenes.disney_material(
+                color=rng.uniform(0, 1, 3) * (k % 5 > 0), metallic=(0.0, 1.0, 0.3)[k % 3],
+                roughness=(0.01, 0.5, 1.0, 10.0)[k % 4], specular=(0.0, 0.5, 2.0)[k % 3],
+                eta=(0.99, 1.01, 1.5, 0.02, 50.0)[k % 5], trans=1.0 if k % 6 == 5 else 0.0,
+                clearcoatgloss=gloss if k % 6 != 5 else 1.0)
+            k += 1
+        pt = wl.PathTracer(gpu_ctx, wl.Accel(gpu_ctx, sc), sc)
+        film, _ = pt.render(wl.pt_config(160, 120, spp=16, max_depth=10, strategy=strategy),
+                            stats=False)
+        films.append(film)
+    assert torch.equal(films[0].view(torch.int32), films[1].view(torch.int32))
+    assert (films[0][:, 0:3] != 0).any()

@@ -614,8 +614,14 @@ void k_guide_infer_pt(PtParams P, PtScene S, PtBuffers B, int parity)
 // GTRAIN: paths carry guide training records (radiance after the recorded
 // vertex is summed; GSAMPLE vertices record themselves).
 // TRACE: also writes the per-vertex record of PtBuffers::trace.
+// The pass is bound by VALU issue (81 % busy on the 2M-triangle scene), so what
+// counts is the instructions of the BSDF: with the terms that vanish for plain
+// materials behind a branch and one sine and cosine for all lobes, two 1024^2
+// Cornell frames 2.53 -> 2.32 ms, 256 small serving requests 9.2 -> 8.8 ms.  Four
+// waves per SIMD: five (96 VGPRs, no spills) is 2-6 % slower.
 template <bool GSAMPLE, bool GTRAIN, bool MULTI, bool TRACE = false>
-__global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ __launch_bounds__(kPtBlock)
+__attribute__((amdgpu_waves_per_eu(GSAMPLE || GTRAIN ? 3 : 4)))
 void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__restrict__ reqs,
              int first)
 {

@@ -135,6 +135,10 @@ struct Mat
     V3 color;
     float metallic, roughness, specular, specularTint, eta, trans, subsurface,
         anisotropic, sheen, sheenTint, clearcoat, clearcoatgloss;
+    // the library's mark (pad_ of its copy of the material, material_plain in
+    // wl_pt_api.cpp): the transmissive, clearcoat, sheen, tint and subsurface
+    // terms below are exact zeros times finite values
+    bool plain;
 };
 
 WL_DEV Mat load_mat(const wl_disney_material *__restrict__ p)
@@ -155,6 +159,7 @@ WL_DEV Mat load_mat(const wl_disney_material *__restrict__ p)
     m.sheenTint = d.x;
     m.clearcoat = d.y;
     m.clearcoatgloss = d.z;
+    m.plain = d.w != 0.0f;
     return m;
 }
 
@@ -191,7 +196,9 @@ WL_DEV V3 eval_transmit(const Mat &mat, V3 Ns, V3 V, V3 L, V3 tex)
     return ((1 - refract) * (1.f - F)) * T * fabsf(num / den);
 }
 
-// Disney BSDF value (reference Evaluate.h:78-191).
+// Disney BSDF value (reference Evaluate.h:78-191).  Terms that vanish for a
+// plain material are computed only where a lane needs them: adding them would
+// add +0 or multiply by 1, so the value is the same to the bit.
 WL_DEV V3 eval_disney(const Mat &mat, V3 Ns, V3 Ng, V3 V, V3 L, V3 tex)
 {
     V3 combined = tex * mat.color;
@@ -199,7 +206,6 @@ WL_DEV V3 eval_disney(const Mat &mat, V3 Ns, V3 Ng, V3 V, V3 L, V3 tex)
     float gNDotL = dot(Ng, L);
     float NDotV = dot(Ns, V);
     float gNDotV = dot(Ng, V);
-    float eta = 1 / mat.eta;
     if (mat.trans < 0.1f && (gNDotL * gNDotV <= 0.0f || NDotL * NDotV <= 0))
         return mk(0, 0, 0);
     if (mat.trans > 0.9f && (gNDotL * gNDotV * NDotL * NDotV <= 0))
@@ -208,49 +214,61 @@ WL_DEV V3 eval_disney(const Mat &mat, V3 Ns, V3 Ng, V3 V, V3 L, V3 tex)
         return eval_transmit(mat, Ns, V, L, tex);
     if (mat.metallic + combined.x + combined.y + combined.z <= 0)
         return mk(0, 0, 0);
-    if (NDotL < 0.0f && NDotV < 0.0f)
+    const bool below = NDotL < 0.0f && NDotV < 0.0f;
+    if (below)
     {
         Ns = -Ns;
-        eta = 1 / eta;
         NDotL *= -1;
         NDotV *= -1;
     }
     V3 H = normalize(L + V);
     float NDotH = dot(Ns, H);
     float LDotH = dot(L, H);
-    float refract = ((1 - NDotV * NDotV) * eta * eta >= 1) ? 1.0f : 0.0f;
     V3 Cdlin = combined;
-    float Cdlum = 0.3f * Cdlin.x + 0.6f * Cdlin.y + 0.1f * Cdlin.z;
-    V3 Ctint = Cdlum > 0.0f ? Cdlin / Cdlum : mk(1, 1, 1);
-    V3 Cspec0 = lerp3((mat.specular * 0.08f) * lerp3(mk(1, 1, 1), Ctint, mat.specularTint),
-                      Cdlin, mat.metallic);
-    V3 Csheen = lerp3(mk(1, 1, 1), Ctint, mat.sheenTint);
     float FL = schlick(NDotL), FV = schlick(NDotV);
     float Fd90 = 0.5f + 2.0f * LDotH * LDotH * mat.roughness;
     float Fd = lerpf(1.0f, Fd90, FL) * lerpf(1.0f, Fd90, FV);
-    float Fss90 = LDotH * LDotH * mat.roughness;
-    float Fss = lerpf(1.0f, Fss90, FL) * lerpf(1.0f, Fss90, FV);
-    float ss = 1.25f * (Fss * (1.0f / (NDotL + NDotV) - 0.5f) + 0.5f);
     float a = fmaxf(0.001f, mat.roughness);
     float Ds = gtr2(NDotH, a);
     float FH = schlick(LDotH);
-    V3 Fs = lerp3(Cspec0, mk(1, 1, 1), FH);
     float roughg = sqrtf(mat.roughness * 0.5f + 0.5f);
     float Gs = smithg(NDotL, roughg) * smithg(NDotV, roughg);
-    V3 Fsheen = (FH * mat.sheen) * Csheen;
-    float trans = mat.trans;
-    float cosThetaI = fabsf(dot(Ns, V));
-    float sin2ThetaI = 1 - cosThetaI * cosThetaI;
-    float sin2ThetaT = eta * eta * sin2ThetaI;
-    float cosThetaT = 1;
-    if (sin2ThetaT <= 1)
-        cosThetaT = sqrtf(1 - sin2ThetaT);
-    float F = fresnel(cosThetaI, cosThetaT, eta);
-    V3 out = ((((1.0f / kPi) * lerpf(Fd, ss, mat.subsurface)) * Cdlin + Fsheen) *
-              (1.0f - mat.metallic)) *
-             (1 - trans * (1 - F) * (1 - refract));
-    if (trans > 0)
-        out = add_scalar(out, Gs * Ds * (1 - trans * (1 - refract) * (1 - F)));
+    // plain: the specular tint of lerp3(1, Ctint, 0), no sheen, no subsurface
+    // (ss is finite unless NDotL + NDotV is tiny), a transmission factor of 1
+    V3 spec = mk(1, 1, 1), Fsheen = mk(0, 0, 0);
+    float diffuse = Fd, keep = 1.0f, keep_spec = 1.0f;
+    const bool plain = mat.plain && NDotL + NDotV > 1e-20f;
+    if (!plain)
+    {
+        float eta = 1 / mat.eta;
+        if (below)
+            eta = 1 / eta;
+        float refract = ((1 - NDotV * NDotV) * eta * eta >= 1) ? 1.0f : 0.0f;
+        float Cdlum = 0.3f * Cdlin.x + 0.6f * Cdlin.y + 0.1f * Cdlin.z;
+        V3 Ctint = Cdlum > 0.0f ? Cdlin / Cdlum : mk(1, 1, 1);
+        spec = lerp3(mk(1, 1, 1), Ctint, mat.specularTint);
+        V3 Csheen = lerp3(mk(1, 1, 1), Ctint, mat.sheenTint);
+        float Fss90 = LDotH * LDotH * mat.roughness;
+        float Fss = lerpf(1.0f, Fss90, FL) * lerpf(1.0f, Fss90, FV);
+        float ss = 1.25f * (Fss * (1.0f / (NDotL + NDotV) - 0.5f) + 0.5f);
+        diffuse = lerpf(Fd, ss, mat.subsurface);
+        Fsheen = (FH * mat.sheen) * Csheen;
+        float trans = mat.trans;
+        float cosThetaI = fabsf(dot(Ns, V));
+        float sin2ThetaI = 1 - cosThetaI * cosThetaI;
+        float sin2ThetaT = eta * eta * sin2ThetaI;
+        float cosThetaT = 1;
+        if (sin2ThetaT <= 1)
+            cosThetaT = sqrtf(1 - sin2ThetaT);
+        float F = fresnel(cosThetaI, cosThetaT, eta);
+        keep = 1 - trans * (1 - F) * (1 - refract);
+        keep_spec = 1 - trans * (1 - refract) * (1 - F);
+    }
+    V3 Cspec0 = lerp3((mat.specular * 0.08f) * spec, Cdlin, mat.metallic);
+    V3 Fs = lerp3(Cspec0, mk(1, 1, 1), FH);
+    V3 out = ((((1.0f / kPi) * diffuse) * Cdlin + Fsheen) * (1.0f - mat.metallic)) * keep;
+    if (mat.trans > 0)
+        out = add_scalar(out, Gs * Ds * keep_spec);
     else
         out = out + (Gs * Ds) * Fs;
     return out;
@@ -260,6 +278,28 @@ WL_DEV V3 eval_disney(const Mat &mat, V3 Ns, V3 Ng, V3 V, V3 L, V3 tex)
 // (reference Pdf.h:42-118).
 WL_DEV float pdf_disney(const Mat &mat, V3 Ns, V3 V, V3 L)
 {
+    float diffuseRatio = 0.5f * (1.f - mat.metallic);
+    float specularRatio = 1.f - diffuseRatio;
+    V3 half = normalize(L + V);
+    float cosTheta = fabsf(dot(half, Ns));
+    float pdfGTR2 = gtr2(cosTheta, mat.roughness) * cosTheta;
+    float pdfDiff = fabsf(dot(L, Ns)) * (1.f / kPi);
+    // plain: no clearcoat, so the specular density is lerpf(GTR1, GTR2, 1) with a
+    // finite GTR1 (its denominator is positive for cosTheta up to here), and
+    // the transmissive terms add zero to a finite density
+    float pdfLobe = pdfGTR2;
+    const bool plain = mat.plain && cosTheta <= 1.0000002f;
+    if (!plain)
+    {
+        float clearcoatAlpha = lerpf(0.1f, 0.001f, mat.clearcoatgloss);
+        float pdfGTR1 = gtr1(cosTheta, clearcoatAlpha) * cosTheta;
+        float ratio = 1.0f / (1.0f + mat.clearcoat);
+        pdfLobe = lerpf(pdfGTR1, pdfGTR2, ratio);
+    }
+    float pdfSpec = pdfLobe / (4.0f * fabsf(dot(L, half)));
+    float base = diffuseRatio * pdfDiff + specularRatio * pdfSpec;
+    if (plain && base < 3.0e38f)
+        return base;
     float transRatio = mat.trans;
     float eta = mat.eta;
     if (dot(Ns, V) < 0)
@@ -269,16 +309,6 @@ WL_DEV float pdf_disney(const Mat &mat, V3 Ns, V3 V, V3 L)
     }
     float NdotV = fabsf(dot(V, Ns));
     V3 wh = -normalize(V + L * eta);
-    float clearcoatAlpha = lerpf(0.1f, 0.001f, mat.clearcoatgloss);
-    float diffuseRatio = 0.5f * (1.f - mat.metallic);
-    float specularRatio = 1.f - diffuseRatio;
-    V3 half = normalize(L + V);
-    float cosTheta = fabsf(dot(half, Ns));
-    float pdfGTR2 = gtr2(cosTheta, mat.roughness) * cosTheta;
-    float pdfGTR1 = gtr1(cosTheta, clearcoatAlpha) * cosTheta;
-    float ratio = 1.0f / (1.0f + mat.clearcoat);
-    float pdfSpec = lerpf(pdfGTR1, pdfGTR2, ratio) / (4.0f * fabsf(dot(L, half)));
-    float pdfDiff = fabsf(dot(L, Ns)) * (1.f / kPi);
     float cosThetaI = fabsf(dot(wh, V));
     float sin2ThetaI = 1 - cosThetaI * cosThetaI;
     float sin2ThetaT = 1 / (eta * eta) * sin2ThetaI;
@@ -286,7 +316,7 @@ WL_DEV float pdf_disney(const Mat &mat, V3 Ns, V3 V, V3 L)
     float temp = (1 - NdotV * NdotV) / (eta * eta);
     if (temp < 1)
         refractRatio = 1 - fresnel(NdotV, sqrtf(1 - temp), eta);
-    float pdf = (diffuseRatio * pdfDiff + specularRatio * pdfSpec) * (1 - transRatio * refractRatio);
+    float pdf = base * (1 - transRatio * refractRatio);
     if (sin2ThetaT <= 1 && dot(L, wh) * dot(V, wh) < 0)
     {
         float sqrtDenom = eta * dot(L, wh) + dot(V, wh);
@@ -300,82 +330,85 @@ WL_DEV float pdf_disney(const Mat &mat, V3 Ns, V3 V, V3 L)
     sin2ThetaI = 1 - cosThetaI * cosThetaI;
     sin2ThetaT = 1 / (eta * eta) * sin2ThetaI;
     if (sin2ThetaT > 1)
-        pdf += (diffuseRatio * pdfDiff + specularRatio * pdfSpec) * transRatio * refractRatio;
+        pdf += base * transRatio * refractRatio;
     return pdf;
 }
 
 // Direction sampling, 7 draws (+2 on the diffuse lobe) in the reference's
 // order (reference Sample.h:134-231, 24-28, 43-53).
+// The three lobes differ in the numbers they take; the azimuth's sine and
+// cosine, the GGX cosine and the frame are computed once for all of them
+// (a wave holds lanes of every lobe).
 WL_DEV V3 sample_disney(const Mat &mat, V3 Ns, V3 V, uint32_t &seed)
 {
     float r1 = rnd(seed);
     float r2 = rnd(seed);
     float r3 = rnd(seed);
     float r4 = rnd(seed);
-    float eta = 1 / mat.eta;
-    if (dot(Ns, V) < 0)
-    {
-        eta = 1 / eta;
+    const bool back = dot(Ns, V) < 0;
+    if (back)
         Ns = -Ns;
-    }
-    float NdotV = fabsf(dot(Ns, V));
     float transprob = rnd(seed);
     float refractprob = rnd(seed);
     float probability = rnd(seed);
     float diffuseRatio = 0.5f * (1.0f - mat.metallic);
+    float eta = 1.0f;
+    bool transmit = false;
     if (transprob < mat.trans)
     {
+        eta = 1 / mat.eta;
+        if (back)
+            eta = 1 / eta;
+        float NdotV = fabsf(dot(Ns, V));
         float refractRatio = 0;
         float temp = (1 - NdotV * NdotV) * (eta * eta);
         if (temp < 1)
             refractRatio = 1 - fresnel(NdotV, sqrtf(1 - temp), eta);
-        if (refractprob < refractRatio)
-        {
-            V3 Ox, Oy;
-            onb(Ns, Ox, Oy);
-            float a = mat.roughness;
-            float phi = r3 * kTwoPi;
-            float cosTheta = sqrtf((1.0f - r4) / (1.0f + (a * a - 1.0f) * r4));
-            float sinTheta = sqrtf(1.0f - (cosTheta * cosTheta));
-            float sinPhi = sinf(phi);
-            float cosPhi = cosf(phi);
-            V3 half = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
-            half = half.x * Ox + half.y * Oy + half.z * Ns;
-            if (dot(V, Ns) == 0)
-                return -V;
-            float cosThetaI = dot(half, V);
-            float sin2ThetaI = 1 - cosThetaI * cosThetaI;
-            float sin2ThetaT = eta * eta * sin2ThetaI;
-            if (sin2ThetaT <= 1)
-            {
-                float cosThetaT = sqrtf(1 - sin2ThetaT);
-                V3 L = normalize(eta * -V + (eta * cosThetaI - cosThetaT) * half);
-                if (cosThetaI < 0)
-                {
-                    float LdotH = dot(L, half);
-                    L = L - (2 * LdotH) * half;
-                }
-                return L;
-            }
-            return half * 2.f * dot(half, V) - V;
-        }
+        transmit = refractprob < refractRatio;
     }
+    const bool diffuse = !transmit && probability < diffuseRatio;
+    float rad = 0.0f, azimuth = transmit ? r3 : r1, elevation = transmit ? r4 : r2;
+    if (diffuse)
+    {
+        rad = rnd(seed);
+        azimuth = rnd(seed);
+    }
+    const float phi = azimuth * kTwoPi;
+    const float sinPhi = sinf(phi), cosPhi = cosf(phi);
     V3 Ox, Oy;
     onb(Ns, Ox, Oy);
-    if (probability < diffuseRatio)
+    if (diffuse)
     {
-        float r = sqrtf(rnd(seed)), theta = rnd(seed) * kTwoPi;
-        float dx = r * cosf(theta), dy = r * sinf(theta);
+        float r = sqrtf(rad);
+        float dx = r * cosPhi, dy = r * sinPhi;
         float z = sqrtf(1 - dx * dx - dy * dy);
         return Ox * dx + Oy * dy + Ns * z;
     }
     float a = mat.roughness;
-    float phi = r1 * kTwoPi;
-    float cosTheta = sqrtf((1.0f - r2) / (1.0f + (a * a - 1.0f) * r2));
+    float cosTheta = sqrtf((1.0f - elevation) / (1.0f + (a * a - 1.0f) * elevation));
     float sinTheta = sqrtf(1.0f - (cosTheta * cosTheta));
-    float sinPhi = sinf(phi);
-    float cosPhi = cosf(phi);
     V3 half = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
+    if (transmit)
+    {
+        half = half.x * Ox + half.y * Oy + half.z * Ns;
+        if (dot(V, Ns) == 0)
+            return -V;
+        float cosThetaI = dot(half, V);
+        float sin2ThetaI = 1 - cosThetaI * cosThetaI;
+        float sin2ThetaT = eta * eta * sin2ThetaI;
+        if (sin2ThetaT <= 1)
+        {
+            float cosThetaT = sqrtf(1 - sin2ThetaT);
+            V3 L = normalize(eta * -V + (eta * cosThetaI - cosThetaT) * half);
+            if (cosThetaI < 0)
+            {
+                float LdotH = dot(L, half);
+                L = L - (2 * LdotH) * half;
+            }
+            return L;
+        }
+        return half * 2.f * dot(half, V) - V;
+    }
     half = half.z * Ns + half.x * Ox + half.y * Oy;
     return (2.0f * dot(V, half)) * half - V;
 }

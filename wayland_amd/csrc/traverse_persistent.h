@@ -9,7 +9,7 @@
 //
 // Each pass of the loop runs the triangle step, the node step or both, for the
 // lanes that can take it.  The kernels are bound by VALU issue (a node step is
-// about 170 instructions, a triangle step about 120, whatever the number of
+// about 165 instructions, a triangle step about 120, whatever the number of
 // lanes in it), so a step waits until enough lanes need it: the triangle step
 // until kTriLanes hold a pending triangle, the node step until kNodeLanes can
 // take a node, unless nothing else can run.  Once the wave's rays are used up
@@ -59,7 +59,7 @@ constexpr int kRefillLanes = 16;
 // Lanes that must wait for a step before a wave runs it while the other step
 // has work (see above).
 constexpr int kTriLanes = 16;
-constexpr int kNodeLanes = 24;
+constexpr int kNodeLanes = 40;
 
 // Number of lanes in m, kept in a scalar register (a compare of the 64-bit
 // count would go to the vector unit).

@@ -137,6 +137,24 @@ wl::PtBuffers carve(wl_scene s)
     return B;
 }
 
+// Whether the shade pass may leave out the material's transmissive, clearcoat,
+// sheen, tint and subsurface terms (Mat::plain in shading_device.h): their
+// factors are zero and what they multiply is finite for every pair of unit
+// directions.  With eta away from 0, 1 and infinity the Fresnel terms and
+// |V + eta L| stay away from 0 / 0; with a roughness of at least 0.01 the GGX
+// denominator 1 + (a^2 - 1) cos^2 stays positive however a cosine rounds; colours
+// in [0, 1e6] bound the tint; a NaN fails every comparison.
+bool material_plain(const wl_disney_material &m)
+{
+    const auto in = [](float x, float lo, float hi) { return x >= lo && x <= hi; };
+    return m.trans == 0.0f && m.clearcoat == 0.0f && m.sheen == 0.0f && m.specularTint == 0.0f &&
+           m.subsurface == 0.0f && (in(m.eta, 0.02f, 0.99f) || in(m.eta, 1.01f, 50.0f)) &&
+           in(m.roughness, 0.01f, 10.0f) && in(m.metallic, 0.0f, 1.0f) &&
+           in(m.clearcoatgloss, 0.0f, 1.0f) && in(m.sheenTint, 0.0f, 1.0f) &&
+           in(m.specular, 0.0f, 1e3f) && in(m.color[0], 0.0f, 1e6f) &&
+           in(m.color[1], 0.0f, 1e6f) && in(m.color[2], 0.0f, 1e6f);
+}
+
 size_t batch_bytes(size_t cap) { return wl::pt_batch_bytes(cap); }
 
 size_t guide_batch_bytes(size_t cap)
@@ -359,7 +377,10 @@ wl_status wl_scene_create(wl_context ctx, wl_accel accel,
     }
     std::vector<wl_disney_material> mats(std::max<uint32_t>(1, num_meshes));
     for (uint32_t m = 0; m < num_meshes; ++m)
+    {
         mats[m] = meshes[m].material;
+        mats[m].pad_ = material_plain(mats[m]) ? 1.0f : 0.0f;
+    }
 
     wl_scene s = new (std::nothrow) wl_scene_s;
     if (!s)

@@ -130,3 +130,40 @@ def test_plain_materials_keep_every_bit(gpu_ctx, strategy):
         films.append(film)
     assert torch.equal(films[0].view(torch.int32), films[1].view(torch.int32))
     assert (films[0][:, 0:3] != 0).any()
+
+
+@pytest.mark.parametrize("name", ["wave", "textured", "deep"])
+@pytest.mark.parametrize("w,h,depth", [(1, 1, 25), (64, 1, 3), (64, 1, 4), (257, 3, 25),
+                                       (300, 217, 16), (1031, 777, 16)])
+def test_finished_batches_equal_launched_bounces(gpu_ctx, name, w, h, depth):
+    """Small batches run all but their first bounces in one kernel
+    (render_samples); the traced render of the same frame launches every
+    bounce: the same radiance, bit for bit."""
+    import torch
+    import wayland_amd as wl
+    print(f"case: {name} {w} x {h} depth {depth}", flush=True)
+    if name == "wave":
+        sc = scenes.wavefront_scene(6, 3, width=w, height=h)
+    elif name == "textured":
+        sc = scenes.textured_cornell_box(w, h)
+    else:
+        sc = _deep_scene()
+    pt = wl.PathTracer(gpu_ctx, wl.Accel(gpu_ctx, sc), sc)
+    cfg = wl.pt_config(w, h, max_depth=depth, rr_depth=3)
+    for frame in (0, 5):
+        a = pt.render_samples(cfg, frame)
+        b, _ = pt.trace_samples(cfg, frame, max_vertices=2)
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+def test_finished_batches_count_their_rays(gpu_ctx):
+    """The ray statistics of a small batch equal those of the same paths in a
+    batch of two lanes (launched bounces)."""
+    import wayland_amd as wl
+    sc = scenes.wavefront_scene(4, 3, width=512, height=512)
+    pt = wl.PathTracer(gpu_ctx, wl.Accel(gpu_ctx, sc), sc)
+    _, big = pt.render(wl.pt_config(512, 512, spp=16, max_depth=8))
+    small = [pt.render(wl.pt_config(512, 512, spp=4, max_depth=8, frame_offset=4 * k))[1]
+             for k in range(4)]
+    for key in ("paths", "extension_rays", "shadow_rays"):
+        assert big[key] == sum(s[key] for s in small), key

@@ -221,8 +221,10 @@ void k_trace_first(PtParams P, PtScene S, PtBuffers B)
     const uint32_t count = P.npix * P.nsamples;
     if (blockIdx.x == 0 && threadIdx.x == 0)
         B.stats[0] += count;
+    auto range = first_chunks(count);
     trav_persistent<kClosest, kPtBlock, STACK != 16, pt_top_nodes<STACK, false>() != 0>(
-        S.nodes, S.tris, stack, first_chunks(count),
+        S.nodes, S.tris, stack,
+        XcdChunks<kPtBlock, decltype(range)>(range, queue_chunks(B, blockIdx.x % 8u), 0u),
         [&](uint32_t i, TravRay &r, uint32_t &) {
             V3 o, d;
             uint32_t seed;
@@ -230,7 +232,69 @@ void k_trace_first(PtParams P, PtScene S, PtBuffers B)
             trav_setup(r, o.x, o.y, o.z, d.x, d.y, d.z, P.epsilon, 1e30f);
         },
         [&](uint32_t i, const TravRay &, const TravResult &h) { store_hit_nt(B.hits, i, h); },
-        reinterpret_cast<const WlBvh8Node *>(top), ntop, queue_chunks(B, blockIdx.x % 8u), 0u);
+        reinterpret_cast<const WlBvh8Node *>(top), ntop);
+}
+
+// Ray i of a queue: the shadow queue or the ray queue of the given parity.
+template <bool MULTI>
+__device__ __forceinline__ void queue_fetch(const PtBuffers &B, int parity,
+                                            const PtReq *__restrict__ reqs, float eps, bool shadow,
+                                            uint32_t i, TravRay &r, uint32_t &root)
+{
+    // the ray queues carry the path's lastPdf and seed in the rays' w words
+    // (the shade pass reads its state back from the ray): every extension ray
+    // is traced on [epsilon, 1e30], epsilon the batch's or the ray's request's
+    const wl_ray *rays = parity ? B.rays1 : B.rays0;
+    const f4v *rp = reinterpret_cast<const f4v *>((shadow ? B.srays : rays) + i);
+    const f4v a = __builtin_nontemporal_load(rp), b = __builtin_nontemporal_load(rp + 1);
+    float tmin = a.w, tmax = b.w;
+    if (!shadow)
+    {
+        tmin = eps;
+        tmax = 1e30f;
+    }
+    if constexpr (MULTI) // the node and triangle arrays are the arena of the requests' BVHs
+    {
+        if (shadow)
+            root = B.sreq[i];
+        else
+        {
+            const PtReq &rq = reqs[(parity ? B.qreq1 : B.qreq0)[i]];
+            root = rq.root;
+            tmin = rq.P.epsilon;
+        }
+    }
+    trav_setup(r, a.x, a.y, a.z, b.x, b.y, b.z, tmin, tmax);
+    r.code |= shadow ? kAnyRay : 0u;
+}
+
+// Its result: the hit of a path's ray, or the NEE contribution of an unoccluded
+// shadow ray (one per path) added to its path's radiance.
+__device__ __forceinline__ void queue_emit(const PtBuffers &B, uint32_t i, const TravRay &r,
+                                           const TravResult &h)
+{
+    if (!(r.code & kAnyRay))
+    {
+        store_hit_nt(B.hits, i, h);
+        return;
+    }
+    if (h.prim != WL_INVALID)
+        return;
+    const uint32_t path = B.spath[i];
+    const float4 c = B.scontrib[i];
+    float4 rr = B.rad[path];
+    rr.x = rr.x + c.x;
+    rr.y = rr.y + c.y;
+    rr.z = rr.z + c.z;
+    B.rad[path] = rr;
+    if (c.w != 0.0f) // the path records guide training radiance
+    {
+        float4 ga = B.gacc[path];
+        ga.x += c.x;
+        ga.y += c.y;
+        ga.z += c.z;
+        B.gacc[path] = ga;
+    }
 }
 
 // The two queues of a bounce are independent (a shadow ray adds to its path's
@@ -254,8 +318,6 @@ void k_trace(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs,
     __shared__ uint4 top[8 * (pt_top_nodes<STACK, MULTI>() ? pt_top_nodes<STACK, MULTI>() : 1)];
     const uint32_t ntop = pt_load_top<STACK, MULTI>(top, S);
     const uint32_t x = blockIdx.x % 8u;
-    const wl_ray *rays = parity ? B.rays1 : B.rays0;
-    const uint32_t *qreq = parity ? B.qreq1 : B.qreq0; // multi-request batches
     const unsigned long long len = *queue_len(B, x, parity);
     const uint32_t flat = first ? B.counters[kPtFlatCount] : 0u;
     const uint32_t nrays = (uint32_t)len, nshadow = (uint32_t)(len >> 32);
@@ -285,61 +347,13 @@ void k_trace(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs,
         next = lo + (uint32_t)(s0 < n ? s0 : n);
         end = lo + (uint32_t)(s0 + chunk < n ? s0 + chunk : n);
     };
-    auto fetch = [&](uint32_t i, TravRay &r, uint32_t &root) {
-        // the queues carry the path's lastPdf and seed in the rays' w words
-        // (the shade pass reads its state back from the ray): every extension
-        // ray is traced on [epsilon, 1e30], epsilon the batch's or the ray's
-        // request's
-        const f4v *rp = reinterpret_cast<const f4v *>((shadow ? B.srays : rays) + i);
-        const f4v a = __builtin_nontemporal_load(rp), b = __builtin_nontemporal_load(rp + 1);
-        float tmin = a.w, tmax = b.w;
-        if (!shadow)
-        {
-            tmin = eps;
-            tmax = 1e30f;
-        }
-        if constexpr (MULTI) // S.nodes / S.tris: the arena of the requests' BVHs
-        {
-            if (shadow)
-                root = B.sreq[i];
-            else
-            {
-                const PtReq &rq = reqs[qreq[i]];
-                root = rq.root;
-                tmin = rq.P.epsilon;
-            }
-        }
-        trav_setup(r, a.x, a.y, a.z, b.x, b.y, b.z, tmin, tmax);
-        r.code |= shadow ? kAnyRay : 0u;
-    };
-    auto emit = [&](uint32_t i, const TravRay &r, const TravResult &h) {
-        if (!(r.code & kAnyRay))
-        {
-            store_hit_nt(B.hits, i, h);
-            return;
-        }
-        if (h.prim != WL_INVALID)
-            return;
-        // unoccluded: add the NEE contribution (one shadow ray per path)
-        const uint32_t path = B.spath[i];
-        const float4 c = B.scontrib[i];
-        float4 rr = B.rad[path];
-        rr.x = rr.x + c.x;
-        rr.y = rr.y + c.y;
-        rr.z = rr.z + c.z;
-        B.rad[path] = rr;
-        if (c.w != 0.0f) // the path records guide training radiance
-        {
-            float4 ga = B.gacc[path];
-            ga.x += c.x;
-            ga.y += c.y;
-            ga.z += c.z;
-            B.gacc[path] = ga;
-        }
-    };
     trav_persistent<kMixed, kPtBlock, STACK != 16, pt_top_nodes<STACK, MULTI>() != 0>(
-        S.nodes, S.tris, stack, range, fetch, emit, reinterpret_cast<const WlBvh8Node *>(top),
-        ntop, queue_chunks(B, x), 0u);
+        S.nodes, S.tris, stack, XcdChunks<kPtBlock, decltype(range)>(range, queue_chunks(B, x), 0u),
+        [&](uint32_t i, TravRay &r, uint32_t &root) {
+            queue_fetch<MULTI>(B, parity, reqs, eps, shadow, i, r, root);
+        },
+        [&](uint32_t i, const TravRay &r, const TravResult &h) { queue_emit(B, i, r, h); },
+        reinterpret_cast<const WlBvh8Node *>(top), ntop);
 }
 
 // ---- material sort of the shade queue ------------------------------------------
@@ -619,6 +633,402 @@ void k_guide_infer_pt(PtParams P, PtScene S, PtBuffers B, int parity)
 // materials behind a branch and one sine and cosine for all lobes, two 1024^2
 // Cornell frames 2.53 -> 2.32 ms, 256 small serving requests 9.2 -> 8.8 ms.  Four
 // waves per SIMD: five (96 VGPRs, no spills) is 2-6 % slower.
+struct Vertex
+{
+    bool cont = false, shadow = false, shadow_gacc = false;
+    uint32_t path = 0, req = 0, root = 0;
+    wl_ray next_ray{}, shadow_ray{};
+    V3 contrib{};
+};
+
+// Shades entry i of the ray queue: what its path does next, in `out`.
+template <bool GSAMPLE, bool GTRAIN, bool MULTI, bool TRACE>
+__device__ __forceinline__ void shade_vertex(const PtParams &P0, const PtScene &S0,
+                                             const PtBuffers &B, int parity,
+                                             const PtReq *__restrict__ reqs, int first, uint32_t i,
+                                             Vertex &out)
+{
+    const uint32_t *qin = parity ? B.qpath1 : B.qpath0;
+    // the first queue is the identity: entry i is path i
+    const bool ident = first != 0;
+    out.path = ident ? i : qin[i];
+    if (MULTI)
+        out.req = (parity ? B.qreq1 : B.qreq0)[i];
+    const PtReq *rq = MULTI ? reqs + out.req : nullptr;
+    if (MULTI)
+        out.root = rq->root;
+    const PtParams &P = MULTI ? rq->P : P0;
+    const PtScene &S = MULTI ? rq->S : S0;
+    const float4 hit = reinterpret_cast<const float4 *>(B.hits)[i];
+    float4 s_pos, s_dir, s_thr, s_ltt;
+    if (first)
+    {
+        // the first vertex: single-scene batches recompute the camera
+        // ray; multi-request ones read it (with lastPdf 1 and the
+        // seed in its w words) from the queue the raygen pass wrote,
+        // whose item lookup the shade pass would otherwise repeat
+        if (MULTI)
+        {
+            const float4 *rp = reinterpret_cast<const float4 *>(B.rays0 + i);
+            s_pos = rp[0];
+            s_dir = rp[1];
+        }
+        else
+        {
+            V3 o, d;
+            uint32_t sd;
+            camera_ray(P, out.path, o, d, sd);
+            s_pos = f4(o, 1.0f);                // w: lastPdf
+            s_dir = f4(d, __uint_as_float(sd)); // w: seed
+        }
+        s_thr = f4(mk(1, 1, 1), __uint_as_float(0u)); // w: depth
+        s_ltt = f4(mk(1, 1, 1), 1.0f); // w: miss weight
+    }
+    else
+    {
+        // the ray this pass shades: origin and lastPdf, then the
+        // direction and the seed (written so by the last pass)
+        const float4 *rp =
+            reinterpret_cast<const float4 *>((parity ? B.rays1 : B.rays0) + i);
+        s_pos = rp[0];
+        s_dir = rp[1];
+        s_thr = B.thr[out.path];
+        s_ltt = B.ltt[out.path];
+    }
+    V3 rayPos = v3of(s_pos);
+    float lastPdf = s_pos.w;
+    V3 rayDir = v3of(s_dir);
+    uint32_t seed = __float_as_uint(s_dir.w);
+    V3 throughput = v3of(s_thr);
+    const uint32_t sw = __float_as_uint(s_thr.w);
+    uint32_t depth = sw & kDepthMask;
+    uint32_t gvis = (sw >> 16) & kGvisMask; // guided vertices passed
+    V3 lastTraceTerm = v3of(s_ltt);
+    float missw = 1.0f; // miss weight of the ray this vertex samples
+    // radiance changes only at a miss or an emitter hit: read and
+    // written back only then
+    const bool gtrain = GTRAIN && (P.gmode & 2u);
+    V3 radiance = mk(0, 0, 0), rad_in = mk(0, 0, 0);
+    bool rad_dirty = false;
+    const uint32_t prim = __float_as_uint(hit.y);
+    bool done = false;
+    // guiding: the path's training record is taken (its first guided
+    // vertex); the radiance added after it goes to gacc
+    const bool grec_done = gtrain && (sw & kGrecBit) != 0;
+    bool grec_now = false;
+    if (prim == WL_INVALID)
+    {
+        // __miss__radiance: radiance += throughput * bg.  The
+        // reference leaves the last vertex's weight f |cos| / pdf
+        // out of this term, so its expectation is throughput * bg
+        // times the probability that the last vertex's sampler
+        // sends the ray to the background.  s_ltt.w keeps that
+        // expectation when a guided vertex sampled the ray: the
+        // reference sampler's density over the mixed density
+        // there, and exactly 1 after every other vertex.
+        radiance = ident ? mk(0, 0, 0) : v3of(B.rad[out.path]);
+        rad_in = radiance;
+        radiance = radiance + throughput * ld3(P.bg) * s_ltt.w;
+        rad_dirty = true;
+        done = true;
+    }
+    else
+    {
+        depth += 1;
+        const float t = hit.x, b1 = hit.z, b2 = hit.w;
+        const float4 *sr = reinterpret_cast<const float4 *>(S.prims) + 3 * (size_t)prim;
+        const float4 w0 = sr[0], w1 = sr[1], w2 = sr[2];
+        const V3 va = mk(w0.x, w0.y, w0.z), vb = mk(w0.w, w1.x, w1.y),
+                 vc = mk(w1.z, w1.w, w2.x);
+        const uint32_t mesh = __float_as_uint(w2.y);
+        const PtMesh M = S.meshes[mesh];
+        V3 Ng = normalize(cross(vb - va, vc - va));
+        V3 Ns;
+        if (M.has_normal)
+        {
+            const float4 *nr = reinterpret_cast<const float4 *>(S.normals) + 3 * (size_t)prim;
+            const float4 n0 = nr[0], n1 = nr[1], n2 = nr[2];
+            const V3 na = mk(n0.x, n0.y, n0.z), nb = mk(n0.w, n1.x, n1.y),
+                     nc = mk(n1.z, n1.w, n2.x);
+            Ns = normalize(na * (1 - b1 - b2) + nb * b1 + nc * b2);
+        }
+        else
+            Ns = Ng;
+        const V3 hitPos = rayPos + rayDir * t;
+        if (M.light != WL_INVALID)
+        {
+            const PtLight lt = S.lights[M.light];
+            if (depth == 1 || (P.strategy != WL_STRATEGY_NEE &&
+                               (lt.two_sided || dot(Ns, rayDir) < 0)))
+            {
+                float neePdf = 0.f;
+                if (P.strategy != WL_STRATEGY_UPT && depth > 1)
+                {
+                    // PdfAreaLightPos (Pdf.h:20-31)
+                    float pdf = 1.0f / (float)P.num_lights;
+                    pdf /= (float)lt.tri_count;
+                    pdf /= tri_area(va, vb, vc);
+                    const float dist = t;
+                    neePdf = pdf * dist * dist / fabsf(dot(Ns, rayDir));
+                }
+                const float uptPdf = lastPdf;
+                radiance = ident ? mk(0, 0, 0) : v3of(B.rad[out.path]);
+                rad_in = radiance;
+                rad_dirty = true;
+                radiance = radiance + throughput * ld3(lt.L) * lastTraceTerm *
+                                          (uptPdf / (uptPdf + neePdf));
+            }
+            done = true;
+        }
+        else if (depth >= P.max_depth)
+        {
+            throughput = mk(0, 0, 0);
+            done = true;
+        }
+        else
+        {
+            const Mat mat = load_mat(S.materials + M.material);
+            // texture colour (PathTracing.cu:261-268)
+            V3 tex = mk(1, 1, 1);
+            if (M.texture != WL_INVALID)
+            {
+                const float4 *ur = reinterpret_cast<const float4 *>(S.uvs) + 2 * (size_t)prim;
+                const float4 u01 = ur[0], u2 = ur[1];
+                const float w0 = 1 - b1 - b2;
+                const float tu = (u01.x * w0 + u01.z * b1) + u2.x * b2;
+                const float tv = (u01.y * w0 + u01.w * b1) + u2.y * b2;
+                const PtTexture T = S.textures[M.texture];
+                tex = tex_bilinear(S.texels + T.offset, T.width, T.height, tu, tv);
+            }
+            if (mat.trans < 0.1f)
+            {
+                if (dot(Ng, rayDir) > 0)
+                    Ng = -Ng;
+                if (dot(Ns, rayDir) > 0)
+                    Ns = -Ns;
+            }
+            const bool guided = GSAMPLE && mat.trans == 0.0f &&
+                                mat.clearcoat == 0.0f && (P.gmode & 1u) &&
+                                (P.gverts == 0 || gvis < P.gverts);
+            if (GSAMPLE && guided)
+                gvis += 1;
+            GuideMix gm;
+            bool took_guide = false;
+            V3 nd;
+            if (GSAMPLE && guided)
+            {
+                const float *gsrc = B.gout + kGuideDecoded * (size_t)i;
+                guide_load(gsrc, gm);
+                if (rnd(seed) < P.galpha)
+                {
+                    const float u0 = rnd(seed);
+                    const float u1 = rnd(seed);
+                    const float u2 = rnd(seed);
+                    nd = guide_sample(gm, gsrc + 40, u0, u1, u2);
+                    took_guide = true;
+                }
+            }
+            if (!took_guide)
+            {
+                nd = sample_disney(mat, Ns, -rayDir, seed);
+                nd = normalize(nd);
+            }
+            float pdf = pdf_disney(mat, Ns, -rayDir, nd);
+            if (GSAMPLE && guided && !(pdf < 0.0f || __builtin_isnan(pdf)))
+            {
+                // the reference sampler's own density: its pdf less
+                // the diffuse term below the surface, where the
+                // sampler draws nothing (trans = 0, clearcoat = 0)
+                const float cl = dot(nd, Ns);
+                const float pb = pdf;
+                float sdens = pdf;
+                if (cl < 0.0f)
+                    sdens -= 0.5f * (1.0f - mat.metallic) * (-cl * (1.0f / kPi));
+                pdf = P.galpha * guide_pdf(gm, nd) + (1.0f - P.galpha) * pdf;
+                if (!(pdf > 0.0f))
+                    pdf = -1.0f; // a zero mixed density ends the path
+                else if (__builtin_isinf(pb))
+                    // the reference pdf is infinite where its GGX
+                    // reflection folds back onto -V (1 / |L.H|, and
+                    // its sampler does land there): the limit of
+                    // s / p_mix as p_bsdf grows, not inf / inf
+                    missw = 1.0f / (1.0f - P.galpha);
+                else
+                    missw = fmaxf(sdens, 0.0f) / pdf; // 0 if only q is infinite
+            }
+            if (pdf < 0.0f || __builtin_isnan(pdf))
+            {
+                done = true;
+            }
+            else
+            {
+                throughput = throughput * lastTraceTerm;
+                const float cosWeight = dot(nd, Ns);
+                V3 bsdf = eval_disney(mat, Ns, Ng, -rayDir, nd, tex);
+                bsdf = clamp3(bsdf, 0.f, 1e30f);
+                lastTraceTerm = bsdf * fabsf(cosWeight) / pdf;
+                if (TRACE && depth - 1 < B.trace_max)
+                {
+                    float4 *tr = reinterpret_cast<float4 *>(
+                        B.trace + 8 * ((size_t)out.path * B.trace_max + depth - 1));
+                    tr[0] = make_float4((float)depth, (float)mesh, pdf,
+                                        (lastTraceTerm.x + lastTraceTerm.y +
+                                         lastTraceTerm.z) / 3.0f);
+                    tr[1] = make_float4((throughput.x + throughput.y + throughput.z) /
+                                            3.0f,
+                                        0.0f, 0.0f, mat.trans);
+                }
+                const V3 lastRayDir = rayDir;
+                if (GSAMPLE && guided && gtrain && !grec_done)
+                {
+                    // training record: query, sampled direction and
+                    // the throughput reaching this vertex
+                    float q[9];
+                    guide_query(P, hitPos, Ng, rayDir, q);
+                    float4 *r = reinterpret_cast<float4 *>(B.grec + 16 * (size_t)out.path);
+                    r[0] = make_float4(q[0], q[1], q[2], q[3]);
+                    r[1] = make_float4(q[4], q[5], q[6], q[7]);
+                    r[2] = make_float4(q[8], nd.x, nd.y, nd.z);
+                    r[3] = make_float4(0.0f, (throughput.x + throughput.y + throughput.z) *
+                                                 (1.0f / 3.0f),
+                                       0.0f, 0.0f);
+                    grec_now = true;
+                }
+                rayPos = hitPos;
+                rayDir = nd;
+                lastPdf = pdf;
+                // ---- NEE at this vertex (PathTracing.cu:81-128)
+                if (P.strategy != WL_STRATEGY_UPT && P.num_lights > 0)
+                {
+                    uint32_t lid = (uint32_t)((float)P.num_lights * rnd(seed));
+                    lid = lid < P.num_lights ? lid : P.num_lights - 1;
+                    const PtLight lt = S.lights[lid];
+                    float lpdf = 1.0f / (float)P.num_lights;
+                    uint32_t triIdx = (uint32_t)(rnd(seed) * (float)lt.tri_count);
+                    triIdx = triIdx < lt.tri_count ? triIdx : lt.tri_count - 1;
+                    lpdf = lpdf / (float)lt.tri_count;
+                    const uint32_t lprim = lt.tri_offset + triIdx;
+                    const float4 *lr = reinterpret_cast<const float4 *>(S.prims) + 3 * (size_t)lprim;
+                    const float4 l0 = lr[0], l1 = lr[1], l2 = lr[2];
+                    const V3 p0 = mk(l0.x, l0.y, l0.z), p1 = mk(l0.w, l1.x, l1.y),
+                             p2 = mk(l1.z, l1.w, l2.x);
+                    float u = rnd(seed), v = rnd(seed);
+                    if (u + v > 1)
+                    {
+                        u = 1 - u;
+                        v = 1 - v;
+                    }
+                    const float cx = 1 - u - v, cy = u;
+                    const V3 lpos = p0 + u * (p1 - p0) + v * (p2 - p0);
+                    lpdf = lpdf / tri_area(p0, p1, p2);
+                    V3 lN;
+                    if (lt.has_normal)
+                    {
+                        const float4 *nr = reinterpret_cast<const float4 *>(S.normals) + 3 * (size_t)lprim;
+                        const float4 n0 = nr[0], n1 = nr[1], n2 = nr[2];
+                        const V3 na = mk(n0.x, n0.y, n0.z), nb = mk(n0.w, n1.x, n1.y),
+                                 nc = mk(n1.z, n1.w, n2.x);
+                        // weights (1 - cx - cy, cx, cy), as Sample.h:121 applies them
+                        lN = normalize(na * (1 - cx - cy) + nb * cx + nc * cy);
+                    }
+                    else
+                        lN = normalize(cross(p1 - p0, p2 - p0));
+                    V3 visRay = lpos - rayPos;
+                    const float dist = length(visRay);
+                    visRay = visRay / dist;
+                    const float cosTheta1 = dot(lN, visRay);
+                    if (lt.two_sided || cosTheta1 < 0)
+                    {
+                        const float cosTheta2 = dot(Ns, visRay);
+                        const float neePdf = lpdf * dist * dist / fabsf(cosTheta1);
+                        float uptPdf = 0.f;
+                        if (P.strategy != WL_STRATEGY_NEE)
+                        {
+                            uptPdf = pdf_disney(mat, Ns, -lastRayDir, visRay);
+                            if (uptPdf < 0 || __builtin_isnan(uptPdf))
+                                uptPdf = 0.f;
+                            if (GSAMPLE && guided)
+                                uptPdf = P.galpha * guide_pdf(gm, visRay) +
+                                         (1.0f - P.galpha) * uptPdf;
+                        }
+                        V3 bv = eval_disney(mat, Ns, Ng, -lastRayDir, visRay, tex);
+                        bv = clamp3(bv, 0.f, 1e30f);
+                        out.contrib = throughput * bv * fabsf(cosTheta2) * ld3(lt.L) / neePdf *
+                                  (1 - uptPdf / (uptPdf + neePdf));
+                        out.shadow = true;
+                        out.shadow_ray = wl_ray{ rayPos.x, rayPos.y, rayPos.z, P.epsilon,
+                                             visRay.x, visRay.y, visRay.z,
+                                             dist * (1 - P.epsilon) };
+                    }
+                }
+                // ---- Russian roulette (PathTracing.cu:130-138)
+                if (depth > P.rr_depth)
+                {
+                    if (rnd(seed) > P.rr_prob)
+                    {
+                        throughput = mk(0, 0, 0);
+                        done = true;
+                    }
+                    else
+                        throughput = throughput / P.rr_prob;
+                }
+            }
+        }
+    }
+    if (rad_dirty || ident) // the first pass starts every path's radiance
+        B.rad[out.path] = f4(radiance, 0.0f);
+    if (gtrain)
+    {
+        // radiance reaching the path after its first guided vertex
+        if (grec_done && rad_dirty)
+        {
+            float4 gacc = B.gacc[out.path];
+            gacc.x += radiance.x - rad_in.x;
+            gacc.y += radiance.y - rad_in.y;
+            gacc.z += radiance.z - rad_in.z;
+            B.gacc[out.path] = gacc;
+        }
+        if (grec_now) // nothing gathered yet; w marks the record
+            B.gacc[out.path] = make_float4(0.f, 0.f, 0.f, 1.0f);
+        else if (ident) // no record yet
+            B.gacc[out.path] = make_float4(0.f, 0.f, 0.f, 0.f);
+        out.shadow_gacc = grec_done;
+    }
+    if (!done)
+    {
+        out.cont = true;
+        B.thr[out.path] = f4(throughput,
+                         __uint_as_float(depth | (gvis << 16) |
+                                         (grec_done || grec_now ? kGrecBit : 0u)));
+        B.ltt[out.path] = f4(lastTraceTerm, missw);
+        // the path's lastPdf and seed ride in the ray's w words
+        out.next_ray = wl_ray{ rayPos.x, rayPos.y, rayPos.z, lastPdf,
+                           rayDir.x, rayDir.y, rayDir.z, __uint_as_float(seed) };
+    }
+}
+
+// Writes a shaded vertex's ray to the other ray queue and its shadow ray.
+template <bool MULTI>
+__device__ __forceinline__ void store_vertex(const PtBuffers &B, int parity, const Vertex &v,
+                                             uint32_t slot, uint32_t sslot)
+{
+    if (v.cont)
+    {
+        (parity ? B.qpath0 : B.qpath1)[slot] = v.path;
+        (parity ? B.rays0 : B.rays1)[slot] = v.next_ray;
+        if (MULTI)
+            (parity ? B.qreq0 : B.qreq1)[slot] = v.req;
+    }
+    if (v.shadow)
+    {
+        B.spath[sslot] = v.path;
+        if (MULTI)
+            B.sreq[sslot] = v.root;
+        B.srays[sslot] = v.shadow_ray;
+        B.scontrib[sslot] = f4(v.contrib, v.shadow_gacc ? 1.0f : 0.0f);
+    }
+}
+
 template <bool GSAMPLE, bool GTRAIN, bool MULTI, bool TRACE = false>
 __global__ __launch_bounds__(kPtBlock)
 __attribute__((amdgpu_waves_per_eu(GSAMPLE || GTRAIN ? 3 : 4)))
@@ -641,9 +1051,6 @@ void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__re
     if (blockIdx.x < 8u && threadIdx.x == 0)
         *queue_chunks(B, blockIdx.x) = 0u; // the next trace counts from zero
     const uint32_t seg = (blockIdx.x % 8u) * B.segcap;
-    const uint32_t *qin = parity ? B.qpath1 : B.qpath0;
-    uint32_t *qout = parity ? B.qpath0 : B.qpath1;
-    wl_ray *rout = parity ? B.rays0 : B.rays1;
     __shared__ BlockAppendLds app;
     uint32_t pass = 0;
     // every thread of the workgroup runs the same passes (k is per
@@ -654,390 +1061,117 @@ void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__re
         const bool in_range = j < q.limit;
         // material-sorted order: the j-th entry of the sorted queue
         const uint32_t i = (!MULTI && P0.sort_bins && in_range) ? B.sort_perm[j] : j;
-        bool cont = false, shadow = false, shadow_gacc = false;
-        uint32_t path = 0, req = 0, root = 0;
-        wl_ray next_ray{}, shadow_ray{};
-        V3 contrib = mk(0, 0, 0);
+        Vertex v;
         if (in_range)
-        {
-            // the first queue is the identity: entry i is path i
-            const bool ident = first != 0;
-            path = ident ? i : qin[i];
-            if (MULTI)
-                req = (parity ? B.qreq1 : B.qreq0)[i];
-            const PtReq *rq = MULTI ? reqs + req : nullptr;
-            if (MULTI)
-                root = rq->root;
-            const PtParams &P = MULTI ? rq->P : P0;
-            const PtScene &S = MULTI ? rq->S : S0;
-            const float4 hit = reinterpret_cast<const float4 *>(B.hits)[i];
-            float4 s_pos, s_dir, s_thr, s_ltt;
-            if (first)
-            {
-                // the first vertex: single-scene batches recompute the camera
-                // ray; multi-request ones read it (with lastPdf 1 and the
-                // seed in its w words) from the queue the raygen pass wrote,
-                // whose item lookup the shade pass would otherwise repeat
-                if (MULTI)
-                {
-                    const float4 *rp = reinterpret_cast<const float4 *>(B.rays0 + i);
-                    s_pos = rp[0];
-                    s_dir = rp[1];
-                }
-                else
-                {
-                    V3 o, d;
-                    uint32_t sd;
-                    camera_ray(P, path, o, d, sd);
-                    s_pos = f4(o, 1.0f);                // w: lastPdf
-                    s_dir = f4(d, __uint_as_float(sd)); // w: seed
-                }
-                s_thr = f4(mk(1, 1, 1), __uint_as_float(0u)); // w: depth
-                s_ltt = f4(mk(1, 1, 1), 1.0f); // w: miss weight
-            }
-            else
-            {
-                // the ray this pass shades: origin and lastPdf, then the
-                // direction and the seed (written so by the last pass)
-                const float4 *rp =
-                    reinterpret_cast<const float4 *>((parity ? B.rays1 : B.rays0) + i);
-                s_pos = rp[0];
-                s_dir = rp[1];
-                s_thr = B.thr[path];
-                s_ltt = B.ltt[path];
-            }
-            V3 rayPos = v3of(s_pos);
-            float lastPdf = s_pos.w;
-            V3 rayDir = v3of(s_dir);
-            uint32_t seed = __float_as_uint(s_dir.w);
-            V3 throughput = v3of(s_thr);
-            const uint32_t sw = __float_as_uint(s_thr.w);
-            uint32_t depth = sw & kDepthMask;
-            uint32_t gvis = (sw >> 16) & kGvisMask; // guided vertices passed
-            V3 lastTraceTerm = v3of(s_ltt);
-            float missw = 1.0f; // miss weight of the ray this vertex samples
-            // radiance changes only at a miss or an emitter hit: read and
-            // written back only then
-            const bool gtrain = GTRAIN && (P.gmode & 2u);
-            V3 radiance = mk(0, 0, 0), rad_in = mk(0, 0, 0);
-            bool rad_dirty = false;
-            const uint32_t prim = __float_as_uint(hit.y);
-            bool done = false;
-            // guiding: the path's training record is taken (its first guided
-            // vertex); the radiance added after it goes to gacc
-            const bool grec_done = gtrain && (sw & kGrecBit) != 0;
-            bool grec_now = false;
-            if (prim == WL_INVALID)
-            {
-                // __miss__radiance: radiance += throughput * bg.  The
-                // reference leaves the last vertex's weight f |cos| / pdf
-                // out of this term, so its expectation is throughput * bg
-                // times the probability that the last vertex's sampler
-                // sends the ray to the background.  s_ltt.w keeps that
-                // expectation when a guided vertex sampled the ray: the
-                // reference sampler's density over the mixed density
-                // there, and exactly 1 after every other vertex.
-                radiance = ident ? mk(0, 0, 0) : v3of(B.rad[path]);
-                rad_in = radiance;
-                radiance = radiance + throughput * ld3(P.bg) * s_ltt.w;
-                rad_dirty = true;
-                done = true;
-            }
-            else
-            {
-                depth += 1;
-                const float t = hit.x, b1 = hit.z, b2 = hit.w;
-                const float4 *sr = reinterpret_cast<const float4 *>(S.prims) + 3 * (size_t)prim;
-                const float4 w0 = sr[0], w1 = sr[1], w2 = sr[2];
-                const V3 va = mk(w0.x, w0.y, w0.z), vb = mk(w0.w, w1.x, w1.y),
-                         vc = mk(w1.z, w1.w, w2.x);
-                const uint32_t mesh = __float_as_uint(w2.y);
-                const PtMesh M = S.meshes[mesh];
-                V3 Ng = normalize(cross(vb - va, vc - va));
-                V3 Ns;
-                if (M.has_normal)
-                {
-                    const float4 *nr = reinterpret_cast<const float4 *>(S.normals) + 3 * (size_t)prim;
-                    const float4 n0 = nr[0], n1 = nr[1], n2 = nr[2];
-                    const V3 na = mk(n0.x, n0.y, n0.z), nb = mk(n0.w, n1.x, n1.y),
-                             nc = mk(n1.z, n1.w, n2.x);
-                    Ns = normalize(na * (1 - b1 - b2) + nb * b1 + nc * b2);
-                }
-                else
-                    Ns = Ng;
-                const V3 hitPos = rayPos + rayDir * t;
-                if (M.light != WL_INVALID)
-                {
-                    const PtLight lt = S.lights[M.light];
-                    if (depth == 1 || (P.strategy != WL_STRATEGY_NEE &&
-                                       (lt.two_sided || dot(Ns, rayDir) < 0)))
-                    {
-                        float neePdf = 0.f;
-                        if (P.strategy != WL_STRATEGY_UPT && depth > 1)
-                        {
-                            // PdfAreaLightPos (Pdf.h:20-31)
-                            float pdf = 1.0f / (float)P.num_lights;
-                            pdf /= (float)lt.tri_count;
-                            pdf /= tri_area(va, vb, vc);
-                            const float dist = t;
-                            neePdf = pdf * dist * dist / fabsf(dot(Ns, rayDir));
-                        }
-                        const float uptPdf = lastPdf;
-                        radiance = ident ? mk(0, 0, 0) : v3of(B.rad[path]);
-                        rad_in = radiance;
-                        rad_dirty = true;
-                        radiance = radiance + throughput * ld3(lt.L) * lastTraceTerm *
-                                                  (uptPdf / (uptPdf + neePdf));
-                    }
-                    done = true;
-                }
-                else if (depth >= P.max_depth)
-                {
-                    throughput = mk(0, 0, 0);
-                    done = true;
-                }
-                else
-                {
-                    const Mat mat = load_mat(S.materials + M.material);
-                    // texture colour (PathTracing.cu:261-268)
-                    V3 tex = mk(1, 1, 1);
-                    if (M.texture != WL_INVALID)
-                    {
-                        const float4 *ur = reinterpret_cast<const float4 *>(S.uvs) + 2 * (size_t)prim;
-                        const float4 u01 = ur[0], u2 = ur[1];
-                        const float w0 = 1 - b1 - b2;
-                        const float tu = (u01.x * w0 + u01.z * b1) + u2.x * b2;
-                        const float tv = (u01.y * w0 + u01.w * b1) + u2.y * b2;
-                        const PtTexture T = S.textures[M.texture];
-                        tex = tex_bilinear(S.texels + T.offset, T.width, T.height, tu, tv);
-                    }
-                    if (mat.trans < 0.1f)
-                    {
-                        if (dot(Ng, rayDir) > 0)
-                            Ng = -Ng;
-                        if (dot(Ns, rayDir) > 0)
-                            Ns = -Ns;
-                    }
-                    const bool guided = GSAMPLE && mat.trans == 0.0f &&
-                                        mat.clearcoat == 0.0f && (P.gmode & 1u) &&
-                                        (P.gverts == 0 || gvis < P.gverts);
-                    if (GSAMPLE && guided)
-                        gvis += 1;
-                    GuideMix gm;
-                    bool took_guide = false;
-                    V3 nd;
-                    if (GSAMPLE && guided)
-                    {
-                        const float *gsrc = B.gout + kGuideDecoded * (size_t)i;
-                        guide_load(gsrc, gm);
-                        if (rnd(seed) < P.galpha)
-                        {
-                            const float u0 = rnd(seed);
-                            const float u1 = rnd(seed);
-                            const float u2 = rnd(seed);
-                            nd = guide_sample(gm, gsrc + 40, u0, u1, u2);
-                            took_guide = true;
-                        }
-                    }
-                    if (!took_guide)
-                    {
-                        nd = sample_disney(mat, Ns, -rayDir, seed);
-                        nd = normalize(nd);
-                    }
-                    float pdf = pdf_disney(mat, Ns, -rayDir, nd);
-                    if (GSAMPLE && guided && !(pdf < 0.0f || __builtin_isnan(pdf)))
-                    {
-                        // the reference sampler's own density: its pdf less
-                        // the diffuse term below the surface, where the
-                        // sampler draws nothing (trans = 0, clearcoat = 0)
-                        const float cl = dot(nd, Ns);
-                        const float pb = pdf;
-                        float sdens = pdf;
-                        if (cl < 0.0f)
-                            sdens -= 0.5f * (1.0f - mat.metallic) * (-cl * (1.0f / kPi));
-                        pdf = P.galpha * guide_pdf(gm, nd) + (1.0f - P.galpha) * pdf;
-                        if (!(pdf > 0.0f))
-                            pdf = -1.0f; // a zero mixed density ends the path
-                        else if (__builtin_isinf(pb))
-                            // the reference pdf is infinite where its GGX
-                            // reflection folds back onto -V (1 / |L.H|, and
-                            // its sampler does land there): the limit of
-                            // s / p_mix as p_bsdf grows, not inf / inf
-                            missw = 1.0f / (1.0f - P.galpha);
-                        else
-                            missw = fmaxf(sdens, 0.0f) / pdf; // 0 if only q is infinite
-                    }
-                    if (pdf < 0.0f || __builtin_isnan(pdf))
-                    {
-                        done = true;
-                    }
-                    else
-                    {
-                        throughput = throughput * lastTraceTerm;
-                        const float cosWeight = dot(nd, Ns);
-                        V3 bsdf = eval_disney(mat, Ns, Ng, -rayDir, nd, tex);
-                        bsdf = clamp3(bsdf, 0.f, 1e30f);
-                        lastTraceTerm = bsdf * fabsf(cosWeight) / pdf;
-                        if (TRACE && depth - 1 < B.trace_max)
-                        {
-                            float4 *tr = reinterpret_cast<float4 *>(
-                                B.trace + 8 * ((size_t)path * B.trace_max + depth - 1));
-                            tr[0] = make_float4((float)depth, (float)mesh, pdf,
-                                                (lastTraceTerm.x + lastTraceTerm.y +
-                                                 lastTraceTerm.z) / 3.0f);
-                            tr[1] = make_float4((throughput.x + throughput.y + throughput.z) /
-                                                    3.0f,
-                                                0.0f, 0.0f, mat.trans);
-                        }
-                        const V3 lastRayDir = rayDir;
-                        if (GSAMPLE && guided && gtrain && !grec_done)
-                        {
-                            // training record: query, sampled direction and
-                            // the throughput reaching this vertex
-                            float q[9];
-                            guide_query(P, hitPos, Ng, rayDir, q);
-                            float4 *r = reinterpret_cast<float4 *>(B.grec + 16 * (size_t)path);
-                            r[0] = make_float4(q[0], q[1], q[2], q[3]);
-                            r[1] = make_float4(q[4], q[5], q[6], q[7]);
-                            r[2] = make_float4(q[8], nd.x, nd.y, nd.z);
-                            r[3] = make_float4(0.0f, (throughput.x + throughput.y + throughput.z) *
-                                                         (1.0f / 3.0f),
-                                               0.0f, 0.0f);
-                            grec_now = true;
-                        }
-                        rayPos = hitPos;
-                        rayDir = nd;
-                        lastPdf = pdf;
-                        // ---- NEE at this vertex (PathTracing.cu:81-128)
-                        if (P.strategy != WL_STRATEGY_UPT && P.num_lights > 0)
-                        {
-                            uint32_t lid = (uint32_t)((float)P.num_lights * rnd(seed));
-                            lid = lid < P.num_lights ? lid : P.num_lights - 1;
-                            const PtLight lt = S.lights[lid];
-                            float lpdf = 1.0f / (float)P.num_lights;
-                            uint32_t triIdx = (uint32_t)(rnd(seed) * (float)lt.tri_count);
-                            triIdx = triIdx < lt.tri_count ? triIdx : lt.tri_count - 1;
-                            lpdf = lpdf / (float)lt.tri_count;
-                            const uint32_t lprim = lt.tri_offset + triIdx;
-                            const float4 *lr = reinterpret_cast<const float4 *>(S.prims) + 3 * (size_t)lprim;
-                            const float4 l0 = lr[0], l1 = lr[1], l2 = lr[2];
-                            const V3 p0 = mk(l0.x, l0.y, l0.z), p1 = mk(l0.w, l1.x, l1.y),
-                                     p2 = mk(l1.z, l1.w, l2.x);
-                            float u = rnd(seed), v = rnd(seed);
-                            if (u + v > 1)
-                            {
-                                u = 1 - u;
-                                v = 1 - v;
-                            }
-                            const float cx = 1 - u - v, cy = u;
-                            const V3 lpos = p0 + u * (p1 - p0) + v * (p2 - p0);
-                            lpdf = lpdf / tri_area(p0, p1, p2);
-                            V3 lN;
-                            if (lt.has_normal)
-                            {
-                                const float4 *nr = reinterpret_cast<const float4 *>(S.normals) + 3 * (size_t)lprim;
-                                const float4 n0 = nr[0], n1 = nr[1], n2 = nr[2];
-                                const V3 na = mk(n0.x, n0.y, n0.z), nb = mk(n0.w, n1.x, n1.y),
-                                         nc = mk(n1.z, n1.w, n2.x);
-                                // weights (1 - cx - cy, cx, cy), as Sample.h:121 applies them
-                                lN = normalize(na * (1 - cx - cy) + nb * cx + nc * cy);
-                            }
-                            else
-                                lN = normalize(cross(p1 - p0, p2 - p0));
-                            V3 visRay = lpos - rayPos;
-                            const float dist = length(visRay);
-                            visRay = visRay / dist;
-                            const float cosTheta1 = dot(lN, visRay);
-                            if (lt.two_sided || cosTheta1 < 0)
-                            {
-                                const float cosTheta2 = dot(Ns, visRay);
-                                const float neePdf = lpdf * dist * dist / fabsf(cosTheta1);
-                                float uptPdf = 0.f;
-                                if (P.strategy != WL_STRATEGY_NEE)
-                                {
-                                    uptPdf = pdf_disney(mat, Ns, -lastRayDir, visRay);
-                                    if (uptPdf < 0 || __builtin_isnan(uptPdf))
-                                        uptPdf = 0.f;
-                                    if (GSAMPLE && guided)
-                                        uptPdf = P.galpha * guide_pdf(gm, visRay) +
-                                                 (1.0f - P.galpha) * uptPdf;
-                                }
-                                V3 bv = eval_disney(mat, Ns, Ng, -lastRayDir, visRay, tex);
-                                bv = clamp3(bv, 0.f, 1e30f);
-                                contrib = throughput * bv * fabsf(cosTheta2) * ld3(lt.L) / neePdf *
-                                          (1 - uptPdf / (uptPdf + neePdf));
-                                shadow = true;
-                                shadow_ray = wl_ray{ rayPos.x, rayPos.y, rayPos.z, P.epsilon,
-                                                     visRay.x, visRay.y, visRay.z,
-                                                     dist * (1 - P.epsilon) };
-                            }
-                        }
-                        // ---- Russian roulette (PathTracing.cu:130-138)
-                        if (depth > P.rr_depth)
-                        {
-                            if (rnd(seed) > P.rr_prob)
-                            {
-                                throughput = mk(0, 0, 0);
-                                done = true;
-                            }
-                            else
-                                throughput = throughput / P.rr_prob;
-                        }
-                    }
-                }
-            }
-            if (rad_dirty || ident) // the first pass starts every path's radiance
-                B.rad[path] = f4(radiance, 0.0f);
-            if (gtrain)
-            {
-                // radiance reaching the path after its first guided vertex
-                if (grec_done && rad_dirty)
-                {
-                    float4 gacc = B.gacc[path];
-                    gacc.x += radiance.x - rad_in.x;
-                    gacc.y += radiance.y - rad_in.y;
-                    gacc.z += radiance.z - rad_in.z;
-                    B.gacc[path] = gacc;
-                }
-                if (grec_now) // nothing gathered yet; w marks the record
-                    B.gacc[path] = make_float4(0.f, 0.f, 0.f, 1.0f);
-                else if (ident) // no record yet
-                    B.gacc[path] = make_float4(0.f, 0.f, 0.f, 0.f);
-                shadow_gacc = grec_done;
-            }
-            if (!done)
-            {
-                cont = true;
-                B.thr[path] = f4(throughput,
-                                 __uint_as_float(depth | (gvis << 16) |
-                                                 (grec_done || grec_now ? kGrecBit : 0u)));
-                B.ltt[path] = f4(lastTraceTerm, missw);
-                // the path's lastPdf and seed ride in the ray's w words
-                next_ray = wl_ray{ rayPos.x, rayPos.y, rayPos.z, lastPdf,
-                                   rayDir.x, rayDir.y, rayDir.z, __uint_as_float(seed) };
-            }
-        }
+            shade_vertex<GSAMPLE, GTRAIN, MULTI, TRACE>(P0, S0, B, parity, reqs, first, i, v);
         // ---- compaction (whole wave participates)
         uint32_t slot, sslot;
-        block_append2(app, pass++, queue_len(B, blockIdx.x % 8u, parity ^ 1), cont, shadow, slot,
-                      sslot);
-        slot += seg;
-        sslot += seg;
-        if (cont)
+        block_append2(app, pass++, queue_len(B, blockIdx.x % 8u, parity ^ 1), v.cont, v.shadow,
+                      slot, sslot);
+        store_vertex<MULTI>(B, parity, v, seg + slot, seg + sslot);
+    }
+}
+
+// ---- finish: the remaining bounces of every path --------------------------------
+// In a batch of up to a few million paths a launch soon takes as long as its
+// slowest ray (70-90 us from the caustic's third bounce on, for a few thousand
+// rays) and an empty one 4.5 us.  So after kLaunchedBounces bounces each
+// workgroup takes a slice of its XCD's ray
+// segment and runs that slice's bounces to the end by itself: shade (appending
+// to its own slice of the other queue), barrier, trace the slice's rays and
+// shadow rays, barrier.  A slow ray then holds up its own workgroup's slice
+// only, and the remaining bounces need no launches of their own.  The slices
+// reuse the queues' memory: an entry appends at most one to each queue, so the
+// slice [e0, e0 + n) of one queue always fits [e0, e0 + n) of the others.
+// Measured with bounces launched / finished here (after 2): 65,536 Cornell paths
+// of 25 bounces 557 / 368 us, 1M 1179 / 956, 3M 2455 / 2256; 1M paths on the
+// 2M-triangle scene 2827 / 2092, 3M 4161 / 3652; 1M caustic paths 1874 / 1320.
+// Finishing after 1, 3 or 5 bounces: within 2 % of 2 on Cornell, 1406 / 1388 /
+// 1498 on the caustic.  Larger batches keep the launched bounces (as two lanes
+// of 3M Cornell paths each 4098 / 4679): their queues stay long, and this kernel
+// holds four waves per SIMD, the shade pass's registers, where k_trace holds six.
+constexpr uint32_t kLaunchedBounces = 2;
+constexpr uint32_t kMaxSlice = 4096;
+
+template <int STACK, bool GTRAIN, bool MULTI>
+__global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(4)))
+void k_finish(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__restrict__ reqs)
+{
+    __shared__ uint32_t stack[STACK * kPtBlock];
+    __shared__ uint4 top[8 * (pt_top_nodes<STACK, MULTI>() ? pt_top_nodes<STACK, MULTI>() : 1)];
+    __shared__ BlockAppendLds app;
+    __shared__ unsigned long long s_len; // the slice's queue lengths: rays, shadow rays
+    __shared__ uint32_t s_chunk;         // its chunk counter
+    const uint32_t x = blockIdx.x % 8u, nblk = gridDim.x / 8u;
+    const uint32_t total = (uint32_t)*queue_len(B, x, parity);
+    // equal slices of whole waves, one per workgroup while they are short
+    const uint32_t share = ((total + nblk - 1u) / nblk + 63u) & ~63u;
+    const uint32_t slice = min(share, kMaxSlice);
+    if ((blockIdx.x / 8u) * slice >= total)
+        return;
+    const uint32_t ntop = pt_load_top<STACK, MULTI>(top, S0);
+    unsigned long long rays = 0, shadows = 0; // traced by this workgroup
+    uint32_t pass = 0;
+    for (uint32_t at = (blockIdx.x / 8u) * slice; at < total; at += nblk * slice)
+    {
+        const uint32_t e0 = x * B.segcap + at;
+        int par = parity;
+        uint32_t n = min(slice, total - at);
+        while (n != 0)
         {
-            qout[slot] = path;
-            rout[slot] = next_ray;
-            if (MULTI)
-                (parity ? B.qreq0 : B.qreq1)[slot] = req;
+            if (threadIdx.x == 0)
+            {
+                s_len = 0ull;
+                s_chunk = 0u;
+            }
+            __syncthreads();
+            for (uint32_t k = 0; k < n; k += kPtBlock)
+            {
+                Vertex v;
+                if (k + threadIdx.x < n)
+                    shade_vertex<false, GTRAIN, MULTI, false>(P0, S0, B, par, reqs, 0,
+                                                              e0 + k + threadIdx.x, v);
+                uint32_t slot, sslot;
+                block_append2(app, pass++, &s_len, v.cont, v.shadow, slot, sslot);
+                store_vertex<MULTI>(B, par, v, e0 + slot, e0 + sslot);
+            }
+            par ^= 1;
+            __syncthreads(); // the appended entries and lengths
+            const unsigned long long len = s_len;
+            const uint32_t nrays = __builtin_amdgcn_readfirstlane((uint32_t)len);
+            const uint32_t nshadow = __builtin_amdgcn_readfirstlane((uint32_t)(len >> 32));
+            rays += nrays;
+            shadows += nshadow;
+            const uint32_t ray_chunks = (nrays + 63u) / 64u;
+            bool shadow = false; // the kind of the wave's current chunk
+            trav_persistent<kMixed, kPtBlock, STACK != 16, pt_top_nodes<STACK, MULTI>() != 0>(
+                S0.nodes, S0.tris, stack,
+                [&](bool, uint32_t &next, uint32_t &end) {
+                    uint32_t c = 0;
+                    if (__lane_id() == 0)
+                        c = atomicAdd(&s_chunk, 1u);
+                    c = __builtin_amdgcn_readfirstlane(c);
+                    shadow = c >= ray_chunks;
+                    const uint32_t m = shadow ? nshadow : nrays;
+                    const uint32_t at0 = (shadow ? c - ray_chunks : c) * 64u;
+                    next = e0 + min(at0, m);
+                    end = e0 + min(at0 + 64u, m);
+                },
+                [&](uint32_t i, TravRay &r, uint32_t &root) {
+                    queue_fetch<MULTI>(B, par, reqs, P0.epsilon, shadow, i, r, root);
+                },
+                [&](uint32_t i, const TravRay &r, const TravResult &h) {
+                    queue_emit(B, i, r, h);
+                },
+                reinterpret_cast<const WlBvh8Node *>(top), ntop);
+            __syncthreads(); // every hit and NEE contribution of this bounce
+            n = nrays;
         }
-        if (shadow)
-        {
-            B.spath[sslot] = path;
-            if (MULTI)
-                B.sreq[sslot] = root;
-            B.srays[sslot] = shadow_ray;
-            B.scontrib[sslot] = f4(contrib, shadow_gacc ? 1.0f : 0.0f);
-        }
+    }
+    if (threadIdx.x == 0)
+    {
+        atomicAdd(&B.stats[0], rays);
+        atomicAdd(&B.stats[1], shadows);
     }
 }
 
@@ -1316,7 +1450,7 @@ static uint32_t grid8(uint32_t blocks, int num_cus, int per_cu)
 }
 
 hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B0,
-                        int num_cus, hipStream_t st)
+                        bool alone, int num_cus, hipStream_t st)
 {
     const uint32_t npaths = P.npix * P.nsamples;
     const uint32_t blocks_all = (npaths + kPtBlock - 1) / kPtBlock;
@@ -1355,7 +1489,12 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B0
     else
         hipLaunchKernelGGL((k_trace_first<WL_BVH8_STACK_DEPTH>), dim3(g_first), dim3(kPtBlock), 0,
                            st, P, S, B);
-    for (uint32_t b = 0; b < P.max_depth; ++b)
+    // the guide's inference and the per-vertex trace belong to the launched bounces
+    const bool finish = alone && npaths < kFinishMaxPaths &&
+                        P.max_depth > kLaunchedBounces + 1 && !B.trace &&
+                        (!(P.gmode & 1u) || (P.gbounces != 0 && P.gbounces <= kLaunchedBounces));
+    const uint32_t bounces = finish ? kLaunchedBounces : P.max_depth;
+    for (uint32_t b = 0; b < bounces; ++b)
     {
         const int parity = (int)(b & 1u), first = b == 0 ? 1 : 0;
         if (P.sort_bins)
@@ -1394,6 +1533,15 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B0
             hipLaunchKernelGGL((k_shade<false, false, false>), dim3(g_shade), dim3(kPtBlock), 0,
                                st, P, S, B, parity, nullptr, first);
         trace(parity ^ 1); // the next bounce's rays, this bounce's shadow rays
+    }
+    if (finish)
+    {
+        const bool gtrain = (P.gmode & 2u) != 0;
+        const auto kernel = shallow ? (gtrain ? k_finish<16, true, false> : k_finish<16, false, false>)
+                                    : (gtrain ? k_finish<WL_BVH8_STACK_DEPTH, true, false>
+                                              : k_finish<WL_BVH8_STACK_DEPTH, false, false>);
+        hipLaunchKernelGGL(kernel, dim3(grid8(4 * blocks_all, num_cus, 4)), dim3(kPtBlock), 0, st,
+                           P, S, B, (int)(kLaunchedBounces & 1u), nullptr);
     }
     return hipGetLastError();
 }
@@ -1442,13 +1590,20 @@ hipError_t pt_run_multi(const PtMultiLaunch &L, const PtBuffers &B0, int num_cus
     hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(kPtBlock), 0, st, L, B);
     hipLaunchKernelGGL(k_raygen_multi, dim3(g_gen), dim3(kPtBlock), 0, st, L, B);
     trace(0, 1);
-    for (uint32_t b = 0; b < L.max_depth; ++b)
+    const bool finish = L.finish && L.max_depth > kLaunchedBounces + 1;
+    const uint32_t bounces = finish ? kLaunchedBounces : L.max_depth;
+    for (uint32_t b = 0; b < bounces; ++b)
     {
         const int parity = (int)(b & 1u);
         hipLaunchKernelGGL((k_shade<false, false, true>), dim3(g_shade), dim3(kPtBlock), 0, st,
                            P0, S0, B, parity, L.reqs, b == 0 ? 1 : 0);
         trace(parity ^ 1, 0);
     }
+    if (finish)
+        hipLaunchKernelGGL((L.stack16 ? k_finish<16, false, true>
+                                      : k_finish<WL_BVH8_STACK_DEPTH, false, true>),
+                           dim3(grid8(4 * blocks_all, num_cus, 4)), dim3(kPtBlock), 0, st, P0, SA,
+                           B, (int)(kLaunchedBounces & 1u), L.reqs);
     hipLaunchKernelGGL(k_accumulate_multi, dim3(g_gen), dim3(kPtBlock), 0, st, L, B);
     hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, L);
     return hipGetLastError();

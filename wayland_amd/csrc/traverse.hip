@@ -80,12 +80,14 @@ void k_trace_closest_p(
     __shared__ uint4 top[8 * (top_nodes<STACK>() ? top_nodes<STACK>() : 1)];
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
+    auto range = eighth_chunks(n, base.chunk);
     trav_persistent<kClosest, kTraceBlock, STACK != 16, top_nodes<STACK>() != 0>(
-        nodes, tris, stack, eighth_chunks(n, base.chunk),
+        nodes, tris, stack,
+        XcdChunks<kTraceBlock, decltype(range)>(range, sched + kSchedStride * (blockIdx.x % 8u),
+                                                base.base[blockIdx.x % 8u]),
         [&](uint32_t i, TravRay &r, uint32_t &) { load_ray_nt(rays, i, r); },
         [&](uint32_t i, const TravRay &, const TravResult &h) { store_hit_nt(hits, i, h); },
-        reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u,
-        sched + kSchedStride * (blockIdx.x % 8u), base.base[blockIdx.x % 8u]);
+        reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u);
 }
 
 template <int STACK>
@@ -98,15 +100,17 @@ void k_trace_any_p(const WlBvh8Node *__restrict__ nodes, const WlTriRecord *__re
     __shared__ uint4 top[8 * (top_nodes<STACK>() ? top_nodes<STACK>() : 1)];
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
+    auto range = eighth_chunks(n, base.chunk);
     trav_persistent<kAny, kTraceBlock, STACK != 16, top_nodes<STACK>() != 0>(
-        nodes, tris, stack, eighth_chunks(n, base.chunk),
+        nodes, tris, stack,
+        XcdChunks<kTraceBlock, decltype(range)>(range, sched + kSchedStride * (blockIdx.x % 8u),
+                                                base.base[blockIdx.x % 8u]),
         [&](uint32_t i, TravRay &r, uint32_t &) { load_ray_nt(rays, i, r); },
         [&](uint32_t i, const TravRay &, const TravResult &h) {
             if (h.prim != WL_INVALID)
                 atomicOr(&bits[i >> 5], 1u << (i & 31u));
         },
-        reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u,
-        sched + kSchedStride * (blockIdx.x % 8u), base.base[blockIdx.x % 8u]);
+        reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u);
 }
 
 // Instrumented closest hit: one ray per lane, per-ray node/triangle counts.

@@ -21,12 +21,9 @@
 // (closest hit) and 679 -> 603 us (any hit), the 1080p wavefront render
 // 46.2 -> 40.9 ms, the 256 small serving requests 13.2 -> 11.5 ms.
 //
-// The rays of a launch come in chunks, a list of them per XCD: the hardware
-// deals workgroups round-robin to the 8 XCDs, each with its own L2, so XCD x's
-// workgroups are those with blockIdx % 8 == x.  An XCD's W waves start on its
-// chunks 0 .. W-1 and then each takes chunk W + k, k counted by one global
-// counter per XCD.  A wave leaves the loop when it got a chunk past its XCD's
-// last and none of its lanes holds a ray, so the grid always drains.
+// The rays come in chunks that a wave takes one after the other (XcdChunks for
+// a launch over the whole GPU).  It leaves the loop when it got an empty chunk
+// and none of its lanes holds a ray.
 #pragma once
 #include "../../include/wayland_hip.h"
 #include "traverse_device.h"
@@ -76,41 +73,57 @@ __device__ __forceinline__ uint32_t lane_prefix(uint64_t m)
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
+// Chunks of a launch over the whole GPU, a list of them per XCD: the hardware
+// deals workgroups round-robin to the 8 XCDs, each with its own L2, so XCD x's
+// workgroups are those with blockIdx % 8 == x (the grid is a multiple of 8).
+// An XCD's W waves start on its chunks 0 .. W-1 and then each takes chunk W + k,
+// k counted by `dyn`, the XCD's counter (dyn_base: its value at launch).
 // range(c, next, end): the ray indices [next, end) of the XCD's chunk c, empty
-// past its last chunk; c and the results are wave-uniform.  fetch(i, TravRay&,
-// root) sets up ray i (root: the index of its first node, 0 unless several
-// BVHs share the node array); emit(i, const TravRay&, const TravResult&)
-// consumes its result.  RAYS: kClosest, kAny, or kMixed, where fetch marks
-// any-hit rays with kAnyRay in TravRay::code.  BLOCK must be a multiple of 64
-// and the grid a multiple of 8.
+// past its last.  Every wave that had a chunk makes exactly one fetch past the
+// XCD's last, so a launch advances the counter by the XCD's number of chunks.
+// A wave that got a chunk asks for its next at once (lane 0 holds the answer,
+// `ahead`), so the atomic's latency passes behind the chunk's own rays.
+template <int BLOCK, class Range>
+struct XcdChunks
+{
+    Range &range;
+    uint32_t *dyn;
+    uint32_t next_chunk, wavesx, dyn_base, ahead;
+    __device__ __forceinline__ XcdChunks(Range &r, uint32_t *d, uint32_t base)
+        : range(r), dyn(d),
+          next_chunk((blockIdx.x / 8u) * (BLOCK / 64) +
+                     __builtin_amdgcn_readfirstlane(threadIdx.x / 64)),
+          wavesx((gridDim.x / 8u) * (BLOCK / 64)), dyn_base(base), ahead(0)
+    {
+    }
+    __device__ __forceinline__ void operator()(bool first, uint32_t &next, uint32_t &end)
+    {
+        range(first ? next_chunk : wavesx + __builtin_amdgcn_readfirstlane(ahead) - dyn_base, next,
+              end);
+        if (next < end && __lane_id() == 0)
+            ahead = atomicAdd(dyn, 1u);
+    }
+};
+
+// chunks(first, next, end): the wave's next chunk [next, end) of ray indices,
+// wave-uniform, empty when there is none left.  fetch(i, TravRay&, root) sets
+// up ray i of the current chunk (root: the index of its first node, 0 unless
+// several BVHs share the node array); emit(i, const TravRay&, const
+// TravResult&) consumes its result.  RAYS: kClosest, kAny, or kMixed, where
+// fetch marks any-hit rays with kAnyRay in TravRay::code.  BLOCK must be a
+// multiple of 64.
 // top / ntop (with TOP): nodes [0, ntop) copied to LDS by the caller (see
 // node_visit).
-// dyn: this XCD's chunk counter, dyn_base its value at launch.  Every wave
-// that had a chunk makes exactly one fetch past the XCD's last, so a launch
-// advances the counter by the XCD's number of chunks.
-template <int RAYS, int BLOCK, bool WIDE, bool TOP, class Range, class Fetch, class Emit>
+template <int RAYS, int BLOCK, bool WIDE, bool TOP, class Chunks, class Fetch, class Emit>
 __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ nodes,
                                                 const WlTriRecord *__restrict__ tris,
-                                                uint32_t *stack, Range range, Fetch fetch,
-                                                Emit emit, const WlBvh8Node *top, uint32_t ntop,
-                                                uint32_t *dyn, uint32_t dyn_base)
+                                                uint32_t *stack, Chunks chunks, Fetch fetch,
+                                                Emit emit, const WlBvh8Node *top, uint32_t ntop)
 {
     static_assert(BLOCK % 64 == 0, "whole waves only");
     constexpr uint32_t kNone = 0xFFFFFFFFu;
-    // this wave among its XCD's
-    const uint32_t wx = (blockIdx.x / 8u) * (BLOCK / 64) +
-                        __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const uint32_t wavesx = (gridDim.x / 8u) * (BLOCK / 64);
-    // chunk c into [next, end); a wave that got one asks for its next at once
-    // (lane 0 holds the answer, `ahead`), so the atomic's latency passes behind
-    // the chunk's own rays
-    uint32_t next, end, ahead = 0;
-    auto take_chunk = [&](uint32_t c) {
-        range(c, next, end);
-        if (next < end && __lane_id() == 0)
-            ahead = atomicAdd(dyn, 1u);
-    };
-    take_chunk(wx);
+    uint32_t next, end;
+    chunks(true, next, end);
     TravRay r;
     trav_setup(r, 0, 0, 0, 1, 0, 0, 0, 0);
     TravState st;
@@ -144,7 +157,7 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
             }
             next = next + nidle < end ? next + nidle : end;
             if (next >= end)
-                take_chunk(wavesx + __builtin_amdgcn_readfirstlane(ahead) - dyn_base);
+                chunks(false, next, end);
         }
         // a lane with a pending triangle takes the triangle step next, any
         // other unfinished lane the node step

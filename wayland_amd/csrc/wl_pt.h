@@ -133,8 +133,12 @@ struct PtBuffers
     uint32_t trace_max;
 };
 
-hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B,
+// One batch.  alone: no other batch runs beside it (a lane of two keeps the
+// launched bounces, see k_finish).
+hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B, bool alone,
                         int num_cus, hipStream_t st);
+// Batches of fewer paths than this finish in one kernel (k_finish).
+constexpr uint32_t kFinishMaxPaths = 1u << 22;
 
 // ---- batched serving: one megabatch mixes paths of many requests ----------
 // A request's scene, parameters and film; the ray queues of a multi-request
@@ -185,6 +189,7 @@ struct PtMultiLaunch
     uint32_t max_depth;  // bounces enqueued (maximum over the requests)
     uint32_t stack16;    // every BVH at most 16 levels deep, the arena within 32-bit offsets
     uint32_t capacity;   // paths the buffers hold
+    uint32_t finish;     // the megabatches are small: their last bounces in one kernel
     uint32_t shade_blocks_per_cu;
 };
 // Enqueues raygen, max_depth x (extend, shade, shadow) and the film update

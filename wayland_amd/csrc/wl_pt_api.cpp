@@ -615,13 +615,13 @@ static wl_status render_two_lanes(wl_scene s, const wl_pt_config *c, float *film
             P.frame0 = c->frame_offset + s0;
             P.pix0 = p0;
             P.npix = na;
-            WL_HIP_CHECK(wl::pt_run_batch(P, S, B, s->ctx->num_cus, hs));
+            WL_HIP_CHECK(wl::pt_run_batch(P, S, B, false, s->ctx->num_cus, hs));
             WL_HIP_CHECK(wl::pt_accumulate(P, B, film, s->ctx->num_cus, hs));
             if (nb)
             {
                 P.pix0 = p0 + na;
                 P.npix = nb;
-                WL_HIP_CHECK(wl::pt_run_batch(P, S, B2, s->ctx->num_cus, h2));
+                WL_HIP_CHECK(wl::pt_run_batch(P, S, B2, false, s->ctx->num_cus, h2));
                 WL_HIP_CHECK(wl::pt_accumulate(P, B2, film, s->ctx->num_cus, h2));
             }
         }
@@ -690,7 +690,7 @@ wl_status wl_pt_render(wl_scene s, const wl_pt_config *c, float *film,
             P.npix = std::min(tile, npix_total - p0);
             P.nsamples = nss;
             P.frame0 = c->frame_offset + s0;
-            WL_HIP_CHECK(wl::pt_run_batch(P, S, B, s->ctx->num_cus, hs));
+            WL_HIP_CHECK(wl::pt_run_batch(P, S, B, true, s->ctx->num_cus, hs));
             WL_HIP_CHECK(wl::pt_accumulate(P, B, film, s->ctx->num_cus, hs));
             st = after_batch(s, P, B, hs);
             if (st != WL_SUCCESS)
@@ -720,7 +720,7 @@ static wl_status one_frame(wl_scene s, const wl_pt_config *c, uint32_t frame,
     P.npix = np;
     P.nsamples = 1;
     P.frame0 = frame;
-    WL_HIP_CHECK(wl::pt_run_batch(P, scene_view(s), B, s->ctx->num_cus, hs));
+    WL_HIP_CHECK(wl::pt_run_batch(P, scene_view(s), B, true, s->ctx->num_cus, hs));
     return after_batch(s, P, B, hs);
 }
 

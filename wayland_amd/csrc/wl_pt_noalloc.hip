@@ -119,7 +119,7 @@ extern "C" wl_status wl_pt_render_noalloc(wl_scene s, const wl_pt_config *c, flo
             P.npix = std::min(tile, npix_total - p0);
             P.nsamples = nss;
             P.frame0 = c->frame_offset + s0;
-            WL_HIP_CHECK(wl::pt_run_batch(P, S, B, s->ctx->num_cus, hs));
+            WL_HIP_CHECK(wl::pt_run_batch(P, S, B, true, s->ctx->num_cus, hs));
             WL_HIP_CHECK(wl::pt_accumulate(P, B, film, s->ctx->num_cus, hs));
         }
     }

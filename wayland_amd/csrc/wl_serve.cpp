@@ -242,11 +242,12 @@ wl_status validate_requests(wl_server s, const wl_serve_config &cfg,
     return WL_SUCCESS;
 }
 
+// `lanes`: how many run at once.
 // Builds the lane's plan and arena and enqueues its megabatches on s->stream
 // after the work already on `user` (the requests are validated); returns
 // without waiting.
 wl_status run_lane(wl_server s, const wl_serve_config &cfg, const wl_render_request *reqs,
-                   uint32_t n, hipStream_t user, LaneRun &out)
+                   uint32_t n, uint32_t lanes, hipStream_t user, LaneRun &out)
 {
     wl_status st = WL_SUCCESS;
     std::vector<wl::PtReq> hreq(n);
@@ -342,6 +343,10 @@ wl_status run_lane(wl_server s, const wl_serve_config &cfg, const wl_render_requ
     L.max_depth = max_depth;
     L.stack16 = max_bvh <= 16 && wl_bvh8_narrow(arena_nodes, arena_tris) ? 1u : 0u;
     L.capacity = s->capacity;
+    uint64_t largest = 0; // megabatch, in paths
+    for (const wl::PtBatchHeader &h : pl.batches)
+        largest = std::max<uint64_t>(largest, h.paths);
+    L.finish = largest * lanes < wl::kFinishMaxPaths ? 1u : 0u;
     L.shade_blocks_per_cu = cfg.shade_blocks_per_cu;
 
     hipEvent_t ready;
@@ -369,6 +374,7 @@ wl_status run_lane(wl_server s, const wl_serve_config &cfg, const wl_render_requ
         std::vector<uint64_t> key = {
             max_depth,
             L.stack16,
+            L.finish,
             cfg.shade_blocks_per_cu,
             s->capacity,
             (uint64_t)(uintptr_t)s->d_buf,
@@ -482,7 +488,7 @@ wl_status run(wl_server s, const wl_render_request *reqs, uint32_t n, wl_serve_s
     LaneRun lr[2];
     st = WL_SUCCESS;
     for (uint32_t l = 0; l < used && st == WL_SUCCESS; ++l)
-        st = run_lane(lane[l], cfg, sub[l].data(), (uint32_t)sub[l].size(), user, lr[l]);
+        st = run_lane(lane[l], cfg, sub[l].data(), (uint32_t)sub[l].size(), used, user, lr[l]);
     unsigned long long origin = 0;
     if (st == WL_SUCCESS)
     {

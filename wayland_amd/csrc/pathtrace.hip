@@ -44,6 +44,24 @@ namespace wl
 
 constexpr int kPtBlock = 256;
 
+// A pointer to device memory that was itself loaded from memory (a request's
+// scene): without this the compiler reads through it with flat instructions,
+// which wait on the LDS counter too.
+template <class T>
+__device__ __forceinline__ const T *global_ptr(const T *p)
+{
+    return (const T *)(const __attribute__((address_space(1))) T *)(uintptr_t)p;
+}
+
+// b if parity, else a.  Written on the address bits: as a select between two
+// members of PtBuffers the compiler indexes a copy of them in scratch memory.
+template <class T>
+__device__ __forceinline__ T *pick(int parity, T *a, T *b)
+{
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return (T *)(__attribute__((address_space(1))) T *)(x ^ ((x ^ y) & (0 - (uintptr_t)parity)));
+}
+
 // ---- queues -------------------------------------------------------------------
 // XCD x's queue lengths of one parity: low word the ray queue's segment, high
 // word the shadow queue's.
@@ -244,7 +262,7 @@ __device__ __forceinline__ void queue_fetch(const PtBuffers &B, int parity,
     // the ray queues carry the path's lastPdf and seed in the rays' w words
     // (the shade pass reads its state back from the ray): every extension ray
     // is traced on [epsilon, 1e30], epsilon the batch's or the ray's request's
-    const wl_ray *rays = parity ? B.rays1 : B.rays0;
+    const wl_ray *rays = pick(parity, B.rays0, B.rays1);
     const f4v *rp = reinterpret_cast<const f4v *>((shadow ? B.srays : rays) + i);
     const f4v a = __builtin_nontemporal_load(rp), b = __builtin_nontemporal_load(rp + 1);
     float tmin = a.w, tmax = b.w;
@@ -259,7 +277,7 @@ __device__ __forceinline__ void queue_fetch(const PtBuffers &B, int parity,
             root = B.sreq[i];
         else
         {
-            const PtReq &rq = reqs[(parity ? B.qreq1 : B.qreq0)[i]];
+            const PtReq &rq = reqs[pick(parity, B.qreq0, B.qreq1)[i]];
             root = rq.root;
             tmin = rq.P.epsilon;
         }
@@ -633,6 +651,7 @@ void k_guide_infer_pt(PtParams P, PtScene S, PtBuffers B, int parity)
 // materials behind a branch and one sine and cosine for all lobes, two 1024^2
 // Cornell frames 2.53 -> 2.32 ms, 256 small serving requests 9.2 -> 8.8 ms.  Four
 // waves per SIMD: five (96 VGPRs, no spills) is 2-6 % slower.
+// What a shaded vertex does next.
 struct Vertex
 {
     bool cont = false, shadow = false, shadow_gacc = false;
@@ -648,12 +667,13 @@ __device__ __forceinline__ void shade_vertex(const PtParams &P0, const PtScene &
                                              const PtReq *__restrict__ reqs, int first, uint32_t i,
                                              Vertex &out)
 {
-    const uint32_t *qin = parity ? B.qpath1 : B.qpath0;
+    const uint32_t *qin = pick(parity, B.qpath0, B.qpath1);
+    const uint32_t *req_in = pick(parity, B.qreq0, B.qreq1);
     // the first queue is the identity: entry i is path i
     const bool ident = first != 0;
     out.path = ident ? i : qin[i];
     if (MULTI)
-        out.req = (parity ? B.qreq1 : B.qreq0)[i];
+        out.req = req_in[i];
     const PtReq *rq = MULTI ? reqs + out.req : nullptr;
     if (MULTI)
         out.root = rq->root;
@@ -689,7 +709,7 @@ __device__ __forceinline__ void shade_vertex(const PtParams &P0, const PtScene &
         // the ray this pass shades: origin and lastPdf, then the
         // direction and the seed (written so by the last pass)
         const float4 *rp =
-            reinterpret_cast<const float4 *>((parity ? B.rays1 : B.rays0) + i);
+            reinterpret_cast<const float4 *>(pick(parity, B.rays0, B.rays1) + i);
         s_pos = rp[0];
         s_dir = rp[1];
         s_thr = B.thr[out.path];
@@ -736,17 +756,17 @@ __device__ __forceinline__ void shade_vertex(const PtParams &P0, const PtScene &
     {
         depth += 1;
         const float t = hit.x, b1 = hit.z, b2 = hit.w;
-        const float4 *sr = reinterpret_cast<const float4 *>(S.prims) + 3 * (size_t)prim;
+        const float4 *sr = reinterpret_cast<const float4 *>(global_ptr(S.prims)) + 3 * (size_t)prim;
         const float4 w0 = sr[0], w1 = sr[1], w2 = sr[2];
         const V3 va = mk(w0.x, w0.y, w0.z), vb = mk(w0.w, w1.x, w1.y),
                  vc = mk(w1.z, w1.w, w2.x);
         const uint32_t mesh = __float_as_uint(w2.y);
-        const PtMesh M = S.meshes[mesh];
+        const PtMesh M = global_ptr(S.meshes)[mesh];
         V3 Ng = normalize(cross(vb - va, vc - va));
         V3 Ns;
         if (M.has_normal)
         {
-            const float4 *nr = reinterpret_cast<const float4 *>(S.normals) + 3 * (size_t)prim;
+            const float4 *nr = reinterpret_cast<const float4 *>(global_ptr(S.normals)) + 3 * (size_t)prim;
             const float4 n0 = nr[0], n1 = nr[1], n2 = nr[2];
             const V3 na = mk(n0.x, n0.y, n0.z), nb = mk(n0.w, n1.x, n1.y),
                      nc = mk(n1.z, n1.w, n2.x);
@@ -757,7 +777,7 @@ __device__ __forceinline__ void shade_vertex(const PtParams &P0, const PtScene &
         const V3 hitPos = rayPos + rayDir * t;
         if (M.light != WL_INVALID)
         {
-            const PtLight lt = S.lights[M.light];
+            const PtLight lt = global_ptr(S.lights)[M.light];
             if (depth == 1 || (P.strategy != WL_STRATEGY_NEE &&
                                (lt.two_sided || dot(Ns, rayDir) < 0)))
             {
@@ -787,18 +807,18 @@ __device__ __forceinline__ void shade_vertex(const PtParams &P0, const PtScene &
         }
         else
         {
-            const Mat mat = load_mat(S.materials + M.material);
+            const Mat mat = load_mat(global_ptr(S.materials) + M.material);
             // texture colour (PathTracing.cu:261-268)
             V3 tex = mk(1, 1, 1);
             if (M.texture != WL_INVALID)
             {
-                const float4 *ur = reinterpret_cast<const float4 *>(S.uvs) + 2 * (size_t)prim;
+                const float4 *ur = reinterpret_cast<const float4 *>(global_ptr(S.uvs)) + 2 * (size_t)prim;
                 const float4 u01 = ur[0], u2 = ur[1];
                 const float w0 = 1 - b1 - b2;
                 const float tu = (u01.x * w0 + u01.z * b1) + u2.x * b2;
                 const float tv = (u01.y * w0 + u01.w * b1) + u2.y * b2;
-                const PtTexture T = S.textures[M.texture];
-                tex = tex_bilinear(S.texels + T.offset, T.width, T.height, tu, tv);
+                const PtTexture T = global_ptr(S.textures)[M.texture];
+                tex = tex_bilinear(global_ptr(S.texels) + T.offset, T.width, T.height, tu, tv);
             }
             if (mat.trans < 0.1f)
             {
@@ -902,13 +922,13 @@ __device__ __forceinline__ void shade_vertex(const PtParams &P0, const PtScene &
                 {
                     uint32_t lid = (uint32_t)((float)P.num_lights * rnd(seed));
                     lid = lid < P.num_lights ? lid : P.num_lights - 1;
-                    const PtLight lt = S.lights[lid];
+                    const PtLight lt = global_ptr(S.lights)[lid];
                     float lpdf = 1.0f / (float)P.num_lights;
                     uint32_t triIdx = (uint32_t)(rnd(seed) * (float)lt.tri_count);
                     triIdx = triIdx < lt.tri_count ? triIdx : lt.tri_count - 1;
                     lpdf = lpdf / (float)lt.tri_count;
                     const uint32_t lprim = lt.tri_offset + triIdx;
-                    const float4 *lr = reinterpret_cast<const float4 *>(S.prims) + 3 * (size_t)lprim;
+                    const float4 *lr = reinterpret_cast<const float4 *>(global_ptr(S.prims)) + 3 * (size_t)lprim;
                     const float4 l0 = lr[0], l1 = lr[1], l2 = lr[2];
                     const V3 p0 = mk(l0.x, l0.y, l0.z), p1 = mk(l0.w, l1.x, l1.y),
                              p2 = mk(l1.z, l1.w, l2.x);
@@ -924,7 +944,7 @@ __device__ __forceinline__ void shade_vertex(const PtParams &P0, const PtScene &
                     V3 lN;
                     if (lt.has_normal)
                     {
-                        const float4 *nr = reinterpret_cast<const float4 *>(S.normals) + 3 * (size_t)lprim;
+                        const float4 *nr = reinterpret_cast<const float4 *>(global_ptr(S.normals)) + 3 * (size_t)lprim;
                         const float4 n0 = nr[0], n1 = nr[1], n2 = nr[2];
                         const V3 na = mk(n0.x, n0.y, n0.z), nb = mk(n0.w, n1.x, n1.y),
                                  nc = mk(n1.z, n1.w, n2.x);
@@ -1014,10 +1034,10 @@ __device__ __forceinline__ void store_vertex(const PtBuffers &B, int parity, con
 {
     if (v.cont)
     {
-        (parity ? B.qpath0 : B.qpath1)[slot] = v.path;
-        (parity ? B.rays0 : B.rays1)[slot] = v.next_ray;
+        pick(parity, B.qpath1, B.qpath0)[slot] = v.path;
+        pick(parity, B.rays1, B.rays0)[slot] = v.next_ray;
         if (MULTI)
-            (parity ? B.qreq0 : B.qreq1)[slot] = v.req;
+            pick(parity, B.qreq1, B.qreq0)[slot] = v.req;
     }
     if (v.shadow)
     {

@@ -1,0 +1,78 @@
+"""The builder's collapse to 8-wide nodes on trees where the choice by cost and
+the greedy one part ways: chains of shrinking triangles, boxes without area,
+triangle counts around the leaf and node sizes."""
+import numpy as np
+import pytest
+
+import hostemu_bind as hb
+import oracle_bind as ob
+from wayland_amd import scenes
+
+
+def _chain(n, f):
+    rng = np.random.default_rng(1)
+    s = f ** np.arange(n)
+    t = rng.uniform(-1, 1, (n, 3, 3)) * 0.4 + np.array([1.0, 0.3, -0.2])
+    return np.ascontiguousarray((t * s[:, None, None]).reshape(n, 9), np.float32)
+
+
+def _check(tris, rays):
+    h = hb.HostBVH8(tris)
+    hits, _, faults = h.trace(rays)
+    assert faults == 0
+    ref = ob.closest_brute(tris, rays)
+    assert np.array_equal(hits[:, 1].view(np.uint32), ref["prim"])
+    assert np.array_equal(hits[:, 0].view(np.uint32), ref["t"].view(np.uint32))
+    anyhit, _, faults = h.trace(rays, any_hit=True)
+    assert faults == 0
+    assert np.array_equal(anyhit[:, 1].view(np.uint32) != 0xFFFFFFFF,
+                          ref["prim"] != 0xFFFFFFFF)
+    return h.info()
+
+
+def _rays(seed):
+    rays = scenes.traversal_rays(3000, seed=seed)
+    rays[:, 0:3] = rays[:, 0:3] * 4 - 2
+    return rays
+
+
+@pytest.mark.parametrize("n,f,depth", [
+    (160, 0.55, 21), (250, 0.5, 22), (300, 0.65, 24), (340, 0.7, 32)])
+def test_shrinking_chain_stays_in_the_stack(n, f, depth):
+    """By cost alone these trees are deeper than the stack: they are built as
+    deep as the greedy collapse makes them, and traced."""
+    assert _check(_chain(n, f), _rays(n))["depth"] <= depth
+
+
+def test_chain_beyond_the_stack_is_refused():
+    with pytest.raises(Exception, match="exceeds the traversal stack"):
+        hb.HostBVH8(_chain(400, 0.75))
+
+
+@pytest.mark.parametrize("kind", ["points", "one point", "segments", "tiny", "mixed"])
+def test_boxes_without_area(kind):
+    """Costs that are all zero, or drowned by their parent's."""
+    rng = np.random.default_rng(7)
+    p = rng.uniform(0, 1, (300, 1, 3)).astype(np.float32)
+    tri = rng.uniform(-1, 1, (300, 3, 3)).astype(np.float32)
+    if kind == "points":
+        tris = np.repeat(p, 3, axis=1)
+    elif kind == "one point":
+        tris = np.repeat(p[:1], 900, axis=0).reshape(300, 3, 3)
+    elif kind == "segments":
+        tris = tri * np.array([1, 0, 0], np.float32)
+    elif kind == "tiny":
+        tris = p + tri * np.float32(1e-25)
+    else:
+        tris = np.concatenate([np.repeat(p, 3, axis=1), tri, tri * np.float32(1e-22)])
+    tris = np.ascontiguousarray(tris.reshape(-1, 9), np.float32)
+    _check(tris, _rays(8))
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 7, 8, 9, 31, 32, 33, 36, 37, 65, 257])
+def test_counts_around_leaf_and_node_sizes(n):
+    rng = np.random.default_rng(n)
+    c = rng.uniform(0, 1, (n, 1, 3))
+    tris = (c + rng.uniform(-0.2, 0.2, (n, 3, 3))).astype(np.float32).reshape(n, 9)
+    info = _check(np.ascontiguousarray(tris), _rays(n))
+    assert info["tris"] == n

@@ -42,6 +42,7 @@
 #include <stdint.h>
 
 #define WL_BVH8_STACK_DEPTH 32
+#define WL_BVH8_SHALLOW_DEPTH 16 // trees up to here: half the stack, more wavefronts
 #define WL_BVH8_MAX_LEAF_TRIS 4
 
 struct alignas(16) WlBvh8Node

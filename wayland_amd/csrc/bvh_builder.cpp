@@ -1,5 +1,6 @@
-// bvh_builder.cpp — host SAH builder: binned-SAH BVH2, greedy collapse to
-// BVH8, octant slot ordering and 16-bit outward-rounded box quantisation.
+// bvh_builder.cpp — host SAH builder: binned-SAH BVH2, collapse to BVH8 by
+// dynamic programming over its subtrees, octant slot ordering and 16-bit
+// outward-rounded box quantisation.
 // Replaces the closed GPU builder behind optixAccelBuild
 // (src/Backend/Optix/Core/AccelStructure.cpp:133-162).
 #include "bvh_builder.h"
@@ -62,9 +63,30 @@ struct Aabb
 struct Node2
 {
     Aabb box;
-    uint32_t left = 0, right = 0; // inner
-    uint32_t first = 0, count = 0; // leaf (count > 0)
+    uint32_t left = 0, right = 0; // inner; both after their parent
+    uint32_t first = 0, total = 0; // the subtree's range of prims
+    uint32_t count = 0;            // total in a leaf, 0 in an inner node
 };
+
+// The cheapest way to hang a BVH2 subtree into an 8-wide node (after Ylitie,
+// Karras, Laine, HPG 2017, who follow Aila and others): cost[k - 1] is the
+// SAH cost of it as at most k children, k = 1..7.  A single child is a leaf of
+// the subtree's triangles or a node of its own; k children are i from the left
+// subtree and k - i from the right: nibble k - 2 of `split` holds the i of
+// k = 2..7, 0 where k - 1 children cost no more.  The subtree's own node has
+// own_k children, own_i of them from the left.
+// Against opening the largest child until eight are found: the 2M-triangle soup
+// takes 268,000 nodes instead of 497,000 and 5.72 visits a ray instead of 5.89;
+// 1080p x 64 spp 35.5 -> 34.6 ms, 1M caustic paths 1.45 -> 1.40 ms, 100,003 rays
+// 65 -> 60 us, 2^23 closest hits 680 -> 672 us.
+struct Collapse
+{
+    float cost[7];
+    uint32_t split : 24, own_k : 4, own_i : 4;
+};
+// Cost of a triangle test relative to a node visit: 1.5 and 2.5 are equally
+// fast, 1.0 (more triangles per leaf) is 2-3 % slower, 0.6 7 %.
+constexpr float kTriCost = 2.0f;
 
 struct Bvh2Builder
 {
@@ -94,6 +116,8 @@ struct Bvh2Builder
             }
             nd.box = box;
             uint32_t cnt = end - begin;
+            nd.first = begin;
+            nd.total = cnt;
             int best_axis = -1, best_bin = 0;
             double best_cost = std::numeric_limits<double>::infinity();
             double leaf_cost = (double)cnt;
@@ -151,7 +175,6 @@ struct Bvh2Builder
                              (best_axis < 0 || leaf_cost <= best_cost);
             if (cnt == 0 || make_leaf)
             {
-                nd.first = begin;
                 nd.count = cnt;
                 return;
             }
@@ -195,6 +218,95 @@ struct Bvh2Builder
     }
 };
 
+// The collapse choice of every subtree (children come after their parents);
+// subtrees that are cheaper as one leaf become leaves.
+std::vector<Collapse> choose_collapse(std::vector<Node2> &nodes, uint32_t n)
+{
+    std::vector<Collapse> out(n);
+    for (uint32_t i = n; i-- > 0;)
+    {
+        Node2 &nd = nodes[i];
+        Collapse &c = out[i];
+        const float area = (float)nd.box.area();
+        c.split = 0;
+        c.own_k = 0;
+        c.own_i = 0;
+        if (nd.count > 0 || nd.total == 0)
+        {
+            for (float &x : c.cost)
+                x = area * kTriCost * (float)nd.total;
+            continue;
+        }
+        const float *l = out[nd.left].cost, *r = out[nd.right].cost;
+        float as[9]; // cost as k children, k = 2..8, and the left subtree's share
+        uint32_t share[9];
+        for (uint32_t k = 2; k <= 8; ++k)
+        {
+            float best = INFINITY;
+            uint32_t at = 1;
+            for (uint32_t j = 1; j < k; ++j)
+                if (l[j - 1] + r[k - j - 1] < best)
+                {
+                    best = l[j - 1] + r[k - j - 1];
+                    at = j;
+                }
+            as[k] = best;
+            share[k] = at;
+        }
+        uint32_t own = 8;
+        for (uint32_t k = 7; k >= 2; --k)
+            if (as[k] <= as[own])
+                own = k;
+        c.own_k = own;
+        c.own_i = share[own];
+        c.cost[0] = area + as[own];
+        const float leaf = area * kTriCost * (float)nd.total;
+        if (nd.total <= WL_BVH8_MAX_LEAF_TRIS && leaf <= c.cost[0])
+        {
+            c.cost[0] = leaf;
+            nd.count = nd.total;
+        }
+        for (uint32_t k = 2; k <= 7; ++k)
+        {
+            const bool fewer = c.cost[k - 2] <= as[k];
+            c.cost[k - 1] = fewer ? c.cost[k - 2] : as[k];
+            if (!fewer)
+                c.split |= share[k] << (4 * (k - 2));
+        }
+    }
+    return out;
+}
+
+// The children of node n's 8-wide node under that choice.
+void chosen_children(const std::vector<Node2> &nodes, const std::vector<Collapse> &choice,
+                     uint32_t n, std::vector<uint32_t> &kids)
+{
+    struct Part
+    {
+        uint32_t node, k; // subtree, children it may take
+    };
+    Part stack[16]; // at most eight parts are open at once
+    int sp = 0;
+    stack[sp++] = { nodes[n].left, choice[n].own_i };
+    stack[sp++] = { nodes[n].right, (uint32_t)(choice[n].own_k - choice[n].own_i) };
+    while (sp > 0)
+    {
+        Part p = stack[--sp];
+        const Node2 &nd = nodes[p.node];
+        uint32_t at = 0;
+        if (nd.count == 0)
+            while (p.k > 1 && (at = choice[p.node].split >> (4 * (p.k - 2)) & 0xFu) == 0)
+                --p.k;
+        if (at == 0) // a child by itself
+        {
+            kids.push_back(p.node);
+            continue;
+        }
+        stack[sp++] = { nd.left, at };
+        stack[sp++] = { nd.right, p.k - at };
+    }
+}
+
 inline float exp2i(int e) { return std::ldexp(1.0f, e); }
 
 // Quantised planes are integers 0..kQMax, stored as binary16 (exact for
@@ -233,34 +345,15 @@ uint16_t half_of_int(int n)
 }
 constexpr uint16_t kHalfMaxFinite = 0x7BFF; // 65504: the empty slot's lo plane
 
-} // namespace
+constexpr size_t kMaxNodes = (size_t)0xFFFFFF * 8; // 24-bit node-group index
 
-bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
-                std::string *err)
+// BVH2 -> BVH8 (breadth-first, so the top levels sit together): by `choice`, or
+// without one by opening the largest child until there are eight.  Returns the
+// SAH cost (node 1, triangle 1).
+double collapse_bvh8(const float *tris, uint32_t ntris, const std::vector<Node2> &nodes,
+                     const std::vector<uint32_t> &prims, const std::vector<Collapse> *choice,
+                     Bvh8Host *out)
 {
-    auto t0 = std::chrono::steady_clock::now();
-    Bvh2Builder b;
-    b.tris = tris;
-    b.n = ntris;
-    b.pbox.resize(ntris);
-    b.cen.resize(3 * (size_t)ntris);
-    b.prims.resize(ntris);
-    for (uint32_t i = 0; i < ntris; ++i)
-    {
-        Aabb a;
-        for (int v = 0; v < 3; ++v)
-            a.grow_point(tris + 9 * (size_t)i + 3 * v);
-        b.pbox[i] = a;
-        for (int k = 0; k < 3; ++k)
-            b.cen[3 * (size_t)i + k] = 0.5f * (a.lo[k] + a.hi[k]);
-        b.prims[i] = i;
-    }
-    b.nodes.resize(std::max<size_t>(1, 2 * (size_t)ntris));
-    b.next_node = 1;
-    b.threads_left = std::max(0, nthreads - 1);
-    b.build_range(0, 0, ntris);
-
-    // ---- collapse to BVH8 (breadth-first, so the top levels sit together)
     out->nodes.clear();
     out->tris.clear();
     // the root owns a group of 8 slots like every other node, so that every
@@ -270,7 +363,7 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
     out->depth = 1;
     out->inner_nodes = 0;
     out->leaves = 0;
-    double root_area = b.nodes[0].box.area();
+    double root_area = nodes[0].box.area();
     double sah = 0.0;
     struct Work
     {
@@ -284,13 +377,15 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
         queue.pop_front();
         out->depth = std::max(out->depth, w.depth);
         out->inner_nodes++;
-        const Node2 &src = b.nodes[w.n2];
+        const Node2 &src = nodes[w.n2];
         std::vector<uint32_t> kids;
         if (src.count > 0 || ntris == 0)
         {
             if (ntris > 0)
                 kids.push_back(w.n2);
         }
+        else if (choice)
+            chosen_children(nodes, *choice, w.n2, kids);
         else
         {
             kids.push_back(src.left);
@@ -301,7 +396,7 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
                 double best_area = -1.0;
                 for (size_t i = 0; i < kids.size(); ++i)
                 {
-                    const Node2 &k = b.nodes[kids[i]];
+                    const Node2 &k = nodes[kids[i]];
                     if (k.count == 0 && k.box.area() > best_area)
                     {
                         best_area = k.box.area();
@@ -311,8 +406,8 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
                 if (best < 0)
                     break;
                 uint32_t id = kids[best];
-                kids[best] = b.nodes[id].left;
-                kids.push_back(b.nodes[id].right);
+                kids[best] = nodes[id].left;
+                kids.push_back(nodes[id].right);
             }
         }
         if (root_area > 0)
@@ -329,7 +424,7 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
             double cost[8][8];
             for (size_t i = 0; i < kids.size(); ++i)
             {
-                const Aabb &cb = b.nodes[kids[i]].box;
+                const Aabb &cb = nodes[kids[i]].box;
                 double off[3];
                 for (int k = 0; k < 3; ++k)
                     off[k] = 0.5 * ((double)cb.lo[k] + cb.hi[k]) - pc[k];
@@ -385,7 +480,7 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
         }
         bool any_inner = false;
         for (size_t i = 0; i < kids.size(); ++i)
-            if (b.nodes[kids[i]].count == 0)
+            if (nodes[kids[i]].count == 0)
                 any_inner = true;
         if (any_inner)
         {
@@ -402,7 +497,7 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
                     i = (int)j;
             if (i < 0)
                 continue;
-            const Node2 &k = b.nodes[kids[i]];
+            const Node2 &k = nodes[kids[i]];
             for (int a = 0; a < 3; ++a)
             {
                 double qlo = std::floor(((double)k.box.lo[a] - node.p[a]) / scale[a]) - 1.0;
@@ -422,7 +517,7 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
                 node.trivalid |= ((1u << k.count) - 1u) << (4 * s);
                 for (uint32_t t = 0; t < k.count; ++t)
                 {
-                    uint32_t p = b.prims[k.first + t];
+                    uint32_t p = prims[k.first + t];
                     WlTriRecord r;
                     std::memcpy(r.v0, tris + 9 * (size_t)p, 36);
                     r.prim = p;
@@ -437,6 +532,55 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
         }
         out->nodes[w.n8] = node;
     }
+    return sah;
+}
+
+} // namespace
+
+bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
+                std::string *err)
+{
+    auto t0 = std::chrono::steady_clock::now();
+    Bvh2Builder b;
+    b.tris = tris;
+    b.n = ntris;
+    b.pbox.resize(ntris);
+    b.cen.resize(3 * (size_t)ntris);
+    b.prims.resize(ntris);
+    for (uint32_t i = 0; i < ntris; ++i)
+    {
+        Aabb a;
+        for (int v = 0; v < 3; ++v)
+            a.grow_point(tris + 9 * (size_t)i + 3 * v);
+        b.pbox[i] = a;
+        for (int k = 0; k < 3; ++k)
+            b.cen[3 * (size_t)i + k] = 0.5f * (a.lo[k] + a.hi[k]);
+        b.prims[i] = i;
+    }
+    b.nodes.resize(std::max<size_t>(1, 2 * (size_t)ntris));
+    b.next_node = 1;
+    b.threads_left = std::max(0, nthreads - 1);
+    b.build_range(0, 0, ntris);
+
+    const uint32_t n2 = b.next_node;
+    double sah;
+    {
+        // The greedy collapse is kept for trees that the choice makes deeper
+        // than the kernels' short stack: chains of ever smaller triangles, of
+        // which it opens the large near ones first (300 triangles that shrink
+        // by 0.65 each: 39 levels, 24 greedily).
+        std::vector<uint32_t> leaf_of(n2);
+        for (uint32_t i = 0; i < n2; ++i)
+            leaf_of[i] = b.nodes[i].count;
+        const std::vector<Collapse> choice = choose_collapse(b.nodes, n2);
+        sah = collapse_bvh8(tris, ntris, b.nodes, b.prims, &choice, out);
+        if (out->depth > WL_BVH8_SHALLOW_DEPTH || out->nodes.size() > kMaxNodes)
+        {
+            for (uint32_t i = 0; i < n2; ++i)
+                b.nodes[i].count = leaf_of[i];
+            sah = collapse_bvh8(tris, ntris, b.nodes, b.prims, nullptr, out);
+        }
+    }
     out->sah_cost = sah;
     auto t1 = std::chrono::steady_clock::now();
     out->build_seconds = std::chrono::duration<double>(t1 - t0).count();
@@ -448,7 +592,7 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
                    std::to_string(WL_BVH8_STACK_DEPTH);
         return false;
     }
-    if (out->nodes.size() > (size_t)0xFFFFFF * 8)
+    if (out->nodes.size() > kMaxNodes)
     {
         if (err)
             *err = "BVH8 node count exceeds the 24-bit node-group index";

@@ -20,6 +20,9 @@
 //              reference's RNG draw order; appends the continuing paths and
 //              the shadow rays to compacted queues (wave64 ballot + mbcnt
 //              prefix, one atomic per workgroup).
+//   finish     batches that are small and alone: all bounces after the second
+//              in one kernel, every workgroup looping over a slice of the queue
+//              (k_finish).
 //   accumulate compensated (Kahan) FP32 film: sum + compensation per pixel.
 //
 // Radiance contributions reach a path in the reference's order (one per
@@ -1476,7 +1479,7 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B0
     const uint32_t blocks_all = (npaths + kPtBlock - 1) / kPtBlock;
     // a BVH at most 16 deep needs at most 15 stack entries per lane; those
     // kernels also address nodes and triangles with 32-bit offsets
-    const bool shallow = S.bvh_depth <= 16 && wl_bvh8_narrow(S.num_nodes, S.num_tris);
+    const bool shallow = S.bvh_depth <= WL_BVH8_SHALLOW_DEPTH && wl_bvh8_narrow(S.num_nodes, S.num_tris);
     // persistent traversal grids: the workgroups that fit the GPU at once.  All
     // grids are multiples of 8 (each XCD its share).
     static int occ16 = 0, occ32 = 0, occf16 = 0, occf32 = 0;

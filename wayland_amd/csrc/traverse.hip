@@ -151,7 +151,7 @@ __global__ void k_zero_words(uint32_t *words, uint32_t nwords)
 // The 16-entry stack kernels: also 32-bit node and triangle offsets.
 static inline bool shallow(const wl_accel_s *a)
 {
-    return a->info.depth <= 16 && wl_bvh8_narrow(a->num_nodes, a->num_tri_records);
+    return a->info.depth <= WL_BVH8_SHALLOW_DEPTH && wl_bvh8_narrow(a->num_nodes, a->num_tri_records);
 }
 
 // Persistent grid: the workgroups that fit the GPU at once (the launch then

@@ -143,8 +143,8 @@ constexpr uint32_t kFinishMaxPaths = 1u << 22;
 // ---- batched serving: one megabatch mixes paths of many requests ----------
 // A request's scene, parameters and film; the ray queues of a multi-request
 // batch carry each entry's request id (qreq0/qreq1), the shadow queue the
-// root of the request's BVH in the node arena (sreq), the one thing the
-// shadow kernel needs.
+// root of the request's BVH in the node arena (sreq), the one thing
+// that tracing it needs.
 struct PtReq
 {
     PtParams P; // pix0 / npix / nsamples / frame0 unused; gmode 0
@@ -192,7 +192,7 @@ struct PtMultiLaunch
     uint32_t finish;     // the megabatches are small: their last bounces in one kernel
     uint32_t shade_blocks_per_cu;
 };
-// Enqueues raygen, max_depth x (extend, shade, shadow) and the film update
+// Enqueues raygen, the first trace, max_depth x (shade, trace) and the film update
 // of one megabatch; every count comes from device memory, so the sequence
 // can be captured once into a hipGraph and replayed.
 hipError_t pt_run_multi(const PtMultiLaunch &L, const PtBuffers &B, int num_cus,

@@ -4,7 +4,7 @@
 // (DeviceManager::Launch, src/Frontend/Core/DeviceManager.cpp:231-241);
 // here the scheduler packs whole requests x sample ranges into megabatches
 // of up to batch_paths paths, and a render call's whole megabatch sequence
-// (per megabatch: raygen, max_depth x extend / shade / shadow, film update)
+// (per megabatch: raygen, first trace, max_depth x shade / trace, film update)
 // is captured into one hipGraph and launched once: the batch descriptors live
 // in device memory and each megabatch's first kernel picks the next one, so
 // the host enqueues one graph launch per lane (one per kGraphBatches

@@ -240,6 +240,38 @@ __device__ __forceinline__ float guide_loss_grad(const floatx4 out[2], V3 om, fl
     return -w * logq;
 }
 
+// The staged layer inputs and deltas: per 16 samples a block of rows, one per
+// feature, of 16 samples each (rows a whole mini-batch long, a power of two
+// apart, met in the same cache sets and L2 channel; the weight-gradient kernel
+// gained from the change, this one's time, its one tile's serial chain, stayed
+// at 16.4 us for 16,384 samples).  Writes the 32 rows from
+// `rows` of a B operand: lane l holds features phi(0, l / 16, 0..7) of sample
+// l % 16; each quad transposes its 4 samples x 8 features in registers, so a
+// lane stores 4 samples of two features and the wave two contiguous 512 B
+// instead of eight times four pieces of 32 B.
+__device__ __forceinline__ void store_feature_major(__bf16 *rows, int lane, bf16x8 v)
+{
+    uint32_t w[4];
+    __builtin_memcpy(w, &v, 16);
+    const uint32_t sel = lane & 1 ? 0x03020706u : 0x05040100u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) // feature 2 k + lane % 2 of two samples
+    {
+        const uint32_t o = __builtin_amdgcn_update_dpp(0, w[k], 0xB1, 0xF, 0xF, true); // lane ^ 1
+        w[k] = __builtin_amdgcn_perm(o, w[k], sel);
+    }
+    const bool hi = lane & 2;
+#pragma unroll
+    for (int k = 0; k < 4; k += 2) // feature 2 k + lane % 4 of four samples
+    {
+        const uint32_t o = __builtin_amdgcn_update_dpp(0, hi ? w[k] : w[k + 1], 0x4E, 0xF, 0xF,
+                                                       true); // lane ^ 2
+        const uint2 q = hi ? make_uint2(o, w[k + 1]) : make_uint2(w[k], o);
+        *reinterpret_cast<uint2 *>(rows + (guide_phi(0, lane >> 4, 2 * k) + (lane & 3)) * 16 +
+                                   (lane & 12)) = q;
+    }
+}
+
 __global__ __launch_bounds__(kGuideBlock) void k_guide_fwdbwd(GuideDev G,
                                                               const float *__restrict__ samples,
                                                               const uint32_t *__restrict__ n_dev, uint32_t n_cap,
@@ -260,7 +292,6 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_fwdbwd(GuideDev G,
     batch_range(*n_dev, n_cap, step, batch, offset, size);
     const uint32_t padded = (size + 31) & ~31u; // dw reads whole 32-sample steps
     const int lane = threadIdx.x & 63, g = lane >> 4;
-    const uint32_t cap = G.cap;
     __bf16 *XT = reinterpret_cast<__bf16 *>(G.xt);
     __bf16 *DT = reinterpret_cast<__bf16 *>(G.dt);
     const uint32_t nwaves = gridDim.x * (kGuideBlock / 64);
@@ -287,14 +318,19 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_fwdbwd(GuideDev G,
         if (valid && g == 0)
             G.loss[s] = loss;
         // layer inputs, feature-major
+        __bf16 *xt = XT + (size_t)tile * kGuideInRows * 16;
+        __bf16 *dt = DT + (size_t)tile * kGuideDeltaRows * 16;
 #pragma unroll
         for (int l = 0; l < 5; ++l)
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
+            {
+                bf16x8 v;
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
-                    XT[((size_t)l * 64 + guide_phi(kb, g, j)) * cap + s] =
-                        valid ? keep[l][kb][j] : (__bf16)0.0f;
+                    v[j] = valid ? keep[l][kb][j] : (__bf16)0.0f;
+                store_feature_major(xt + (l * 64 + 32 * kb) * 16, lane, v);
+            }
         // output delta: rows 16 t + 4 g + i = phi(0, g, 4 t + i)
         bf16x8 dB[2];
 #pragma unroll
@@ -302,8 +338,8 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_fwdbwd(GuideDev G,
         {
             dB[0][j] = (__bf16)d[j / 4][j % 4];
             dB[1][j] = (__bf16)0.0f;
-            DT[((size_t)256 + guide_phi(0, g, j)) * cap + s] = dB[0][j];
         }
+        store_feature_major(dt + 256 * 16, lane, dB[0]);
         // back through layers 4..1: delta_in = (W_l^T delta_out) * relu'(x_l)
 #pragma unroll
         for (int l = 4; l >= 1; --l)
@@ -319,18 +355,24 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_fwdbwd(GuideDev G,
             }
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
+            {
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
                 {
                     const float v = (float)keep[l][kb][j] > 0.f ? acc[2 * kb + j / 4][j % 4] : 0.f;
                     dB[kb][j] = (__bf16)v;
-                    DT[((size_t)(l - 1) * 64 + guide_phi(kb, g, j)) * cap + s] = dB[kb][j];
                 }
+                store_feature_major(dt + ((l - 1) * 64 + 32 * kb) * 16, lane, dB[kb]);
+            }
         }
     }
 }
 
 // ---- training: weight gradients --------------------------------------------------
+// Bound by reading the staged rows: 512 samples x 1,216 B a slice, each row by
+// four tiles or more.  At 16,384 samples 13.4 us with rows a mini-batch long
+// (16 pieces of 64 B, 32 KB apart, per load), 9.6 us with rows of 16 samples (a
+// load is two runs of 512 B), 6.7 us with a slice's tiles on one XCD.
 // Work item = (tile, split); tiles 0..63: layers 0..3, 4 x 4 tiles of 16 x 16;
 // tiles 64..71: layer 4, 2 x 4 tiles.  Tiles with im == 0 also sum the bias
 // gradient of their 16 rows.
@@ -338,10 +380,13 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_dw(GuideDev G,
                                                           const uint32_t *__restrict__ n_dev, uint32_t n_cap,
                                                           uint32_t step, uint32_t batch)
 {
-    const uint32_t item = blockIdx.x * (kGuideBlock / 64) + threadIdx.x / 64;
-    if (item >= 72u * kGuideSplits)
-        return;
-    const int tile = (int)(item % 72u), ks = (int)(item / 72u);
+    // workgroups go to the 8 XCDs in turn: XCD x takes the slices x, x + 8, ...
+    // whole, so that each slice of the staged rows passes one L2
+    static_assert(kGuideSplits % 8 == 0 && 72 % (kGuideBlock / 64) == 0);
+    constexpr uint32_t kBlocks = 72 / (kGuideBlock / 64); // per slice
+    const uint32_t at = blockIdx.x / 8;
+    const int ks = (int)(blockIdx.x % 8 + 8 * (at / kBlocks));
+    const int tile = (int)((at % kBlocks) * (kGuideBlock / 64) + threadIdx.x / 64);
     int l, om, im;
     if (tile < 64)
     {
@@ -361,11 +406,14 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_dw(GuideDev G,
     const uint32_t per = (steps + kGuideSplits - 1) / kGuideSplits;
     const uint32_t st0 = min(steps, (uint32_t)ks * per), st1 = min(steps, st0 + per);
     const int lane = threadIdx.x & 63, g = lane >> 4;
-    const uint32_t cap = G.cap;
+    // samples 8 g .. 8 g + 7 of a 32-sample step: half a row of its block g / 2
     const __bf16 *D = reinterpret_cast<const __bf16 *>(G.dt) +
-                      (size_t)(l < 4 ? l * 64 : 256) * cap + (size_t)(om * 16 + (lane & 15)) * cap;
-    const __bf16 *X = reinterpret_cast<const __bf16 *>(G.xt) + (size_t)l * 64 * cap +
-                      (size_t)(im * 16 + (lane & 15)) * cap;
+                      ((g >> 1) * kGuideDeltaRows + l * 64 + om * 16 + (lane & 15)) * 16 +
+                      8 * (g & 1);
+    const __bf16 *X = reinterpret_cast<const __bf16 *>(G.xt) +
+                      ((g >> 1) * kGuideInRows + l * 64 + im * 16 + (lane & 15)) * 16 +
+                      8 * (g & 1);
+    constexpr size_t kStepD = 32 * kGuideDeltaRows, kStepX = 32 * kGuideInRows;
     floatx4 acc = { 0.f, 0.f, 0.f, 0.f };
     float bs = 0.f;
     // four 32-sample steps per round, their eight loads issued before the
@@ -378,9 +426,8 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_dw(GuideDev G,
 #pragma unroll
         for (uint32_t k = 0; k < kRound; ++k)
         {
-            const size_t s0 = (size_t)(st + k) * 32 + 8 * g;
-            a[k] = *reinterpret_cast<const bf16x8 *>(D + s0);
-            b[k] = *reinterpret_cast<const bf16x8 *>(X + s0);
+            a[k] = *reinterpret_cast<const bf16x8 *>(D + (st + k) * kStepD);
+            b[k] = *reinterpret_cast<const bf16x8 *>(X + (st + k) * kStepX);
         }
 #pragma unroll
         for (uint32_t k = 0; k < kRound; ++k)
@@ -396,9 +443,8 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_dw(GuideDev G,
     }
     for (; st < st1; ++st)
     {
-        const size_t s0 = (size_t)st * 32 + 8 * g;
-        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(D + s0);
-        const bf16x8 b = *reinterpret_cast<const bf16x8 *>(X + s0);
+        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(D + st * kStepD);
+        const bf16x8 b = *reinterpret_cast<const bf16x8 *>(X + st * kStepX);
         acc = mfma16(a, b, acc);
         if (im == 0)
         {
@@ -559,8 +605,7 @@ hipError_t guide_step(const GuideDev &G, const float *samples, const uint32_t *n
         1, std::min<uint32_t>((batch + 63) / 64, 2u * (uint32_t)std::max(1, num_cus)));
     hipLaunchKernelGGL(k_guide_fwdbwd, dim3(g_fb), dim3(kGuideBlock), 0, s, G, samples, n_dev,
                        n_cap, step, batch);
-    const uint32_t items = 72u * kGuideSplits;
-    hipLaunchKernelGGL(k_guide_dw, dim3((items + 3) / 4), dim3(kGuideBlock), 0, s, G, n_dev,
+    hipLaunchKernelGGL(k_guide_dw, dim3(72 * kGuideSplits / (kGuideBlock / 64)), dim3(kGuideBlock), 0, s, G, n_dev,
                        n_cap, step, batch);
     GuideAdam a{};
     if (adam)

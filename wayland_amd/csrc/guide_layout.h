@@ -19,6 +19,9 @@ constexpr int kGuideLobes = 8;
 constexpr int kGuideFwdVecs = 2304; // layers 0-3: 4 tiles x 2 k-blocks x 64 lanes; layer 4: 2 x 2 x 64
 constexpr int kGuideBwdVecs = 1792; // layers 1-3: 4 x 2 x 64; layer 4: 4 x 1 x 64
 constexpr int kGuideBiases = 4 * 64 + 32;
+// staged rows per 16 samples: inputs of layers 0-4, deltas of layers 0-3 and the output
+constexpr int kGuideInRows = 5 * 64;
+constexpr int kGuideDeltaRows = 4 * 64 + 32;
 
 WL_GUIDE_HD constexpr int guide_w_off(int l) { return l * (64 * 64 + 64); }
 WL_GUIDE_HD constexpr int guide_b_off(int l) { return guide_w_off(l) + (l < 4 ? 64 : 32) * 64; }

@@ -18,8 +18,8 @@ struct GuideDev
     void *fwd;       // packed BF16 forward operands (2304 x 16 B)
     void *bwd;       // packed BF16 backward operands (1792 x 16 B)
     float *partials; // kGuideSplits x 18720 gradient partial sums
-    void *xt;        // BF16 layer inputs, feature-major [5][64][cap]
-    void *dt;        // BF16 deltas, feature-major [4 * 64 + 32][cap]
+    void *xt;        // BF16 layer inputs, feature-major [cap / 16][5 * 64][16]
+    void *dt;        // BF16 deltas, feature-major [cap / 16][4 * 64 + 32][16]
     float *loss;     // per-sample loss [cap]
     uint32_t *count; // [0] samples in the training buffer, [1] scratch
     float *train;    // training samples, 16 floats each [train_cap]

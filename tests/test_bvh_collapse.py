@@ -9,8 +9,8 @@ import oracle_bind as ob
 from wayland_amd import scenes
 
 
-def _chain(n, f):
-    rng = np.random.default_rng(1)
+def _chain(n, f, seed=1):
+    rng = np.random.default_rng(seed)
     s = f ** np.arange(n)
     t = rng.uniform(-1, 1, (n, 3, 3)) * 0.4 + np.array([1.0, 0.3, -0.2])
     return np.ascontiguousarray((t * s[:, None, None]).reshape(n, 9), np.float32)
@@ -47,6 +47,16 @@ def test_shrinking_chain_stays_in_the_stack(n, f, depth):
 def test_chain_beyond_the_stack_is_refused():
     with pytest.raises(Exception, match="exceeds the traversal stack"):
         hb.HostBVH8(_chain(400, 0.75))
+
+
+@pytest.mark.parametrize("n,f,seed,depth", [
+    (400, 0.85, 2, 27), (450, 0.87, 2, 32), (600, 0.9, 1, 32), (800, 0.93, 2, 31),
+    (400, 0.9, 1, 22), (500, 0.9, 1, 25), (200, 0.8, 1, 20)])
+def test_greedy_replaces_only_a_deeper_tree(n, f, seed, depth):
+    """Both collapses leave these trees deeper than the short stack, and the
+    greedy one is the deeper of the two (33 to 34 levels in the first four
+    cases, beyond the stack): the tree chosen by cost stays, and is traced."""
+    assert _check(_chain(n, f, seed), _rays(n))["depth"] <= depth
 
 
 @pytest.mark.parametrize("kind", ["points", "one point", "segments", "tiny", "mixed"])

@@ -565,20 +565,31 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
     const uint32_t n2 = b.next_node;
     double sah;
     {
-        // The greedy collapse is kept for trees that the choice makes deeper
-        // than the kernels' short stack: chains of ever smaller triangles, of
-        // which it opens the large near ones first (300 triangles that shrink
-        // by 0.65 each: 39 levels, 24 greedily).
+        // A tree that the choice makes deeper than the kernels' short stack is
+        // also collapsed greedily, and the shallower one is taken: chains of
+        // ever smaller triangles, of which the greedy collapse opens the large
+        // near ones first, come out either way (300 triangles that shrink by
+        // 0.65 each: 39 levels, 24 greedily; 600 that shrink by 0.9: 32, 34
+        // greedily, more than the traversal stack holds).
         std::vector<uint32_t> leaf_of(n2);
         for (uint32_t i = 0; i < n2; ++i)
             leaf_of[i] = b.nodes[i].count;
         const std::vector<Collapse> choice = choose_collapse(b.nodes, n2);
         sah = collapse_bvh8(tris, ntris, b.nodes, b.prims, &choice, out);
-        if (out->depth > WL_BVH8_SHALLOW_DEPTH || out->nodes.size() > kMaxNodes)
+        const bool fits = out->nodes.size() <= kMaxNodes;
+        if (out->depth > WL_BVH8_SHALLOW_DEPTH || !fits)
         {
             for (uint32_t i = 0; i < n2; ++i)
                 b.nodes[i].count = leaf_of[i];
-            sah = collapse_bvh8(tris, ntris, b.nodes, b.prims, nullptr, out);
+            Bvh8Host greedy;
+            const double greedy_sah = collapse_bvh8(tris, ntris, b.nodes, b.prims, nullptr,
+                                                    &greedy);
+            const bool greedy_fits = greedy.nodes.size() <= kMaxNodes;
+            if (greedy_fits != fits ? greedy_fits : greedy.depth < out->depth)
+            {
+                *out = std::move(greedy);
+                sah = greedy_sah;
+            }
         }
     }
     out->sah_cost = sah;

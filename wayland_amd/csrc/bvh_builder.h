@@ -23,9 +23,9 @@ struct Bvh8Host
 // Build over `ntris` world-space triangles (9 floats each, global primitive
 // order).  Binned SAH (32 bins) BVH2 with at most WL_BVH8_MAX_LEAF_TRIS
 // triangles per leaf, collapsed to 8-wide nodes by the SAH cost of every way to
-// do so (greedily where that would be deeper than the short traversal stack),
-// children slot-ordered by octant and boxes quantised to 16
-// bits.  Returns false with *err set on failure (e.g. depth limit).
+// do so (greedily where that is deeper than the short traversal stack and the
+// greedy tree is shallower), children slot-ordered by octant and boxes
+// quantised to 16 bits.  Returns false with *err set on failure (e.g. depth limit).
 bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
                 std::string *err);
 

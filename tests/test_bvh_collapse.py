@@ -86,3 +86,33 @@ def test_counts_around_leaf_and_node_sizes(n):
     tris = (c + rng.uniform(-0.2, 0.2, (n, 3, 3))).astype(np.float32).reshape(n, 9)
     info = _check(np.ascontiguousarray(tris), _rays(n))
     assert info["tris"] == n
+
+
+def _soup(n=5000):
+    rng = np.random.default_rng(11)
+    return rng.uniform(0, 1, (n, 1, 3)) + rng.uniform(-0.02, 0.02, (n, 3, 3))
+
+
+@pytest.mark.parametrize("e", [-74, -70, 62, 66, 84])
+def test_tree_does_not_depend_on_the_units(e):
+    """Areas that would leave the range of a float at either end."""
+    t = _soup().reshape(-1, 9).astype(np.float32)
+    one, other = hb.HostBVH8(t).info(), hb.HostBVH8(t * np.float32(2.0 ** e)).info()
+    assert one == other
+
+
+@pytest.mark.parametrize("soup", [False, True])
+@pytest.mark.parametrize("m", [64, 300, 4096])
+def test_collapsed_triangles_share_wide_nodes(m, soup):
+    """m triangles collapsed into one point: leaves of at most four and nodes of
+    eight take m / 24 nodes, and opening the largest child first m / 10 to m /
+    15.  A ray through the point visits them all."""
+    p = np.array([0.25, 0.5, 0.75])
+    cluster = np.repeat(np.repeat(p[None, None], 3, axis=1), m, axis=0)
+    tris = np.concatenate([_soup(2000), cluster]) if soup else cluster
+    tris = np.ascontiguousarray(tris.reshape(-1, 9), np.float32)
+    rays = _rays(12)
+    rays[:, 4:7] = p.astype(np.float32) - rays[:, 0:3]
+    _check(tris, rays)
+    _, counts, _ = hb.HostBVH8(tris).trace(rays)
+    assert counts[:, 0].mean() <= m / 8 + (25 if soup else 0)

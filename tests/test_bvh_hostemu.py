@@ -1,6 +1,8 @@
 """CPU checks of the library's own BVH8 builder and traversal code (compiled
 for the host from the same traverse_device.h the gfx950 kernels use, with
 every node / triangle / stack index checked against its allocation)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,15 @@ def test_large_scene_depth_and_subsample():
     info = h.info()
     assert info["depth"] <= 32
     assert counts[:, 0].mean() > 1
+
+
+@pytest.mark.parametrize("depth,nodes,tris,variant", [
+    (1, 8, 1, 0), (16, 1 << 25, 89_478_485, 0),       # 4 GB of nodes, just below 4 GB of triangles
+    (16, (1 << 25) + 8, 1, 1), (16, 8, 89_478_486, 1), (10, 1 << 26, 1 << 28, 1),
+    (17, 8, 1, 2), (32, 1 << 27, 1 << 30, 2)])
+def test_traversal_variant(depth, nodes, tris, variant):
+    """Arrays past 4 GB take 64-bit addresses (1) and keep the short stack, which
+    only the depth decides (2: the deep one)."""
+    f = hb.lib().wlh_trav_variant
+    f.restype, f.argtypes = C.c_uint32, [C.c_uint32, C.c_uint64, C.c_uint64]
+    assert f(depth, nodes, tris) == variant

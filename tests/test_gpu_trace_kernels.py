@@ -167,3 +167,49 @@ def test_finished_batches_count_their_rays(gpu_ctx):
              for k in range(4)]
     for key in ("paths", "extension_rays", "shadow_rays"):
         assert big[key] == sum(s[key] for s in small), key
+
+
+def _wide(accel):
+    """The accel's rays take the 64-bit kernels from here on."""
+    import ctypes as C
+    from wayland_amd import _lib
+    f = _lib.load().wl_accel_test_wide
+    f.restype, f.argtypes = C.c_uint32, [C.c_void_p]
+    assert f(accel.h) == 1
+
+
+@pytest.mark.parametrize("name", ["cornell", "ico"])
+def test_wide_addresses_equal_32_bit_offsets(gpu_ctx, name):
+    """The kernels of a shallow BVH past 4 GB, on one that is small: the same
+    hits and films, bit for bit, from the raw traces, a finished batch, a batch
+    of two lanes and a server."""
+    import torch
+    import wayland_amd as wl
+    print(f"case: wide {name}", flush=True)
+    if name == "cornell":
+        sc = scenes.textured_cornell_box(256, 256)  # fewer nodes than the LDS copy holds
+    else:
+        sc = scenes.wavefront_scene(6, 3, width=256, height=256)
+    rays = scenes.traversal_rays(100_003, seed=17)
+    if name == "cornell":
+        rays[:, 0:3] = rays[:, 0:3] * 2 - np.float32([1, 0, 1])
+
+    def results(wide):
+        accel = wl.Accel(gpu_ctx, sc)
+        if wide:
+            _wide(accel)
+        pt = wl.PathTracer(gpu_ctx, accel, sc)
+        h, occ = _hits(accel, rays)
+        out = [h[k].view(np.uint32) for k in ("t", "prim", "b1", "b2")] + [occ]
+        for spp in (2, 72):  # 131,072 and 4,718,592 paths
+            film, _ = pt.render(wl.pt_config(256, 256, spp=spp, max_depth=6), stats=False)
+            out.append(film.view(torch.int32).cpu().numpy())
+        server = wl.Server(gpu_ctx, batch_paths=1 << 20)
+        films = [torch.zeros((256 * 256, 6), device="cuda") for _ in range(2)]
+        server.render([dict(pt=pt, width=256, height=256, spp=2, frame_offset=8 * k, film=f)
+                       for k, f in enumerate(films)])
+        torch.cuda.synchronize()
+        return out + [f.view(torch.int32).cpu().numpy() for f in films]
+
+    for a, b in zip(results(False), results(True)):
+        assert np.array_equal(a, b)

@@ -70,9 +70,21 @@ struct alignas(16) WlTriRecord
 static_assert(sizeof(WlBvh8Node) == 128, "BVH8 node must be 128 bytes");
 static_assert(sizeof(WlTriRecord) == 48, "triangle record must be 48 bytes");
 
-// Whether byte offsets of 32 bits reach every node and triangle record: the
-// traversal kernels then address them from a uniform base.
-static inline bool wl_bvh8_narrow(uint64_t nodes, uint64_t tris)
+// The traversal kernels' variants: the short stack (with it the wavefronts and,
+// in single-BVH launches, the top levels in LDS) wherever the tree is shallow,
+// and byte offsets of 32 bits from a uniform base where they reach every node
+// and triangle record; a BVH whose arrays pass 4 GB (89M triangles or 33M node
+// slots) takes 64-bit addresses.  Deep trees, which are rare, share one variant.
+enum
 {
-    return nodes * sizeof(WlBvh8Node) <= (1ull << 32) && tris * sizeof(WlTriRecord) < (1ull << 32);
+    WL_TRAV_SHORT = 0,      // WL_BVH8_SHALLOW_DEPTH entries, 32-bit offsets
+    WL_TRAV_SHORT_WIDE = 1, // WL_BVH8_SHALLOW_DEPTH entries, 64-bit addresses
+    WL_TRAV_DEEP = 2        // WL_BVH8_STACK_DEPTH entries, 64-bit addresses
+};
+static inline uint32_t wl_bvh8_variant(uint32_t depth, uint64_t nodes, uint64_t tris)
+{
+    const bool narrow = nodes * sizeof(WlBvh8Node) <= (1ull << 32) &&
+                        tris * sizeof(WlTriRecord) < (1ull << 32);
+    return depth > WL_BVH8_SHALLOW_DEPTH ? WL_TRAV_DEEP
+                                         : (narrow ? WL_TRAV_SHORT : WL_TRAV_SHORT_WIDE);
 }

@@ -245,6 +245,12 @@ uint64_t wlh_serve_check(const uint32_t *req4, uint32_t n, uint32_t capacity, ui
     return bad;
 }
 
+// The traversal variant of a BVH (bvh8.h).
+uint32_t wlh_trav_variant(uint32_t depth, uint64_t nodes, uint64_t tris)
+{
+    return wl_bvh8_variant(depth, nodes, tris);
+}
+
 // Entries of a queue segment of a batch of n paths (wl_pt.h).
 uint32_t wlh_pt_segment(uint64_t n) { return wl::pt_segment(n); }
 

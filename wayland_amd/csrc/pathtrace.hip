@@ -232,7 +232,7 @@ __device__ __forceinline__ auto first_chunks(uint32_t n)
 // The first bounce of a single-scene batch: queue entry i is path i, and its
 // camera ray is computed here (the same camera_ray as the shade pass uses),
 // not read from a ray queue: nothing is written before the first traversal.
-template <int STACK>
+template <int STACK, bool WIDE>
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(5)))
 void k_trace_first(PtParams P, PtScene S, PtBuffers B)
 {
@@ -243,7 +243,7 @@ void k_trace_first(PtParams P, PtScene S, PtBuffers B)
     if (blockIdx.x == 0 && threadIdx.x == 0)
         B.stats[0] += count;
     auto range = first_chunks(count);
-    trav_persistent<kClosest, kPtBlock, STACK != 16, pt_top_nodes<STACK, false>() != 0>(
+    trav_persistent<kClosest, kPtBlock, WIDE, pt_top_nodes<STACK, false>() != 0>(
         S.nodes, S.tris, stack,
         XcdChunks<kPtBlock, decltype(range)>(range, queue_chunks(B, blockIdx.x % 8u), 0u),
         [&](uint32_t i, TravRay &r, uint32_t &) {
@@ -330,7 +330,7 @@ __device__ __forceinline__ void queue_emit(const PtBuffers &B, uint32_t i, const
 // 1.35 -> 0.87 ms, 1080p x 64 spp 40.2 -> 36.0 ms, 64 serving requests 393 (at
 // equal ranges before any of this) -> 309 ms.
 // first: the multi-request raygen's queue (all rays, no shadow rays).
-template <int STACK, bool MULTI>
+template <int STACK, bool WIDE, bool MULTI>
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(STACK == 16 ? 6 : 5)))
 void k_trace(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs, float eps,
              int first)
@@ -368,7 +368,7 @@ void k_trace(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs,
         next = lo + (uint32_t)(s0 < n ? s0 : n);
         end = lo + (uint32_t)(s0 + chunk < n ? s0 + chunk : n);
     };
-    trav_persistent<kMixed, kPtBlock, STACK != 16, pt_top_nodes<STACK, MULTI>() != 0>(
+    trav_persistent<kMixed, kPtBlock, WIDE, pt_top_nodes<STACK, MULTI>() != 0>(
         S.nodes, S.tris, stack, XcdChunks<kPtBlock, decltype(range)>(range, queue_chunks(B, x), 0u),
         [&](uint32_t i, TravRay &r, uint32_t &root) {
             queue_fetch<MULTI>(B, parity, reqs, eps, shadow, i, r, root);
@@ -1116,7 +1116,7 @@ void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__re
 constexpr uint32_t kLaunchedBounces = 2;
 constexpr uint32_t kMaxSlice = 4096;
 
-template <int STACK, bool GTRAIN, bool MULTI>
+template <int STACK, bool WIDE, bool GTRAIN, bool MULTI>
 __global__ __launch_bounds__(kPtBlock) __attribute__((amdgpu_waves_per_eu(4)))
 void k_finish(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__restrict__ reqs)
 {
@@ -1167,7 +1167,7 @@ void k_finish(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__r
             shadows += nshadow;
             const uint32_t ray_chunks = (nrays + 63u) / 64u;
             bool shadow = false; // the kind of the wave's current chunk
-            trav_persistent<kMixed, kPtBlock, STACK != 16, pt_top_nodes<STACK, MULTI>() != 0>(
+            trav_persistent<kMixed, kPtBlock, WIDE, pt_top_nodes<STACK, MULTI>() != 0>(
                 S0.nodes, S0.tris, stack,
                 [&](bool, uint32_t &next, uint32_t &end) {
                     uint32_t c = 0;
@@ -1477,21 +1477,18 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B0
 {
     const uint32_t npaths = P.npix * P.nsamples;
     const uint32_t blocks_all = (npaths + kPtBlock - 1) / kPtBlock;
-    // a BVH at most 16 deep needs at most 15 stack entries per lane; those
-    // kernels also address nodes and triangles with 32-bit offsets
-    const bool shallow = S.bvh_depth <= WL_BVH8_SHALLOW_DEPTH && wl_bvh8_narrow(S.num_nodes, S.num_tris);
     // persistent traversal grids: the workgroups that fit the GPU at once.  All
     // grids are multiples of 8 (each XCD its share).
-    static int occ16 = 0, occ32 = 0, occf16 = 0, occf32 = 0;
-    if (!occ16)
-    {
-        occf16 = blocks_per_cu(k_trace_first<16>);
-        occf32 = blocks_per_cu(k_trace_first<WL_BVH8_STACK_DEPTH>);
-        occ32 = blocks_per_cu(k_trace<WL_BVH8_STACK_DEPTH, false>);
-        occ16 = blocks_per_cu(k_trace<16, false>);
-    }
-    const uint32_t g_trav = grid8(4 * blocks_all, num_cus, shallow ? occ16 : occ32);
-    const uint32_t g_first = grid8(4 * blocks_all, num_cus, shallow ? occf16 : occf32);
+    static int occ[3] = {}, occ_first[3] = {}; // per traversal variant
+    const uint32_t trav = S.trav_variant;
+    if (!occ[trav])
+        with_variant(trav, [&](auto v) {
+            using V = decltype(v);
+            occ_first[trav] = blocks_per_cu(k_trace_first<V::STACK, V::WIDE>);
+            occ[trav] = blocks_per_cu(k_trace<V::STACK, V::WIDE, false>);
+        });
+    const uint32_t g_trav = grid8(4 * blocks_all, num_cus, occ[trav]);
+    const uint32_t g_first = grid8(4 * blocks_all, num_cus, occ_first[trav]);
     const uint32_t g_shade = grid8(blocks_all, num_cus, 8);
     const uint32_t g_sort = grid8(blocks_all, num_cus, 4);
     // guide inference: up to 4 workgroups per CU
@@ -1499,19 +1496,18 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B0
     PtBuffers B = B0;
     B.segcap = pt_segment(npaths);
     auto trace = [&](int parity) {
-        if (shallow)
-            hipLaunchKernelGGL((k_trace<16, false>), dim3(g_trav), dim3(kPtBlock), 0, st, S, B,
-                               parity, nullptr, P.epsilon, 0);
-        else
-            hipLaunchKernelGGL((k_trace<WL_BVH8_STACK_DEPTH, false>), dim3(g_trav),
-                               dim3(kPtBlock), 0, st, S, B, parity, nullptr, P.epsilon, 0);
+        with_variant(trav, [&](auto v) {
+            using V = decltype(v);
+            hipLaunchKernelGGL((k_trace<V::STACK, V::WIDE, false>), dim3(g_trav), dim3(kPtBlock),
+                               0, st, S, B, parity, nullptr, P.epsilon, 0);
+        });
     };
     hipLaunchKernelGGL(k_batch_start, dim3(1), dim3(kPtBlock), 0, st, P, B);
-    if (shallow)
-        hipLaunchKernelGGL((k_trace_first<16>), dim3(g_first), dim3(kPtBlock), 0, st, P, S, B);
-    else
-        hipLaunchKernelGGL((k_trace_first<WL_BVH8_STACK_DEPTH>), dim3(g_first), dim3(kPtBlock), 0,
+    with_variant(trav, [&](auto v) {
+        using V = decltype(v);
+        hipLaunchKernelGGL((k_trace_first<V::STACK, V::WIDE>), dim3(g_first), dim3(kPtBlock), 0,
                            st, P, S, B);
+    });
     // the guide's inference and the per-vertex trace belong to the launched bounces
     const bool finish = alone && npaths < kFinishMaxPaths &&
                         P.max_depth > kLaunchedBounces + 1 && !B.trace &&
@@ -1560,24 +1556,27 @@ hipError_t pt_run_batch(const PtParams &P, const PtScene &S, const PtBuffers &B0
     if (finish)
     {
         const bool gtrain = (P.gmode & 2u) != 0;
-        const auto kernel = shallow ? (gtrain ? k_finish<16, true, false> : k_finish<16, false, false>)
-                                    : (gtrain ? k_finish<WL_BVH8_STACK_DEPTH, true, false>
-                                              : k_finish<WL_BVH8_STACK_DEPTH, false, false>);
-        hipLaunchKernelGGL(kernel, dim3(grid8(4 * blocks_all, num_cus, 4)), dim3(kPtBlock), 0, st,
-                           P, S, B, (int)(kLaunchedBounces & 1u), nullptr);
+        with_variant(trav, [&](auto v) {
+            using V = decltype(v);
+            hipLaunchKernelGGL((gtrain ? k_finish<V::STACK, V::WIDE, true, false>
+                                       : k_finish<V::STACK, V::WIDE, false, false>),
+                               dim3(grid8(4 * blocks_all, num_cus, 4)), dim3(kPtBlock), 0, st, P,
+                               S, B, (int)(kLaunchedBounces & 1u), nullptr);
+        });
     }
     return hipGetLastError();
 }
 
-static int g_multi_occ16 = 0, g_multi_occ32 = 0;
+static int g_multi_occ[3] = {}; // per traversal variant
 
 void pt_multi_init()
 {
-    if (!g_multi_occ16)
-    {
-        g_multi_occ32 = blocks_per_cu(k_trace<WL_BVH8_STACK_DEPTH, true>);
-        g_multi_occ16 = blocks_per_cu(k_trace<16, true>);
-    }
+    for (uint32_t trav = 3; trav-- > 0;)
+        if (!g_multi_occ[trav])
+            with_variant(trav, [&](auto v) {
+                using V = decltype(v);
+                g_multi_occ[trav] = blocks_per_cu(k_trace<V::STACK, V::WIDE, true>);
+            });
 }
 
 hipError_t pt_clock_stamp(unsigned long long *dst, hipStream_t st)
@@ -1591,8 +1590,7 @@ hipError_t pt_run_multi(const PtMultiLaunch &L, const PtBuffers &B0, int num_cus
     pt_multi_init();
     const uint32_t blocks_all = (L.capacity + kPtBlock - 1) / kPtBlock;
     const uint32_t g_gen = grid8(blocks_all, num_cus, 8);
-    const uint32_t g_trav =
-        grid8(4 * blocks_all, num_cus, L.stack16 ? g_multi_occ16 : g_multi_occ32);
+    const uint32_t g_trav = grid8(4 * blocks_all, num_cus, g_multi_occ[L.trav_variant]);
     const uint32_t g_shade =
         grid8(blocks_all, num_cus, (int)std::max<uint32_t>(1, L.shade_blocks_per_cu));
     const PtParams P0{};
@@ -1603,12 +1601,11 @@ hipError_t pt_run_multi(const PtMultiLaunch &L, const PtBuffers &B0, int num_cus
     PtBuffers B = B0;
     B.segcap = pt_segment(L.capacity);
     auto trace = [&](int parity, int first) {
-        if (L.stack16)
-            hipLaunchKernelGGL((k_trace<16, true>), dim3(g_trav), dim3(kPtBlock), 0, st, SA, B,
-                               parity, L.reqs, 0.0f, first);
-        else
-            hipLaunchKernelGGL((k_trace<WL_BVH8_STACK_DEPTH, true>), dim3(g_trav),
-                               dim3(kPtBlock), 0, st, SA, B, parity, L.reqs, 0.0f, first);
+        with_variant(L.trav_variant, [&](auto v) {
+            using V = decltype(v);
+            hipLaunchKernelGGL((k_trace<V::STACK, V::WIDE, true>), dim3(g_trav), dim3(kPtBlock), 0,
+                               st, SA, B, parity, L.reqs, 0.0f, first);
+        });
     };
     hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(kPtBlock), 0, st, L, B);
     hipLaunchKernelGGL(k_raygen_multi, dim3(g_gen), dim3(kPtBlock), 0, st, L, B);
@@ -1623,10 +1620,12 @@ hipError_t pt_run_multi(const PtMultiLaunch &L, const PtBuffers &B0, int num_cus
         trace(parity ^ 1, 0);
     }
     if (finish)
-        hipLaunchKernelGGL((L.stack16 ? k_finish<16, false, true>
-                                      : k_finish<WL_BVH8_STACK_DEPTH, false, true>),
-                           dim3(grid8(4 * blocks_all, num_cus, 4)), dim3(kPtBlock), 0, st, P0, SA,
-                           B, (int)(kLaunchedBounces & 1u), L.reqs);
+        with_variant(L.trav_variant, [&](auto v) {
+            using V = decltype(v);
+            hipLaunchKernelGGL((k_finish<V::STACK, V::WIDE, false, true>),
+                               dim3(grid8(4 * blocks_all, num_cus, 4)), dim3(kPtBlock), 0, st, P0,
+                               SA, B, (int)(kLaunchedBounces & 1u), L.reqs);
+        });
     hipLaunchKernelGGL(k_accumulate_multi, dim3(g_gen), dim3(kPtBlock), 0, st, L, B);
     hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, st, L);
     return hipGetLastError();

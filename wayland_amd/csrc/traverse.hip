@@ -69,7 +69,7 @@ __device__ __forceinline__ auto eighth_chunks(uint32_t n, uint32_t chunk)
 // ntop: nodes copied to LDS, min(node count, top_nodes<STACK>()); sched /
 // base: the launching stream's chunk counters and their values at launch.
 // The grid is a multiple of 8.
-template <int STACK>
+template <int STACK, bool WIDE>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6, 8)))
 void k_trace_closest_p(
     const WlBvh8Node *__restrict__ nodes, const WlTriRecord *__restrict__ tris,
@@ -81,7 +81,7 @@ void k_trace_closest_p(
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
     auto range = eighth_chunks(n, base.chunk);
-    trav_persistent<kClosest, kTraceBlock, STACK != 16, top_nodes<STACK>() != 0>(
+    trav_persistent<kClosest, kTraceBlock, WIDE, top_nodes<STACK>() != 0>(
         nodes, tris, stack,
         XcdChunks<kTraceBlock, decltype(range)>(range, sched + kSchedStride * (blockIdx.x % 8u),
                                                 base.base[blockIdx.x % 8u]),
@@ -90,7 +90,7 @@ void k_trace_closest_p(
         reinterpret_cast<const WlBvh8Node *>(top), top_nodes<STACK>() ? ntop : 0u);
 }
 
-template <int STACK>
+template <int STACK, bool WIDE>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(7, 8)))
 void k_trace_any_p(const WlBvh8Node *__restrict__ nodes, const WlTriRecord *__restrict__ tris,
                    const wl_ray *__restrict__ rays, uint32_t n, uint32_t *__restrict__ bits,
@@ -101,7 +101,7 @@ void k_trace_any_p(const WlBvh8Node *__restrict__ nodes, const WlTriRecord *__re
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
     auto range = eighth_chunks(n, base.chunk);
-    trav_persistent<kAny, kTraceBlock, STACK != 16, top_nodes<STACK>() != 0>(
+    trav_persistent<kAny, kTraceBlock, WIDE, top_nodes<STACK>() != 0>(
         nodes, tris, stack,
         XcdChunks<kTraceBlock, decltype(range)>(range, sched + kSchedStride * (blockIdx.x % 8u),
                                                 base.base[blockIdx.x % 8u]),
@@ -148,16 +148,10 @@ __global__ void k_zero_words(uint32_t *words, uint32_t nwords)
         words[k] = 0;
 }
 
-// The 16-entry stack kernels: also 32-bit node and triangle offsets.
-static inline bool shallow(const wl_accel_s *a)
-{
-    return a->info.depth <= WL_BVH8_SHALLOW_DEPTH && wl_bvh8_narrow(a->num_nodes, a->num_tri_records);
-}
-
 // Persistent grid: the workgroups that fit the GPU at once (the launch then
 // takes at most one workgroup per 256 rays).
 template <class K>
-static uint32_t persistent_grid(K kernel, uint32_t /*unused*/, int num_cus)
+static uint32_t persistent_grid(K kernel, int num_cus)
 {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kTraceBlock, 0) !=
@@ -198,7 +192,7 @@ static uint32_t xcd_grid(uint32_t grid_cache, uint32_t n, uint32_t chunk)
     return (g + 7u) & ~7u;
 }
 
-template <int STACK>
+template <class V>
 static hipError_t closest_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t n,
                                wl_hit *hits, hipStream_t s)
 {
@@ -206,7 +200,7 @@ static hipError_t closest_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t
     static int cus_cache = -1;
     if (cus_cache != a->ctx->num_cus)
     {
-        grid_cache = persistent_grid(k_trace_closest_p<STACK>, 0xFFFFFFFFu, a->ctx->num_cus);
+        grid_cache = persistent_grid(k_trace_closest_p<V::STACK, V::WIDE>, a->ctx->num_cus);
         cus_cache = a->ctx->num_cus;
     }
     const uint32_t chunk = trace_chunk(n, grid_cache);
@@ -217,13 +211,13 @@ static hipError_t closest_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t
     if (e != hipSuccess)
         return e;
     const TraceSched base = take_bases(sb, n, chunk);
-    hipLaunchKernelGGL(k_trace_closest_p<STACK>, dim3(grid), dim3(kTraceBlock), 0, s,
+    hipLaunchKernelGGL((k_trace_closest_p<V::STACK, V::WIDE>), dim3(grid), dim3(kTraceBlock), 0, s,
                        a->d_nodes, a->d_tris, rays, n, hits,
-                       std::min<uint32_t>(a->num_nodes, top_nodes<STACK>()), sb->dev, base);
+                       std::min<uint32_t>(a->num_nodes, top_nodes<V::STACK>()), sb->dev, base);
     return hipGetLastError();
 }
 
-template <int STACK>
+template <class V>
 static hipError_t any_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t n,
                            uint32_t *bits, hipStream_t s)
 {
@@ -231,7 +225,7 @@ static hipError_t any_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t n,
     static int cus_cache = -1;
     if (cus_cache != a->ctx->num_cus)
     {
-        grid_cache = persistent_grid(k_trace_any_p<STACK>, 0xFFFFFFFFu, a->ctx->num_cus);
+        grid_cache = persistent_grid(k_trace_any_p<V::STACK, V::WIDE>, a->ctx->num_cus);
         cus_cache = a->ctx->num_cus;
     }
     const uint32_t chunk = trace_chunk(n, grid_cache);
@@ -245,9 +239,9 @@ static hipError_t any_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t n,
     const uint32_t words = (n + 31) / 32;
     hipLaunchKernelGGL(k_zero_words, dim3(std::min<uint32_t>((words + 255) / 256, 4096)),
                        dim3(256), 0, s, bits, words);
-    hipLaunchKernelGGL(k_trace_any_p<STACK>, dim3(grid), dim3(kTraceBlock), 0, s, a->d_nodes,
+    hipLaunchKernelGGL((k_trace_any_p<V::STACK, V::WIDE>), dim3(grid), dim3(kTraceBlock), 0, s, a->d_nodes,
                        a->d_tris, rays, n, bits,
-                       std::min<uint32_t>(a->num_nodes, top_nodes<STACK>()), sb->dev, base);
+                       std::min<uint32_t>(a->num_nodes, top_nodes<V::STACK>()), sb->dev, base);
     return hipGetLastError();
 }
 
@@ -257,20 +251,20 @@ hipError_t launch_trace_closest(const wl_accel_s *a, const wl_ray *rays,
 {
     if (n == 0)
         return hipSuccess;
-    const bool sh = shallow(a);
     if (counts)
     {
         dim3 grid((n + kTraceBlock - 1) / kTraceBlock), block(kTraceBlock);
-        if (sh)
-            hipLaunchKernelGGL(k_trace_closest_counted<16>, grid, block, 0, s, a->d_nodes,
-                               a->d_tris, rays, n, hits, counts);
-        else
+        if (a->trav_variant == WL_TRAV_DEEP)
             hipLaunchKernelGGL(k_trace_closest_counted<WL_BVH8_STACK_DEPTH>, grid, block, 0, s,
+                               a->d_nodes, a->d_tris, rays, n, hits, counts);
+        else
+            hipLaunchKernelGGL(k_trace_closest_counted<WL_BVH8_SHALLOW_DEPTH>, grid, block, 0, s,
                                a->d_nodes, a->d_tris, rays, n, hits, counts);
         return hipGetLastError();
     }
-    return sh ? closest_impl<16>(a, rays, n, hits, s)
-              : closest_impl<WL_BVH8_STACK_DEPTH>(a, rays, n, hits, s);
+    return with_variant(a->trav_variant, [&](auto v) {
+        return closest_impl<decltype(v)>(a, rays, n, hits, s);
+    });
 }
 
 hipError_t launch_trace_any(const wl_accel_s *a, const wl_ray *rays,
@@ -278,8 +272,8 @@ hipError_t launch_trace_any(const wl_accel_s *a, const wl_ray *rays,
 {
     if (n == 0)
         return hipSuccess;
-    return shallow(a) ? any_impl<16>(a, rays, n, bits, s)
-                      : any_impl<WL_BVH8_STACK_DEPTH>(a, rays, n, bits, s);
+    return with_variant(a->trav_variant,
+                        [&](auto v) { return any_impl<decltype(v)>(a, rays, n, bits, s); });
 }
 
 } // namespace wl

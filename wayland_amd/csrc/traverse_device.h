@@ -229,9 +229,9 @@ struct NodeHits
 };
 
 // TOP: nodes [0, ntop) are also held in LDS at `top`, read there instead of
-// from memory (the builder lays the top levels out first).  WIDE: 64-bit
-// addresses per lane; otherwise a byte offset of 32 bits from the uniform base
-// (wl_bvh8_narrow), which the LDS path shares.
+// from memory (the builder lays the top levels out first) with byte offsets of
+// 32 bits.  WIDE: 64-bit addresses per lane for the rest; otherwise the same
+// offsets from the uniform base (wl_bvh8_variant).
 template <bool TOP, bool WIDE>
 WL_HD NodeHits node_visit(const WlBvh8Node *__restrict__ nodes, uint32_t node,
                           const TravRay &r, float t_best, const WlBvh8Node *top = nullptr,
@@ -240,7 +240,8 @@ WL_HD NodeHits node_visit(const WlBvh8Node *__restrict__ nodes, uint32_t node,
     // near/far quantised planes chosen by the ray's direction signs: the lo and
     // hi planes of an axis are a 16-byte aligned pair, so a per-lane bit of the
     // address picks one and its complement the other
-    const uint32_t at = WIDE ? 0u : node << 7;
+    const bool in_top = TOP && node < ntop;
+    const uint32_t at = WIDE && !in_top ? 0u : node << 7;
     const uint32_t nx = at | (r.code & 16u), ny = at | ((r.code >> 1) & 16u),
                    nz = at | ((r.code >> 2) & 16u);
     uint4 h0, h1, nqx, fqx, nqy, fqy, nqz, fqz;
@@ -264,14 +265,13 @@ WL_HD NodeHits node_visit(const WlBvh8Node *__restrict__ nodes, uint32_t node,
     typedef __attribute__((address_space(1))) const char glb_c;
     auto as_lds = [](lds_c *p) { return (lds_u4 *)p; };
     auto as_glb = [](glb_c *p) { return (glb_u4 *)p; };
-    static_assert(!(TOP && WIDE), "the LDS copy is read with 32-bit offsets");
-    if (TOP && node < ntop)
+    if (in_top)
         fetch((lds_c *)reinterpret_cast<const char *>(top), as_lds);
     else
         fetch((glb_c *)reinterpret_cast<const char *>(WIDE ? nodes + node : nodes), as_glb);
 #else
     auto as_any = [](const char *p) { return reinterpret_cast<const uint4 *>(p); };
-    fetch(reinterpret_cast<const char *>(WIDE ? nodes + node : nodes), as_any);
+    fetch(reinterpret_cast<const char *>(in_top ? top : WIDE ? nodes + node : nodes), as_any);
 #endif
     const float px = wl_u2f(h0.x), py = wl_u2f(h0.y), pz = wl_u2f(h0.z);
     const uint32_t ew = h0.w;

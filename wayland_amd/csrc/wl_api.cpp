@@ -344,6 +344,7 @@ wl_status wl_accel_build_triangles(wl_context ctx, const wl_tri_input *inputs,
     a->num_nodes = (uint32_t)host.nodes.size();
     a->num_tris = total;
     a->num_tri_records = (uint32_t)host.tris.size();
+    a->trav_variant = wl_bvh8_variant(host.depth, host.nodes.size(), host.tris.size());
     a->h_tris = std::move(tris);
     wl_accel_info &inf = a->info;
     inf.num_triangles = total;
@@ -359,6 +360,14 @@ wl_status wl_accel_build_triangles(wl_context ctx, const wl_tri_input *inputs,
     wl::ctx_retain(ctx);
     *out = a;
     return WL_SUCCESS;
+}
+
+// For the tests, and not in the header: lets this BVH's rays take the 64-bit
+// addresses of one whose arrays pass 4 GB.  Returns its WL_TRAV_* variant.
+uint32_t wl_accel_test_wide(wl_accel a)
+{
+    a->trav_variant = std::max<uint32_t>(a->trav_variant, WL_TRAV_SHORT_WIDE);
+    return a->trav_variant;
 }
 
 wl_status wl_accel_destroy(wl_accel a)

@@ -58,6 +58,7 @@ struct wl_accel_s
     uint32_t num_nodes = 0;
     uint64_t num_tris = 0;
     uint32_t num_tri_records = 0; // entries of d_tris (leaf triangle records)
+    uint32_t trav_variant = 0;    // WL_TRAV_*: the kernels that its rays take
     std::vector<uint32_t> input_offsets;
     std::vector<uint32_t> input_tri_counts;
     std::vector<uint32_t> input_num_vertices;

@@ -54,9 +54,8 @@ struct PtScene
     const float *uvs;           // 8 floats per primitive: uv of v0, v1, v2, pad
     const PtTexture *textures;
     const uint32_t *texels;
-    uint32_t bvh_depth;
+    uint32_t trav_variant; // WL_TRAV_*
     uint32_t num_nodes; // BVH8 nodes (the top ones are copied to LDS by traversal)
-    uint32_t num_tris;  // triangle records
 };
 
 // One batch = pixels [pix0, pix0 + npix) x samples [frame0, frame0 + nsamples)
@@ -187,7 +186,7 @@ struct PtMultiLaunch
     const WlBvh8Node *nodes;
     const WlTriRecord *tris;
     uint32_t max_depth;  // bounces enqueued (maximum over the requests)
-    uint32_t stack16;    // every BVH at most 16 levels deep, the arena within 32-bit offsets
+    uint32_t trav_variant; // WL_TRAV_* of the deepest BVH and the whole arena
     uint32_t capacity;   // paths the buffers hold
     uint32_t finish;     // the megabatches are small: their last bounces in one kernel
     uint32_t shade_blocks_per_cu;

@@ -72,9 +72,8 @@ PtScene pt_scene_view(wl_scene s)
     S.uvs = s->d_uvs;
     S.textures = (const PtTexture *)s->d_textures;
     S.texels = s->d_texels;
-    S.bvh_depth = s->accel->info.depth;
+    S.trav_variant = s->accel->trav_variant;
     S.num_nodes = s->accel->num_nodes;
-    S.num_tris = s->accel->num_tri_records;
     return S;
 }
 

@@ -251,7 +251,7 @@ wl_status run_lane(wl_server s, const wl_serve_config &cfg, const wl_render_requ
 {
     wl_status st = WL_SUCCESS;
     std::vector<wl::PtReq> hreq(n);
-    uint32_t max_npix = 0, max_depth = 0, max_bvh = 0;
+    uint32_t max_npix = 0, max_depth = 0, max_bvh = 0, max_trav = 0;
     for (uint32_t k = 0; k < n; ++k)
     {
         const wl_render_request &r = reqs[k];
@@ -271,6 +271,7 @@ wl_status run_lane(wl_server s, const wl_serve_config &cfg, const wl_render_requ
         max_npix = std::max(max_npix, r.width * r.height);
         max_depth = std::max(max_depth, r.max_depth);
         max_bvh = std::max(max_bvh, r.scene->accel->info.depth);
+        max_trav = std::max(max_trav, r.scene->accel->trav_variant);
     }
     // traversal arena: each distinct BVH once, its child and triangle indices
     // rebased, so the multi-request traversal starts a ray at its request's
@@ -341,7 +342,7 @@ wl_status run_lane(wl_server s, const wl_serve_config &cfg, const wl_render_requ
     L.nodes = s->d_arena_nodes;
     L.tris = s->d_arena_tris;
     L.max_depth = max_depth;
-    L.stack16 = max_bvh <= 16 && wl_bvh8_narrow(arena_nodes, arena_tris) ? 1u : 0u;
+    L.trav_variant = std::max(max_trav, wl_bvh8_variant(max_bvh, arena_nodes, arena_tris));
     L.capacity = s->capacity;
     uint64_t largest = 0; // megabatch, in paths
     for (const wl::PtBatchHeader &h : pl.batches)
@@ -373,7 +374,7 @@ wl_status run_lane(wl_server s, const wl_serve_config &cfg, const wl_render_requ
     {
         std::vector<uint64_t> key = {
             max_depth,
-            L.stack16,
+            L.trav_variant,
             L.finish,
             cfg.shade_blocks_per_cu,
             s->capacity,

@@ -31,10 +31,18 @@ def lib():
                                 C.c_void_p, C.c_int]
         L.wlh_serve_check.restype = C.c_uint64
         L.wlh_serve_check.argtypes = [C.c_void_p, C.c_uint32, C.c_uint32, C.c_void_p]
-        L.wlh_dyn_chunks.restype = C.c_uint32
-        L.wlh_dyn_chunks.argtypes = [C.c_uint32, C.c_uint32, C.c_uint32]
+        L.wlh_eighth_count.restype = C.c_uint32
+        L.wlh_eighth_count.argtypes = [C.c_uint32] * 3
         _lib = L
     return _lib
+
+
+def chunk(kind, *args):
+    """A chunk or block of the kernels' index arithmetic, wlh_<kind>(args):
+    (begin, end), and for a segment's chunk whether its rays are shadow rays."""
+    out = (C.c_uint32 * 3)()
+    getattr(lib(), "wlh_" + kind)(*map(C.c_uint32, args), out)
+    return (out[0], out[1], bool(out[2])) if kind == "segment_chunk" else (out[0], out[1])
 
 
 class HostBVH8:

@@ -1,7 +1,7 @@
-"""The path tracer's queue segments and traversal chunks, walked on the CPU as
-the kernels walk them (pathtrace.hip: queue_walk, first_chunks, k_trace's
-chunks): every entry is taken once, and no segment gets more entries than it
-holds."""
+"""The path tracer's queue segments and traversal chunks, walked on the CPU with
+the kernels' own index arithmetic (traverse_device.h: QueueWalk, DealtChunks,
+SegmentChunks): every entry is taken once, and no segment gets more entries
+than it holds."""
 import ctypes as C
 
 import numpy as np
@@ -23,14 +23,18 @@ SIZES = (1, 63, 64, 65, 255, 256, 257, 2047, 2048, 2049, 4095, 12345, 65537, (1 
 
 @pytest.mark.parametrize("n", SIZES)
 def test_first_queue_is_walked_once_and_fits_the_segments(n):
-    """Blocks of 256 entries dealt to the XCDs in turn: each appends at most
-    one entry per entry it walks to its XCD's segment."""
+    """Each XCD appends at most one entry per entry it walks to its segment."""
     seen = np.zeros(n, np.int32)
     for x in range(8):
-        walked = 0
-        for at in range(x * BLOCK, n, 8 * BLOCK):
-            seen[at:at + BLOCK] += 1
-            walked += min(BLOCK, n - at)
+        walked, k = 0, 0
+        while True:
+            lo, hi = hb.chunk("dealt_block", n, x, k)
+            if lo >= hi:
+                break
+            assert hi - lo <= BLOCK
+            seen[lo:hi] += 1
+            walked += hi - lo
+            k += 1
         assert walked <= segment(n), (n, x)
     assert (seen == 1).all()
     # later queues: an XCD walks its own segment only, so it appends at most
@@ -44,32 +48,29 @@ def test_first_trace_chunks(n, chunk):
     seen = np.zeros(n, np.int32)
     per = BLOCK // chunk
     for x in range(8):
-        c, empty = 0, False
-        while c < n // chunk + 16:
-            s0 = ((c // per) * 8 + x) * BLOCK + (c % per) * chunk
-            lo, hi = min(s0, n), min(s0 + chunk, n)
+        empty = False
+        for c in range(n // chunk // 8 + 2 * per + 3):
+            lo, hi = hb.chunk("dealt_chunk", n, x, chunk, c)
             # the schedule stops at the first empty chunk: none may follow it
-            assert not (empty and lo < hi)
+            assert lo <= hi <= n and not (empty and lo < hi)
             empty = empty or lo >= hi
             seen[lo:hi] += 1
-            c += 1
+        assert empty
     assert (seen == 1).all()
 
 
+@pytest.mark.parametrize("lo", [0, 77 * 256])
 @pytest.mark.parametrize("chunk", [64, 128])
 @pytest.mark.parametrize("nrays,nshadow", [(0, 0), (0, 1), (1, 0), (64, 64), (65, 127), (1000, 0),
-                                           (0, 1000), (777, 888)])
-def test_ray_chunks_then_shadow_chunks(nrays, nshadow, chunk):
+                                           (0, 1000), (777, 888), (4096, 4096)])
+def test_ray_chunks_then_shadow_chunks(nrays, nshadow, chunk, lo):
     rays, shadow = np.zeros(nrays, np.int32), np.zeros(nshadow, np.int32)
-    ray_chunks = (nrays + chunk - 1) // chunk
-    total = ray_chunks + (nshadow + chunk - 1) // chunk
+    total = (nrays + chunk - 1) // chunk + (nshadow + chunk - 1) // chunk
     for c in range(total + 3):
-        is_shadow = c >= ray_chunks
-        n = nshadow if is_shadow else nrays
-        s0 = (c - ray_chunks if is_shadow else c) * chunk
-        lo, hi = min(s0, n), min(s0 + chunk, n)
-        assert (lo < hi) == (c < total)
-        (shadow if is_shadow else rays)[lo:hi] += 1
+        b, e, is_shadow = hb.chunk("segment_chunk", lo, nrays, nshadow, chunk, c)
+        assert (b < e) == (c < total) and lo <= b <= e
+        (shadow if is_shadow else rays)[b - lo:e - lo] += 1
+        assert e - lo <= (nshadow if is_shadow else nrays)
     assert (rays == 1).all() and (shadow == 1).all()
 
 

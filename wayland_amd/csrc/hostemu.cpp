@@ -254,10 +254,32 @@ uint32_t wlh_trav_variant(uint32_t depth, uint64_t nodes, uint64_t tris)
 // Entries of a queue segment of a batch of n paths (wl_pt.h).
 uint32_t wlh_pt_segment(uint64_t n) { return wl::pt_segment(n); }
 
-// The counter advance of the run-time chunk schedule (dyn_xcd_chunks).
-uint32_t wlh_dyn_chunks(uint32_t n, uint32_t xcd, uint32_t chunk)
+// The chunks and blocks that the kernels walk (traverse_device.h): [out[0],
+// out[1]), and for a segment's chunk whether it is of shadow rays in out[2].
+void wlh_eighth_chunk(uint32_t n, uint32_t xcd, uint32_t chunk, uint32_t c, uint32_t *out)
 {
-    return wl::dyn_xcd_chunks(n, xcd, chunk);
+    wl::EighthChunks(n, xcd, chunk)(c, out[0], out[1]);
+}
+uint32_t wlh_eighth_count(uint32_t n, uint32_t xcd, uint32_t chunk)
+{
+    return wl::EighthChunks(n, xcd, chunk).count();
+}
+void wlh_dealt_block(uint32_t n, uint32_t xcd, uint32_t k, uint32_t *out)
+{
+    const wl::QueueWalk q = wl::dealt_walk<wl::kPtBlock>(n, xcd);
+    out[0] = std::min(q.at(k), q.limit);
+    out[1] = std::min(q.at(k) + (uint32_t)wl::kPtBlock, q.limit);
+}
+void wlh_dealt_chunk(uint32_t n, uint32_t xcd, uint32_t chunk, uint32_t c, uint32_t *out)
+{
+    wl::DealtChunks<wl::kPtBlock>(n, xcd, chunk)(c, out[0], out[1]);
+}
+void wlh_segment_chunk(uint32_t lo, uint32_t nrays, uint32_t nshadow, uint32_t chunk, uint32_t c,
+                       uint32_t *out)
+{
+    bool shadow = false;
+    wl::SegmentChunks(lo, nrays, nshadow, chunk)(c, out[0], out[1], shadow);
+    out[2] = shadow;
 }
 
 } // extern "C"

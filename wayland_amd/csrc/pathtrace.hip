@@ -45,8 +45,6 @@
 namespace wl
 {
 
-constexpr int kPtBlock = 256;
-
 // A pointer to device memory that was itself loaded from memory (a request's
 // scene): without this the compiler reads through it with flat instructions,
 // which wait on the LDS counter too.
@@ -80,18 +78,12 @@ __device__ __forceinline__ uint32_t *queue_chunks(const PtBuffers &B, uint32_t x
     return B.counters + kPtCounterStride * (4 * xcd + 2);
 }
 
-// The entries of the ray queue that this XCD's workgroups take, in blocks of
-// kPtBlock: block k of the walk is [at(k), at(k) + kPtBlock) clipped to limit.
-struct QueueWalk
-{
-    uint32_t base, step, limit;
-    __device__ __forceinline__ uint32_t at(uint32_t k) const { return base + k * step; }
-};
+// The entries of the ray queue that this XCD's workgroups take.
 __device__ __forceinline__ QueueWalk queue_walk(const PtBuffers &B, int parity, bool first)
 {
     const uint32_t x = blockIdx.x % 8u;
     if (first)
-        return QueueWalk{ x * kPtBlock, 8u * kPtBlock, B.counters[kPtFlatCount] };
+        return dealt_walk<kPtBlock>(B.counters[kPtFlatCount], x);
     const uint32_t lo = x * B.segcap;
     return QueueWalk{ lo, kPtBlock, lo + (uint32_t)*queue_len(B, x, parity) };
 }
@@ -217,16 +209,9 @@ __device__ __forceinline__ uint32_t queue_chunk(uint32_t n_xcd)
     return n_xcd / 128u < wavesx ? 64u : 128u;
 }
 
-// The first queue's chunks: the XCD's blocks of kPtBlock entries, in pieces.
-__device__ __forceinline__ auto first_chunks(uint32_t n)
+__device__ __forceinline__ DealtChunks<kPtBlock> first_chunks(uint32_t n)
 {
-    const uint32_t chunk = queue_chunk(n / 8u), per = kPtBlock / chunk;
-    const uint32_t x = blockIdx.x % 8u;
-    return [=](uint32_t c, uint32_t &next, uint32_t &end) {
-        const uint64_t s0 = ((uint64_t)(c / per) * 8u + x) * kPtBlock + (c % per) * chunk;
-        next = (uint32_t)(s0 < n ? s0 : n);
-        end = (uint32_t)(s0 + chunk < n ? s0 + chunk : n);
-    };
+    return DealtChunks<kPtBlock>(n, blockIdx.x % 8u, queue_chunk(n / 8u));
 }
 
 // The first bounce of a single-scene batch: queue entry i is path i, and its
@@ -242,7 +227,7 @@ void k_trace_first(PtParams P, PtScene S, PtBuffers B)
     const uint32_t count = P.npix * P.nsamples;
     if (blockIdx.x == 0 && threadIdx.x == 0)
         B.stats[0] += count;
-    auto range = first_chunks(count);
+    const auto range = first_chunks(count);
     trav_persistent<kClosest, kPtBlock, WIDE, pt_top_nodes<STACK, false>() != 0>(
         S.nodes, S.tris, stack,
         XcdChunks<kPtBlock, decltype(range)>(range, queue_chunks(B, blockIdx.x % 8u), 0u),
@@ -352,21 +337,13 @@ void k_trace(PtScene S, PtBuffers B, int parity, const PtReq *__restrict__ reqs,
             atomicAdd(&B.stats[1], (unsigned long long)nshadow);
     }
     const auto flat_range = first_chunks(flat);
-    const uint32_t lo = x * B.segcap;
-    const uint32_t chunk = queue_chunk(nrays + nshadow);
-    const uint32_t ray_chunks = (nrays + chunk - 1u) / chunk;
+    const SegmentChunks seg_range(x * B.segcap, nrays, nshadow, queue_chunk(nrays + nshadow));
     bool shadow = false; // the kind of the wave's current chunk
     auto range = [&](uint32_t c, uint32_t &next, uint32_t &end) {
         if (first)
-        {
             flat_range(c, next, end);
-            return;
-        }
-        shadow = c >= ray_chunks;
-        const uint32_t n = shadow ? nshadow : nrays;
-        const uint64_t s0 = (uint64_t)(shadow ? c - ray_chunks : c) * chunk;
-        next = lo + (uint32_t)(s0 < n ? s0 : n);
-        end = lo + (uint32_t)(s0 + chunk < n ? s0 + chunk : n);
+        else
+            seg_range(c, next, end, shadow);
     };
     trav_persistent<kMixed, kPtBlock, WIDE, pt_top_nodes<STACK, MULTI>() != 0>(
         S.nodes, S.tris, stack, XcdChunks<kPtBlock, decltype(range)>(range, queue_chunks(B, x), 0u),
@@ -1069,7 +1046,7 @@ void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__re
             for (uint32_t x = 0; x < 8u; ++x)
                 total += (uint32_t)*queue_len(B, x, parity);
         }
-        q = QueueWalk{ (blockIdx.x % 8u) * kPtBlock, 8u * kPtBlock, total };
+        q = dealt_walk<kPtBlock>(total, blockIdx.x % 8u);
     }
     if (blockIdx.x < 8u && threadIdx.x == 0)
         *queue_chunks(B, blockIdx.x) = 0u; // the next trace counts from zero
@@ -1165,7 +1142,7 @@ void k_finish(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__r
             const uint32_t nshadow = __builtin_amdgcn_readfirstlane((uint32_t)(len >> 32));
             rays += nrays;
             shadows += nshadow;
-            const uint32_t ray_chunks = (nrays + 63u) / 64u;
+            const SegmentChunks range(e0, nrays, nshadow, 64u);
             bool shadow = false; // the kind of the wave's current chunk
             trav_persistent<kMixed, kPtBlock, WIDE, pt_top_nodes<STACK, MULTI>() != 0>(
                 S0.nodes, S0.tris, stack,
@@ -1173,12 +1150,7 @@ void k_finish(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__r
                     uint32_t c = 0;
                     if (__lane_id() == 0)
                         c = atomicAdd(&s_chunk, 1u);
-                    c = __builtin_amdgcn_readfirstlane(c);
-                    shadow = c >= ray_chunks;
-                    const uint32_t m = shadow ? nshadow : nrays;
-                    const uint32_t at0 = (shadow ? c - ray_chunks : c) * 64u;
-                    next = e0 + min(at0, m);
-                    end = e0 + min(at0 + 64u, m);
+                    range(__builtin_amdgcn_readfirstlane(c), next, end, shadow);
                 },
                 [&](uint32_t i, TravRay &r, uint32_t &root) {
                     queue_fetch<MULTI>(B, par, reqs, P0.epsilon, shadow, i, r, root);

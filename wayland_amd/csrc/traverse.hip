@@ -52,20 +52,6 @@ __device__ __forceinline__ void load_top(uint4 *top, const WlBvh8Node *__restric
     __syncthreads();
 }
 
-// The raw traces' chunks: XCD x owns the x-th eighth of the n rays (see
-// dyn_xcd_chunks), whose rays and hits then go through one L2.
-__device__ __forceinline__ auto eighth_chunks(uint32_t n, uint32_t chunk)
-{
-    const uint32_t n8 = (n + 7u) / 8u, xcd = blockIdx.x % 8u;
-    const uint32_t lo = xcd * n8 < n ? xcd * n8 : n;
-    const uint32_t hi = lo + n8 < n ? lo + n8 : n;
-    return [=](uint32_t c, uint32_t &next, uint32_t &end) {
-        const uint64_t s0 = lo + (uint64_t)c * chunk;
-        next = (uint32_t)(s0 < hi ? s0 : hi);
-        end = (uint32_t)(s0 + chunk < hi ? s0 + chunk : hi);
-    };
-}
-
 // ntop: nodes copied to LDS, min(node count, top_nodes<STACK>()); sched /
 // base: the launching stream's chunk counters and their values at launch.
 // The grid is a multiple of 8.
@@ -80,7 +66,7 @@ void k_trace_closest_p(
     __shared__ uint4 top[8 * (top_nodes<STACK>() ? top_nodes<STACK>() : 1)];
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
-    auto range = eighth_chunks(n, base.chunk);
+    const EighthChunks range(n, blockIdx.x % 8u, base.chunk);
     trav_persistent<kClosest, kTraceBlock, WIDE, top_nodes<STACK>() != 0>(
         nodes, tris, stack,
         XcdChunks<kTraceBlock, decltype(range)>(range, sched + kSchedStride * (blockIdx.x % 8u),
@@ -100,7 +86,7 @@ void k_trace_any_p(const WlBvh8Node *__restrict__ nodes, const WlTriRecord *__re
     __shared__ uint4 top[8 * (top_nodes<STACK>() ? top_nodes<STACK>() : 1)];
     if (top_nodes<STACK>())
         load_top(top, nodes, ntop);
-    auto range = eighth_chunks(n, base.chunk);
+    const EighthChunks range(n, blockIdx.x % 8u, base.chunk);
     trav_persistent<kAny, kTraceBlock, WIDE, top_nodes<STACK>() != 0>(
         nodes, tris, stack,
         XcdChunks<kTraceBlock, decltype(range)>(range, sched + kSchedStride * (blockIdx.x % 8u),
@@ -177,7 +163,7 @@ static TraceSched take_bases(wl_context_s::SchedBlock *sb, uint32_t n, uint32_t 
     for (uint32_t x = 0; x < 8; ++x)
     {
         t.base[x] = sb->base[x];
-        sb->base[x] += dyn_xcd_chunks(n, x, t.chunk);
+        sb->base[x] += EighthChunks(n, x, t.chunk).count();
     }
     return t;
 }

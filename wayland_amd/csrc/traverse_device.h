@@ -391,16 +391,82 @@ WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t i, const Tra
     return false;
 }
 
-// The raw traces' chunks (traverse_persistent.h): XCD xcd's eighth of n rays is
-// [xcd * ceil(n / 8), (xcd + 1) * ceil(n / 8)) clipped to n, in this many
-// chunks, which is what a launch advances the XCD's counter by.
-WL_HD uint32_t dyn_xcd_chunks(uint32_t n, uint32_t xcd, uint32_t chunk)
+// ---- chunks of ray indices (traverse_persistent.h hands them out) ------------
+// chunk c of an XCD is [next, end), empty past its last; no chunk after an empty
+// one holds a ray.
+
+// The raw traces: XCD xcd's eighth of n rays is [xcd * ceil(n / 8),
+// (xcd + 1) * ceil(n / 8)) clipped to n, so its rays and hits go through one L2.
+struct EighthChunks
 {
-    const uint32_t n8 = (n + 7u) / 8u;
-    const uint32_t lo = xcd * n8 < n ? xcd * n8 : n;
-    const uint32_t hi = lo + n8 < n ? lo + n8 : n;
-    return (hi - lo + chunk - 1u) / chunk;
+    uint32_t lo, hi, chunk;
+    WL_HD EighthChunks(uint32_t n, uint32_t xcd, uint32_t chunk_) : chunk(chunk_)
+    {
+        const uint32_t n8 = (n + 7u) / 8u;
+        lo = xcd * n8 < n ? xcd * n8 : n;
+        hi = lo + n8 < n ? lo + n8 : n;
+    }
+    // what a launch advances the XCD's counter by
+    WL_HD uint32_t count() const { return (hi - lo + chunk - 1u) / chunk; }
+    WL_HD void operator()(uint32_t c, uint32_t &next, uint32_t &end) const
+    {
+        const uint64_t s0 = lo + (uint64_t)c * chunk;
+        next = (uint32_t)(s0 < hi ? s0 : hi);
+        end = (uint32_t)(s0 + chunk < hi ? s0 + chunk : hi);
+    }
+};
+
+// The entries of a path tracer's queue that an XCD's workgroups take, in blocks
+// of BLOCK: block k of the walk is [at(k), at(k) + BLOCK) clipped to limit.
+struct QueueWalk
+{
+    uint32_t base, step, limit;
+    WL_HD uint32_t at(uint32_t k) const { return base + k * step; }
+};
+// A queue without segments (a batch's first, or a sorted one): the blocks are
+// dealt to the XCDs in turn.
+template <uint32_t BLOCK>
+WL_HD QueueWalk dealt_walk(uint32_t n, uint32_t xcd)
+{
+    return QueueWalk{ xcd * BLOCK, 8u * BLOCK, n };
 }
+
+// That queue's traversal: the XCD's blocks in pieces.
+template <uint32_t BLOCK>
+struct DealtChunks
+{
+    uint32_t n, xcd, chunk, per;
+    WL_HD DealtChunks(uint32_t n_, uint32_t xcd_, uint32_t chunk_)
+        : n(n_), xcd(xcd_), chunk(chunk_), per(BLOCK / chunk_)
+    {
+    }
+    WL_HD void operator()(uint32_t c, uint32_t &next, uint32_t &end) const
+    {
+        const uint64_t s0 = ((uint64_t)(c / per) * 8u + xcd) * BLOCK + (c % per) * chunk;
+        next = (uint32_t)(s0 < n ? s0 : n);
+        end = (uint32_t)(s0 + chunk < n ? s0 + chunk : n);
+    }
+};
+
+// A segment's traversal: the chunks of its rays, then those of its shadow rays,
+// both from entry lo on in queues of their own.
+struct SegmentChunks
+{
+    uint32_t lo, nrays, nshadow, chunk, ray_chunks;
+    WL_HD SegmentChunks(uint32_t lo_, uint32_t nrays_, uint32_t nshadow_, uint32_t chunk_)
+        : lo(lo_), nrays(nrays_), nshadow(nshadow_), chunk(chunk_),
+          ray_chunks((nrays_ + chunk_ - 1u) / chunk_)
+    {
+    }
+    WL_HD void operator()(uint32_t c, uint32_t &next, uint32_t &end, bool &shadow) const
+    {
+        shadow = c >= ray_chunks;
+        const uint32_t n = shadow ? nshadow : nrays;
+        const uint64_t s0 = (uint64_t)(shadow ? c - ray_chunks : c) * chunk;
+        next = lo + (uint32_t)(s0 < n ? s0 : n);
+        end = lo + (uint32_t)(s0 + chunk < n ? s0 + chunk : n);
+    }
+};
 
 // Whether the ray has nothing left to do.
 WL_HD bool trav_done(const TravState &st) { return (st.grp_mask | st.trimask) == 0; }

@@ -80,7 +80,6 @@ struct PtParams
     float gbox_lo[3], gbox_inv[3]; // position normalisation to [0,1]^3
 };
 
-// Path state (structure of float4 arrays, one entry per path) and queues.
 // Counters of a batch: for XCD x the 64-bit lengths of its segments of the two
 // ray queues (parity 0, 1; low word rays, high word shadow rays) and its chunk
 // counter, each in a cache line of its own: word kPtCounterStride * (4 x + 0, 1,
@@ -89,13 +88,20 @@ constexpr uint32_t kPtCounterStride = 32;
 constexpr uint32_t kPtCounters = 8 * 4 * kPtCounterStride;
 constexpr uint32_t kPtFlatCount = 3 * kPtCounterStride;
 
+// Threads of a workgroup of the path tracer's kernels.
+constexpr uint32_t kPtBlock = 256;
+
 // Entries of one of the eight queue segments of a batch of n paths: the shade
-// pass takes an XCD's entries in workgroups of 256, and every entry appends at
-// most one to each queue.
-constexpr uint32_t pt_segment(uint64_t n) { return (uint32_t)(((n + 255) / 256 + 7) / 8 * 256); }
+// pass takes an XCD's entries in workgroups of kPtBlock, and every entry appends
+// at most one to each queue.
+constexpr uint32_t pt_segment(uint64_t n)
+{
+    return (uint32_t)(((n + kPtBlock - 1) / kPtBlock + 7) / 8 * kPtBlock);
+}
 // Entries of a whole queue of a batch of n paths.
 constexpr size_t pt_queue_entries(uint64_t n) { return 8 * (size_t)pt_segment(n); }
 
+// Path state (structure of float4 arrays, one entry per path) and queues.
 struct PtBuffers
 {
     float4 *thr;      // throughput, w = depth (bits 0-15), guided vertices (16-31)

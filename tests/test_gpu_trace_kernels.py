@@ -169,23 +169,23 @@ def test_finished_batches_count_their_rays(gpu_ctx):
         assert big[key] == sum(s[key] for s in small), key
 
 
-def _wide(accel):
-    """The accel's rays take the 64-bit kernels from here on."""
+def _variant(accel, variant):
+    """The accel's rays take that variant's kernels from here on."""
     import ctypes as C
     from wayland_amd import _lib
-    f = _lib.load().wl_accel_test_wide
-    f.restype, f.argtypes = C.c_uint32, [C.c_void_p]
-    assert f(accel.h) == 1
+    f = _lib.load().wl_accel_test_variant
+    f.restype, f.argtypes = C.c_uint32, [C.c_void_p, C.c_uint32]
+    assert f(accel.h, variant) == variant
 
 
 @pytest.mark.parametrize("name", ["cornell", "ico"])
-def test_wide_addresses_equal_32_bit_offsets(gpu_ctx, name):
-    """The kernels of a shallow BVH past 4 GB, on one that is small: the same
-    hits and films, bit for bit, from the raw traces, a finished batch, a batch
-    of two lanes and a server."""
+def test_traversal_variants_agree(gpu_ctx, name):
+    """The kernels of a shallow BVH past 4 GB (1) and of a deep one (2), on one
+    that is small: the same hits and films, bit for bit, from the raw traces, a
+    finished batch, a batch of two lanes and a server."""
     import torch
     import wayland_amd as wl
-    print(f"case: wide {name}", flush=True)
+    print(f"case: variants {name}", flush=True)
     if name == "cornell":
         sc = scenes.textured_cornell_box(256, 256)  # fewer nodes than the LDS copy holds
     else:
@@ -194,10 +194,9 @@ def test_wide_addresses_equal_32_bit_offsets(gpu_ctx, name):
     if name == "cornell":
         rays[:, 0:3] = rays[:, 0:3] * 2 - np.float32([1, 0, 1])
 
-    def results(wide):
+    def results(variant):
         accel = wl.Accel(gpu_ctx, sc)
-        if wide:
-            _wide(accel)
+        _variant(accel, variant)
         pt = wl.PathTracer(gpu_ctx, accel, sc)
         h, occ = _hits(accel, rays)
         out = [h[k].view(np.uint32) for k in ("t", "prim", "b1", "b2")] + [occ]
@@ -211,5 +210,7 @@ def test_wide_addresses_equal_32_bit_offsets(gpu_ctx, name):
         torch.cuda.synchronize()
         return out + [f.view(torch.int32).cpu().numpy() for f in films]
 
-    for a, b in zip(results(False), results(True)):
-        assert np.array_equal(a, b)
+    short = results(0)
+    for variant in (1, 2):
+        for a, b in zip(short, results(variant)):
+            assert np.array_equal(a, b), variant

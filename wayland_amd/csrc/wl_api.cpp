@@ -362,11 +362,12 @@ wl_status wl_accel_build_triangles(wl_context ctx, const wl_tri_input *inputs,
     return WL_SUCCESS;
 }
 
-// For the tests, and not in the header: lets this BVH's rays take the 64-bit
-// addresses of one whose arrays pass 4 GB.  Returns its WL_TRAV_* variant.
-uint32_t wl_accel_test_wide(wl_accel a)
+// For the tests, and not in the header: lets this BVH's rays take the kernels of
+// a larger (WL_TRAV_SHORT_WIDE) or deeper one (WL_TRAV_DEEP); each variant takes
+// every BVH of those before it.  Returns the BVH's variant.
+uint32_t wl_accel_test_variant(wl_accel a, uint32_t variant)
 {
-    a->trav_variant = std::max<uint32_t>(a->trav_variant, WL_TRAV_SHORT_WIDE);
+    a->trav_variant = std::max(a->trav_variant, std::min<uint32_t>(variant, WL_TRAV_DEEP));
     return a->trav_variant;
 }
 

@@ -9,6 +9,8 @@ every interleaving of the fetches, each ray must be taken exactly once and the
 counter must advance by EighthChunks::count, the amount the host adds to the
 base it keeps for the next launch on the stream.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -63,14 +65,24 @@ def test_every_ray_once_and_counter_advance(grid, chunk):
 
 @pytest.mark.parametrize("chunk", [64, 128])
 def test_largest_launches_stay_in_range(chunk):
-    """The last chunks of about 2^31 and 2^32 rays, and those past them."""
-    for n in ((1 << 31) + 5, (1 << 32) - 9):
-        n8 = (n + 7) // 8
-        for x in range(8):
-            lo, hi = min(x * n8, n), min((x + 1) * n8, n)
-            count = hb.lib().wlh_eighth_count(n, x, chunk)
-            assert count == (hi - lo + chunk - 1) // chunk
-            assert hb.chunk("eighth_chunk", n, x, chunk, 0)[0] == lo
-            assert hb.chunk("eighth_chunk", n, x, chunk, count - 1)[1] == hi
-            b, e = hb.chunk("eighth_chunk", n, x, chunk, count + 7)
-            assert b == e == hi
+    """The launches of up to 2^32 - 1 rays: their first and last chunks, and those
+    past them.  A wave's next index, up to 64 past its last ray, fits 32 bits."""
+    f = hb.lib().wlh_launch_rays
+    f.restype, f.argtypes = C.c_uint32, [C.c_uint32]
+    for total in ((1 << 31) + 5, (1 << 32) - 70, (1 << 32) - 9, (1 << 32) - 7, (1 << 32) - 1):
+        left = total
+        while left:
+            n = f(left)
+            assert 0 < n <= left and n % 32 * (left - n) == 0  # any-hit words are not shared
+            left -= n
+            n8 = (n + 7) // 8
+            for x in range(8):
+                lo, hi = min(x * n8, n), min((x + 1) * n8, n)
+                assert hi + 64 < 1 << 32
+                count = hb.lib().wlh_eighth_count(n, x, chunk)
+                assert count == (hi - lo + chunk - 1) // chunk
+                if count:
+                    assert hb.chunk("eighth_chunk", n, x, chunk, 0)[0] == lo
+                    assert hb.chunk("eighth_chunk", n, x, chunk, count - 1)[1] == hi
+                b, e = hb.chunk("eighth_chunk", n, x, chunk, count + 7)
+                assert b == e == hi

@@ -264,6 +264,7 @@ uint32_t wlh_eighth_count(uint32_t n, uint32_t xcd, uint32_t chunk)
 {
     return wl::EighthChunks(n, xcd, chunk).count();
 }
+uint32_t wlh_launch_rays(uint32_t left) { return wl::launch_rays(left); }
 void wlh_dealt_block(uint32_t n, uint32_t xcd, uint32_t k, uint32_t *out)
 {
     const wl::QueueWalk q = wl::dealt_walk<wl::kPtBlock>(n, xcd);

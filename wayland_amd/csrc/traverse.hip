@@ -231,6 +231,20 @@ static hipError_t any_impl(const wl_accel_s *a, const wl_ray *rays, uint32_t n,
     return hipGetLastError();
 }
 
+// f(first, rays) for every launch of a trace of n rays.
+template <class F>
+static hipError_t for_launches(uint32_t n, F f)
+{
+    hipError_t e = hipSuccess;
+    for (uint32_t first = 0; e == hipSuccess && first < n;)
+    {
+        const uint32_t m = launch_rays(n - first);
+        e = f(first, m);
+        first += m;
+    }
+    return e;
+}
+
 hipError_t launch_trace_closest(const wl_accel_s *a, const wl_ray *rays,
                                 uint32_t n, wl_hit *hits, uint32_t *counts,
                                 hipStream_t s)
@@ -239,7 +253,7 @@ hipError_t launch_trace_closest(const wl_accel_s *a, const wl_ray *rays,
         return hipSuccess;
     if (counts)
     {
-        dim3 grid((n + kTraceBlock - 1) / kTraceBlock), block(kTraceBlock);
+        dim3 grid(n / kTraceBlock + (n % kTraceBlock != 0)), block(kTraceBlock);
         if (a->trav_variant == WL_TRAV_DEEP)
             hipLaunchKernelGGL(k_trace_closest_counted<WL_BVH8_STACK_DEPTH>, grid, block, 0, s,
                                a->d_nodes, a->d_tris, rays, n, hits, counts);
@@ -249,7 +263,9 @@ hipError_t launch_trace_closest(const wl_accel_s *a, const wl_ray *rays,
         return hipGetLastError();
     }
     return with_variant(a->trav_variant, [&](auto v) {
-        return closest_impl<decltype(v)>(a, rays, n, hits, s);
+        return for_launches(n, [&](uint32_t first, uint32_t m) {
+            return closest_impl<decltype(v)>(a, rays + first, m, hits + first, s);
+        });
     });
 }
 
@@ -258,8 +274,11 @@ hipError_t launch_trace_any(const wl_accel_s *a, const wl_ray *rays,
 {
     if (n == 0)
         return hipSuccess;
-    return with_variant(a->trav_variant,
-                        [&](auto v) { return any_impl<decltype(v)>(a, rays, n, bits, s); });
+    return with_variant(a->trav_variant, [&](auto v) {
+        return for_launches(n, [&](uint32_t first, uint32_t m) {
+            return any_impl<decltype(v)>(a, rays + first, m, bits + first / 32, s);
+        });
+    });
 }
 
 } // namespace wl

@@ -395,6 +395,11 @@ WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t i, const Tra
 // chunk c of an XCD is [next, end), empty past its last; no chunk after an empty
 // one holds a ray.
 
+// Rays of the next launch of a raw trace with `left` to go: the kernels' ray
+// indices are 32 bits and run up to 64 past the last one, so a trace of more than
+// 2^31 rays takes two launches.
+WL_HD uint32_t launch_rays(uint32_t left) { return left < 1u << 31 ? left : 1u << 31; }
+
 // The raw traces: XCD xcd's eighth of n rays is [xcd * ceil(n / 8),
 // (xcd + 1) * ceil(n / 8)) clipped to n, so its rays and hits go through one L2.
 struct EighthChunks

@@ -15,8 +15,8 @@ extern "C" {
 int wlh_build(const float *tris, uint32_t ntris, void **out, char *err, int errlen);
 void wlh_free(void *p);
 void wlh_info(void *p, uint32_t *out6);
-uint64_t wlh_trace(void *p, const float *rays, uint32_t n, float *hits, int any,
-                   uint32_t *counts, int nthreads);
+uint64_t wlh_trace(void *p, const float *rays, uint32_t n, float *hits, int kind,
+                   uint32_t *counts, int nthreads, uint32_t variant);
 uint64_t wlh_serve_check(const uint32_t *req4, uint32_t n, uint32_t capacity, uint64_t *out4);
 }
 
@@ -65,8 +65,12 @@ int main()
             r[6] = i % 17 ? z : 0.0f; // some axis-parallel directions
             r[7] = i % 5 ? INFINITY : 0.4f;
         }
-        faults += wlh_trace(h, rays.data(), nr, hits.data(), 0, counts.data(), 3);
-        faults += wlh_trace(h, rays.data(), nr, hits.data(), 1, nullptr, 2);
+        for (uint32_t variant = 0; variant < 3; ++variant)
+        {
+            faults += wlh_trace(h, rays.data(), nr, hits.data(), 0, counts.data(), 3, variant);
+            faults += wlh_trace(h, rays.data(), nr, hits.data(), 1, nullptr, 2, variant);
+            faults += wlh_trace(h, rays.data(), nr, hits.data(), 2, nullptr, 2, variant);
+        }
         printf("%u tris: %u nodes, depth %u\n", nt, info[0], info[2]);
         wlh_free(h);
     }

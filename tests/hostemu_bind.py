@@ -28,7 +28,7 @@ def lib():
         L.wlh_info.argtypes = [C.c_void_p, C.POINTER(C.c_uint32)]
         L.wlh_trace.restype = C.c_uint64
         L.wlh_trace.argtypes = [C.c_void_p, C.c_void_p, C.c_uint32, C.c_void_p, C.c_int,
-                                C.c_void_p, C.c_int]
+                                C.c_void_p, C.c_int, C.c_uint32]
         L.wlh_serve_check.restype = C.c_uint64
         L.wlh_serve_check.argtypes = [C.c_void_p, C.c_uint32, C.c_uint32, C.c_void_p]
         L.wlh_eighth_count.restype = C.c_uint32
@@ -60,13 +60,16 @@ class HostBVH8:
         lib().wlh_info(self.h, out)
         return dict(zip(["nodes", "tris", "depth", "inner", "leaves", "sah"], list(out)))
 
-    def trace(self, rays, any_hit=False, nthreads=8):
+    def trace(self, rays, any_hit=False, nthreads=8, variant=0, mixed=False):
+        """mixed: odd rays are any-hit rays, the others closest-hit ones.
+        variant: at least that one of bvh8.h's traversal variants."""
         rays = np.ascontiguousarray(rays, np.float32).reshape(-1, 8)
         n = rays.shape[0]
         hits = np.zeros((n, 4), np.float32)
         counts = np.zeros((n, 2), np.uint32)
         faults = lib().wlh_trace(self.h, rays.ctypes.data, n, hits.ctypes.data,
-                                 1 if any_hit else 0, counts.ctypes.data, nthreads)
+                                 2 if mixed else 1 if any_hit else 0, counts.ctypes.data,
+                                 nthreads, variant)
         return hits, counts, int(faults)
 
     def __del__(self):

@@ -26,6 +26,13 @@ def _check(tris, rays):
     assert fa == 0
     occ = ha[:, 1].view(np.uint32) != 0xFFFFFFFF
     assert np.array_equal(occ, hit)
+    # both kinds of ray in one launch, and the variants of larger and deeper trees
+    both = np.where(np.arange(len(rays))[:, None] % 2 == 0, hits, ha)
+    for variant in range(3):
+        for kw, want in ((dict(mixed=True), both), (dict(), hits), (dict(any_hit=True), ha)):
+            got, _, faults = h.trace(rays, variant=variant, **kw)
+            assert faults == 0
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
     return h, counts
 
 
@@ -88,3 +95,12 @@ def test_traversal_variant(depth, nodes, tris, variant):
     f = hb.lib().wlh_trav_variant
     f.restype, f.argtypes = C.c_uint32, [C.c_uint32, C.c_uint64, C.c_uint64]
     assert f(depth, nodes, tris) == variant
+
+
+def test_the_stack_bound_is_checked():
+    """Rays that need more stack entries than there are count as faults."""
+    h = hb.HostBVH8(scenes.icosphere_scene(25, 4).triangles())
+    depth = h.info()["depth"]
+    rays = scenes.traversal_rays(20000, seed=3)
+    assert h.trace(rays, variant=(depth - 2) << 8)[2] == 0  # one entry per level at most
+    assert h.trace(rays, variant=2 << 8)[2] > 0

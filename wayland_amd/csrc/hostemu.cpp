@@ -17,6 +17,7 @@
 
 static thread_local size_t wl_trav_nodes_bound = 0;
 static thread_local size_t wl_trav_tris_bound = 0;
+static thread_local uint32_t wl_trav_stack_bound = 0;
 static std::atomic<uint64_t> g_faults{ 0 };
 static thread_local const char *g_fault_what = nullptr;
 
@@ -34,9 +35,11 @@ static thread_local const char *g_fault_what = nullptr;
 #include "traverse_device.h"
 #include "wl_pt.h"
 
+using wl::Bvh8Host;
+
 struct HostEmu
 {
-    wl::Bvh8Host bvh;
+    Bvh8Host bvh;
 };
 
 extern "C" {
@@ -72,29 +75,42 @@ void wlh_info(void *p, uint32_t *out6)
     out6[5] = (uint32_t)(h->bvh.sah_cost);
 }
 
-// rays: n x 8 floats; hits: n x 4 (t, prim bits, b1, b2); counts: n x 2 or NULL
+// rays: n x 8 floats; hits: n x 4 (t, prim bits, b1, b2); counts: n x 2 or NULL.
+// kind: 0 closest hits, 1 any hits, 2 both in one run, odd rays any hits.  The
+// traversal is that of the kernels that the BVH's variant takes, or of a larger
+// variant if the low byte of `variant` says so, with that variant's stack, or one
+// of as many entries as the bits above that byte say.
 uint64_t wlh_trace(void *p, const float *rays, uint32_t n, float *hits,
-                   int any, uint32_t *counts, int nthreads)
+                   int kind, uint32_t *counts, int nthreads, uint32_t variant)
 {
     HostEmu *h = (HostEmu *)p;
+    const Bvh8Host &bvh = h->bvh;
     g_faults = 0;
-    auto work = [&](uint32_t b, uint32_t e) {
-        wl_trav_nodes_bound = h->bvh.nodes.size();
-        wl_trav_tris_bound = h->bvh.tris.size();
-        uint32_t stack[WL_BVH8_STACK_DEPTH];
+    const uint32_t entries = variant >> 8;
+    variant = std::max(variant & 0xFFu,
+                       wl_bvh8_variant(bvh.depth, bvh.nodes.size(), bvh.tris.size()));
+    // a copy of the top levels, as the short-stack kernels of one BVH hold it
+    const std::vector<WlBvh8Node> top(bvh.nodes.begin(),
+                                      bvh.nodes.begin() + std::min<size_t>(73, bvh.nodes.size()));
+    auto run = [&](auto v, auto rays_kind, uint32_t b, uint32_t e) {
+        using V = decltype(v);
+        constexpr int RAYS = decltype(rays_kind)::value;
+        constexpr bool TOP = V::STACK == WL_BVH8_SHALLOW_DEPTH;
+        wl_trav_nodes_bound = bvh.nodes.size();
+        wl_trav_tris_bound = bvh.tris.size();
+        wl_trav_stack_bound = entries ? entries : V::STACK;
+        std::vector<uint32_t> stack(wl_trav_stack_bound); // on the heap: seen by a sanitizer
         for (uint32_t i = b; i < e; ++i)
         {
             const float *r = rays + 8 * (size_t)i;
             wl::TravRay tr;
             wl::trav_setup(tr, r[0], r[1], r[2], r[4], r[5], r[6], r[3], r[7]);
+            if (RAYS == wl::kMixed && i % 2)
+                tr.code |= wl::kAnyRay;
             uint32_t nn = 0, nt = 0;
-            wl::TravResult res;
-            if (any)
-                res = wl::trav_run<wl::kAny, true, 1>(h->bvh.nodes.data(), h->bvh.tris.data(),
-                                                  tr, true, stack, 0, nn, nt);
-            else
-                res = wl::trav_run<wl::kClosest, true, 1>(h->bvh.nodes.data(), h->bvh.tris.data(),
-                                                   tr, true, stack, 0, nn, nt);
+            const wl::TravResult res = wl::trav_run<RAYS, true, 1, false, TOP, V::WIDE>(
+                bvh.nodes.data(), bvh.tris.data(), tr, true, stack.data(), 0, nn, nt, top.data(),
+                (uint32_t)top.size());
             float *o = hits + 4 * (size_t)i;
             o[0] = res.t;
             std::memcpy(&o[1], &res.prim, 4);
@@ -106,6 +122,16 @@ uint64_t wlh_trace(void *p, const float *rays, uint32_t n, float *hits,
                 counts[2 * (size_t)i + 1] = nt;
             }
         }
+    };
+    auto work = [&](uint32_t b, uint32_t e) {
+        wl::with_variant(variant, [&](auto v) {
+            if (kind == 0)
+                run(v, std::integral_constant<int, wl::kClosest>{}, b, e);
+            else if (kind == 1)
+                run(v, std::integral_constant<int, wl::kAny>{}, b, e);
+            else
+                run(v, std::integral_constant<int, wl::kMixed>{}, b, e);
+        });
     };
     if (nthreads < 1)
         nthreads = 1;

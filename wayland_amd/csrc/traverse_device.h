@@ -391,6 +391,22 @@ WL_HD bool tri_visit(const WlTriRecord *__restrict__ tris, uint32_t i, const Tra
     return false;
 }
 
+// A traversal variant (WL_TRAV_*) as template arguments, and f called with that
+// of v.
+template <int STACK_, bool WIDE_>
+struct TravVariant
+{
+    static constexpr int STACK = STACK_;
+    static constexpr bool WIDE = WIDE_;
+};
+template <class F>
+auto with_variant(uint32_t v, F f)
+{
+    return v == WL_TRAV_SHORT        ? f(TravVariant<WL_BVH8_SHALLOW_DEPTH, false>{})
+           : v == WL_TRAV_SHORT_WIDE ? f(TravVariant<WL_BVH8_SHALLOW_DEPTH, true>{})
+                                     : f(TravVariant<WL_BVH8_STACK_DEPTH, true>{});
+}
+
 // ---- chunks of ray indices (traverse_persistent.h hands them out) ------------
 // chunk c of an XCD is [next, end), empty past its last; no chunk after an empty
 // one holds a ray.
@@ -497,7 +513,7 @@ WL_HD bool trav_node(const WlBvh8Node *__restrict__ nodes, const TravRay &r, Tra
     {
         if (rest)
         {
-            WL_TRAV_CHECK(st.sp < WL_BVH8_STACK_DEPTH * BLOCK, "stack depth");
+            WL_TRAV_CHECK(st.sp < wl_trav_stack_bound * BLOCK, "stack depth");
             lds_stack[st.sp] = st.grp_base << 5 | rest; // base / 8 in the upper 24 bits
             st.sp += BLOCK;
         }
@@ -542,17 +558,17 @@ WL_HD void trav_finish(TravResult &res)
 }
 
 // Traverse one ray to completion.  lane: the ray's first entry of the stack.
-template <int RAYS, bool COUNT, int BLOCK, bool AUX = false>
+template <int RAYS, bool COUNT, int BLOCK, bool AUX = false, bool TOP = false, bool WIDE = true>
 WL_HD TravResult trav_run(const WlBvh8Node *__restrict__ nodes,
                           const WlTriRecord *__restrict__ tris, const TravRay &r, bool active,
                           uint32_t *lds_stack, uint32_t lane, uint32_t &n_nodes,
-                          uint32_t &n_tris)
+                          uint32_t &n_tris, const WlBvh8Node *top = nullptr, uint32_t ntop = 0)
 {
     TravState st;
     trav_init(st, r, active, lane);
     while (st.grp_mask)
     {
-        if (trav_node<BLOCK>(nodes, r, st, lds_stack))
+        if (trav_node<BLOCK, TOP, WIDE>(nodes, r, st, lds_stack, top, ntop))
             break; // CPU emulation only: an index out of range
         if (COUNT)
             ++n_nodes;
@@ -560,7 +576,7 @@ WL_HD TravResult trav_run(const WlBvh8Node *__restrict__ nodes,
         {
             if (COUNT)
                 ++n_tris;
-            if (trav_tri<RAYS, AUX>(tris, r, st))
+            if (trav_tri<RAYS, AUX, WIDE>(tris, r, st))
                 break;
         }
     }

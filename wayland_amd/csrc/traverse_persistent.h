@@ -105,22 +105,6 @@ struct XcdChunks
     }
 };
 
-// A traversal variant (WL_TRAV_*) as template arguments, and f called with that
-// of v.
-template <int STACK_, bool WIDE_>
-struct TravVariant
-{
-    static constexpr int STACK = STACK_;
-    static constexpr bool WIDE = WIDE_;
-};
-template <class F>
-auto with_variant(uint32_t v, F f)
-{
-    return v == WL_TRAV_SHORT        ? f(TravVariant<WL_BVH8_SHALLOW_DEPTH, false>{})
-           : v == WL_TRAV_SHORT_WIDE ? f(TravVariant<WL_BVH8_SHALLOW_DEPTH, true>{})
-                                     : f(TravVariant<WL_BVH8_STACK_DEPTH, true>{});
-}
-
 // chunks(first, next, end): the wave's next chunk [next, end) of ray indices,
 // wave-uniform, empty when there is none left.  fetch(i, TravRay&, root) sets
 // up ray i of the current chunk (root: the index of its first node, 0 unless

@@ -208,3 +208,53 @@ def test_trained_network_is_published(gpu_ctx):
     g.close()
     fresh.close()
     pt.close()
+
+
+def _all_guidable(name, w, h):
+    if name == "cornell":
+        return scenes.cornell_box(w, h)
+    sc = scenes.wavefront_scene(6, 3, width=w, height=h)
+    rng = np.random.default_rng(2)
+    for m in sc.meshes:
+        if m.light_L is None:
+            m.material = scenes.disney_material(color=rng.uniform(0.2, 0.9, 3),
+                                                roughness=rng.uniform(0.1, 1.0))
+    return sc
+
+
+@pytest.mark.parametrize("name", ["cornell", "wave"])
+@pytest.mark.parametrize("bounces", [1, 2])
+def test_finished_training_batches_equal_launched_bounces(gpu_ctx, name, bounces):
+    """A training render whose guide is limited to the first bounces runs the
+    others in one kernel; with every bounce allowed it launches each.  Where a
+    path's first vertex is its only guided one the two do the same, bit for
+    bit: the films, the number of training samples and, where one workgroup
+    gathers them (2048 paths: in path order), the trained parameters."""
+    import torch
+    import wayland_amd as wl
+    params = wl.Guide(gpu_ctx, seed=9).get_params()
+    for w, h in ((64, 32), (509, 401)):
+        print(f"case: training batch {name} {w} x {h}, bounces {bounces}", flush=True)
+        sc = _all_guidable(name, w, h)
+        accel = wl.Accel(gpu_ctx, sc)
+        got = []
+        for limit in (bounces, 0):
+            pt = wl.PathTracer(gpu_ctx, accel, sc)
+            guide = wl.Guide(gpu_ctx, batch_size=1024, steps_per_batch=2,
+                             guided_bounces=limit, guided_vertices=1)
+            guide.set_params(params)
+            pt.set_guide(guide, wl.GUIDE_SAMPLE | wl.GUIDE_TRAIN)
+            films = []
+            for frame in range(3 if w * h <= 2048 else 1):
+                film, _ = pt.render(wl.pt_config(w, h, spp=1, frame_offset=frame, max_depth=12,
+                                                 max_batch_paths=w * h), stats=False)
+                films.append(film.view(torch.int32).cpu().numpy())
+            got.append((films, guide.info(), guide.get_params()))
+            pt.set_guide(None)
+        (fa, ia, pa), (fb, ib, pb) = got
+        for a, b in zip(fa, fb):
+            assert np.array_equal(a, b)
+        assert ia == ib and ia["last_samples"] > 0
+        if w * h <= 2048:
+            assert np.array_equal(pa.view(np.uint32), pb.view(np.uint32))
+            assert not np.array_equal(pa, params)

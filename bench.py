@@ -55,6 +55,8 @@ def parse():
                    help="guided glossy-caustic run length in spp (0 = skip)")
     p.add_argument("--guide-res", type=int, default=1024)
     p.add_argument("--guide-runs", type=int, default=60)
+    p.add_argument("--guide-scores", default="",
+                   help="write the relMSE of every guided and plain run to this JSON file")
     p.add_argument("--guide-steps", type=int, default=0,
                    help="Adam steps per pass (0: the library default)")
     p.add_argument("--serve-requests", type=int, default=64,
@@ -296,19 +298,14 @@ def bench_guide(args, ctx, wl, torch):
     g_sc, p_sc, c_sc = np.array(g_sc), np.array(p_sc), np.array(c_sc)
 
     def side(k):
-        g, p, c = g_sc[:, k].tolist(), p_sc[:, k].tolist(), c_sc[:, k].tolist()
-        per_run = np.asarray(g) / np.maximum(np.asarray(c), 1e-300)
-        return {"relmse_guided": g, "relmse_plain": p,
-                "relmse_ratio_equal_time": float(np.mean(g) / np.mean(p)),
-                "relmse_ratio_ci95": bootstrap_ratio_ci(g, p),
-                "relmse_median_ratio": float(np.median(g) / np.median(p)),
-                "common_seeds": {
-                    "relmse_plain": c,
-                    "relmse_ratio_equal_time": float(np.mean(g) / np.mean(c)),
-                    "relmse_ratio_ci95": bootstrap_paired_ratio_ci(g, c),
-                    "median_of_run_ratios": float(np.median(per_run)),
-                    "runs_guided_below_plain": int((per_run < 1.0).sum())}}
+        return guide_side(g_sc[:, k], p_sc[:, k], c_sc[:, k])
 
+    if args.guide_scores:
+        with open(args.guide_scores, "w") as f:
+            json.dump({name: {"guided": g_sc[:, k].tolist(), "plain": p_sc[:, k].tolist(),
+                              "plain_common_seeds": c_sc[:, k].tolist()}
+                       for k, name in enumerate(("full_view", "floor", "caustic_window",
+                                                 "off_sphere", "sphere"))}, f)
     out = {"workload": f"glossy caustic {res}x{res}, {sc.num_triangles} tris, depth {depth}",
            "runs": runs,
            "guided": {"spp": args.guide_spp, "seconds": float(np.mean(g_t)), "adam_steps": steps},
@@ -342,6 +339,26 @@ def bench_guide(args, ctx, wl, torch):
         out["full_view"]["relmse_ratio_equal_time"]
     log(f"guide: {out}")
     return out
+
+
+def guide_side(g, p, c):
+    """Statistics over the runs of one region: relMSE of the guided runs g, of
+    the plain runs p and of the plain runs with the guided runs' frame offsets
+    c.  The result line carries these, not the runs (--guide-scores), so that
+    it stays a few kilobytes whatever the number of runs."""
+    per_run = g / np.maximum(c, 1e-300)
+    return {"relmse_guided_mean": float(np.mean(g)), "relmse_guided_median": float(np.median(g)),
+            "relmse_plain_mean": float(np.mean(p)), "relmse_plain_median": float(np.median(p)),
+            "relmse_ratio_equal_time": float(np.mean(g) / np.mean(p)),
+            "relmse_ratio_ci95": bootstrap_ratio_ci(g, p),
+            "relmse_median_ratio": float(np.median(g) / np.median(p)),
+            "common_seeds": {
+                "relmse_plain_mean": float(np.mean(c)),
+                "relmse_plain_median": float(np.median(c)),
+                "relmse_ratio_equal_time": float(np.mean(g) / np.mean(c)),
+                "relmse_ratio_ci95": bootstrap_paired_ratio_ci(g, c),
+                "median_of_run_ratios": float(np.median(per_run)),
+                "runs_guided_below_plain": int((per_run < 1.0).sum())}}
 
 
 def bootstrap_ratio_ci(a, b, n=10000, seed=0):

@@ -394,7 +394,7 @@ __global__ __launch_bounds__(kPtBlock) void k_sort_count(PtParams P, PtScene S, 
             atomicAdd(&B.sort_bins[b], hist[b]);
 }
 
-// One block: bin counts -> running bin offsets; clears the counts.
+// One block: bin counts -> running bin offsets and their total; clears the counts.
 __global__ void k_sort_scan(PtParams P, PtBuffers B)
 {
     __shared__ uint32_t part[kPtBlock];
@@ -415,6 +415,7 @@ __global__ void k_sort_scan(PtParams P, PtBuffers B)
             part[t] = run;
             run += v;
         }
+        B.counters[kPtSortTotal] = run;
     }
     __syncthreads();
     uint32_t run = part[threadIdx.x];
@@ -1039,14 +1040,8 @@ void k_shade(PtParams P0, PtScene S0, PtBuffers B, int parity, const PtReq *__re
     if (!MULTI && P0.sort_bins)
     {
         // the sorted order of the whole queue, dealt in blocks as the first's
-        uint32_t total = B.counters[kPtFlatCount];
-        if (!first)
-        {
-            total = 0;
-            for (uint32_t x = 0; x < 8u; ++x)
-                total += (uint32_t)*queue_len(B, x, parity);
-        }
-        q = dealt_walk<kPtBlock>(total, blockIdx.x % 8u);
+        // (one word: the eight segments' lengths cost every workgroup 2 us more)
+        q = dealt_walk<kPtBlock>(B.counters[kPtSortTotal], blockIdx.x % 8u);
     }
     if (blockIdx.x < 8u && threadIdx.x == 0)
         *queue_chunks(B, blockIdx.x) = 0u; // the next trace counts from zero

@@ -83,10 +83,12 @@ struct PtParams
 // Counters of a batch: for XCD x the 64-bit lengths of its segments of the two
 // ray queues (parity 0, 1; low word rays, high word shadow rays) and its chunk
 // counter, each in a cache line of its own: word kPtCounterStride * (4 x + 0, 1,
-// 2).  kPtFlatCount: the length of the first queue, which has no segments.
+// 2).  kPtFlatCount: the length of the first queue, which has no segments;
+// kPtSortTotal: the entries that the material sort put in order.
 constexpr uint32_t kPtCounterStride = 32;
 constexpr uint32_t kPtCounters = 8 * 4 * kPtCounterStride;
 constexpr uint32_t kPtFlatCount = 3 * kPtCounterStride;
+constexpr uint32_t kPtSortTotal = kPtFlatCount + 1;
 
 // Threads of a workgroup of the path tracer's kernels.
 constexpr uint32_t kPtBlock = 256;

@@ -236,7 +236,10 @@ enum
 };
 enum
 {
-    WL_PT_SORT_BY_MATERIAL = 1u << 0 /* shade queue binned by material id */
+    /* Shade queue binned by material id.  A batch of fewer than 2^22 paths
+     * bins its first two bounces only (the others run in one kernel).  Samples
+     * are the same with and without. */
+    WL_PT_SORT_BY_MATERIAL = 1u << 0
 };
 
 typedef struct wl_pt_config

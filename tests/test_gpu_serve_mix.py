@@ -1,5 +1,5 @@
 """Batched serving at the workload's full size, and its multi-request
-kernels (k_raygen_multi, k_extend / k_shade / k_shadow with request ids,
+kernels (k_raygen_multi, k_trace / k_shade / k_finish with request ids,
 k_accumulate_multi) against the oracle.
 
 * The 64-request mix of the serving workload (Cornell and icosphere

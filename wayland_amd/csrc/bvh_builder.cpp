@@ -76,9 +76,10 @@ struct Node2
 // k = 2..7, 0 where k - 1 children cost no more.  The subtree's own node has
 // own_k children, own_i of them from the left.
 // Against opening the largest child until eight are found: the 2M-triangle soup
-// takes 268,000 nodes instead of 497,000 and 5.72 visits a ray instead of 5.89;
-// 1080p x 64 spp 35.5 -> 34.6 ms, 1M caustic paths 1.45 -> 1.40 ms, 100,003 rays
-// 65 -> 60 us, 2^23 closest hits 680 -> 672 us.
+// takes 294,000 nodes instead of 497,000 and 5.75 visits a ray instead of 5.89;
+// 1080p x 64 spp 35.5 -> 34.7 ms, 1M caustic paths 1.43 -> 1.38 ms, 100,003 rays
+// 65 -> 62 us, 2^23 closest hits 680 -> 674 us.  The build takes about 6 % longer
+// (2M triangles on 8 CPUs, four builds each twice: 3.7-5.0 -> 4.0-5.3 s).
 struct Collapse
 {
     float cost[7];
@@ -218,15 +219,16 @@ struct Bvh2Builder
     }
 };
 
-// The collapse choice of every subtree (children come after their parents);
-// subtrees that are cheaper as one leaf become leaves.  Areas are scaled
-// by a power of two that puts the root's near 2^64, so that a float holds them,
-// and their sums over 2^31 triangles, in any unit (unscaled, all costs were
-// equal at coordinates of 1e20 or 1e-23, and a ray took 46 to 60 visits where it
-// takes 24).  A box without area, triangles collapsed into a
-// point or a line, counts as kNoArea: the cheapest choice is then the one of the
-// fewest nodes (4096 triangles in one point: 1023 nodes at 0, 147 so).
+// A box without area, triangles collapsed into a point or a line, counts as this
+// in the choice: the cheapest one is then that of the fewest nodes (4096 triangles
+// in one point: 1023 nodes at 0, 147 so).
 constexpr float kNoArea = 1e-30f;
+
+// The collapse choice of every subtree (children come after their parents);
+// subtrees that are cheaper as one leaf become leaves.  Areas are scaled by a
+// power of two that puts the root's near 2^64, so that a float holds them, and
+// their sums over 2^31 triangles, in any unit (unscaled, all costs were equal at
+// coordinates of 1e20 or 1e-23, and a ray took 46 to 60 visits where it takes 24).
 std::vector<Collapse> choose_collapse(std::vector<Node2> &nodes, uint32_t n)
 {
     std::vector<Collapse> out(n);

@@ -23,13 +23,13 @@ constexpr int kTraceBlock = 256;
 // BVHs have no room for it.
 constexpr uint32_t kTopNodes = 73;
 
-// Chunks of this many rays (traverse_persistent.h), taken at run time from one counter per XCD, each counter in a cache line of
-// its own and each chunk asked for one ahead.  2^23 rays, closest / any hit:
-// 64: 696 / 534 us, 96: 688 / 522, 128: 691 / 521, 256: 713 / 523, 512: 730 /
-// 524 (727 / 603 us with 256 and the eight counters in one line).  A launch
-// with fewer than 128 rays per resident wave takes 64, which fill one wave's
-// lanes: 100,003 rays 112 -> 65 us (16: 94, 32: 79, 128: 81 before the last
-// rays' both-steps rule of trav_persistent).
+// Chunks of this many rays (traverse_persistent.h), taken at run time from one
+// counter per XCD, each counter in a cache line of its own and each chunk asked
+// for one ahead.  2^23 rays, closest / any hit: 64: 696 / 534 us, 96: 688 / 522,
+// 128: 691 / 521, 256: 713 / 523, 512: 730 / 524 (727 / 603 us with 256 and the
+// eight counters in one line).  A launch with fewer than 128 rays per resident
+// wave takes 64, which fill one wave's lanes: 100,003 rays 112 -> 65 us (16: 94,
+// 32: 79, 128: 81 before the last rays' both-steps rule of trav_persistent).
 constexpr uint32_t kTraceChunk = 128;
 
 // The chunk counters' values at launch, one per XCD, and the launch's chunk.

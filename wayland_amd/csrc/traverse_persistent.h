@@ -2,8 +2,8 @@
 //
 // Incoherent rays finish after very different numbers of steps, so a wave
 // that runs one ray per lane to completion idles most of its lanes near the
-// end.  Here a fixed grid of waves loops; once at least REFILL lanes of a wave
-// are idle, they hand out their finished results and start the next rays of
+// end.  Here a fixed grid of waves loops; once at least kRefillLanes lanes of
+// a wave are idle, they hand out their finished results and start the next rays of
 // the wave's own ray indices (after Aila & Laine, "Understanding the
 // Efficiency of Ray Traversal on GPUs", HPG 2009).
 //
@@ -173,6 +173,5 @@ __device__ __forceinline__ void trav_persistent(const WlBvh8Node *__restrict__ n
             trav_node<BLOCK, TOP, WIDE>(nodes, r, st, stack, top, ntop);
     }
 }
-
 
 } // namespace wl

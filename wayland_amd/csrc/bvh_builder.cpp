@@ -69,8 +69,8 @@ struct Node2
 };
 
 // The cheapest way to hang a BVH2 subtree into an 8-wide node (after Ylitie,
-// Karras, Laine, HPG 2017, who follow Aila and others): cost[k - 1] is the
-// SAH cost of it as at most k children, k = 1..7.  A single child is a leaf of
+// Karras, Laine, HPG 2017, who follow Aila and others): CollapseCost::k[k - 1] is
+// the SAH cost of it as at most k children, k = 1..7.  A single child is a leaf of
 // the subtree's triangles or a node of its own; k children are i from the left
 // subtree and k - i from the right: nibble k - 2 of `split` holds the i of
 // k = 2..7, 0 where k - 1 children cost no more.  The subtree's own node has
@@ -82,8 +82,11 @@ struct Node2
 // (2M triangles on 8 CPUs, four builds each twice: 3.7-5.0 -> 4.0-5.3 s).
 struct Collapse
 {
-    float cost[7];
     uint32_t split : 24, own_k : 4, own_i : 4;
+};
+struct CollapseCost // while choosing only: the larger part of the two
+{
+    float k[7];
 };
 // Cost of a triangle test relative to a node visit: 1.5 and 2.5 are equally
 // fast, 1.0 (more triangles per leaf) is 2-3 % slower, 0.6 7 %.
@@ -232,6 +235,7 @@ constexpr float kNoArea = 1e-30f;
 std::vector<Collapse> choose_collapse(std::vector<Node2> &nodes, uint32_t n)
 {
     std::vector<Collapse> out(n);
+    std::vector<CollapseCost> costs(n);
     const double root_area = nodes[0].box.area();
     const double unit = root_area > 0 && std::isfinite(root_area)
                             ? std::ldexp(1.0, 64 - std::ilogb(root_area))
@@ -240,6 +244,7 @@ std::vector<Collapse> choose_collapse(std::vector<Node2> &nodes, uint32_t n)
     {
         Node2 &nd = nodes[i];
         Collapse &c = out[i];
+        float *cost = costs[i].k;
         const double box_area = nd.box.area() * unit;
         const float area = box_area > 0 ? (float)box_area : kNoArea;
         c.split = 0;
@@ -247,11 +252,10 @@ std::vector<Collapse> choose_collapse(std::vector<Node2> &nodes, uint32_t n)
         c.own_i = 0;
         if (nd.count > 0 || nd.total == 0)
         {
-            for (float &x : c.cost)
-                x = area * kTriCost * (float)nd.total;
+            std::fill(cost, cost + 7, area * kTriCost * (float)nd.total);
             continue;
         }
-        const float *l = out[nd.left].cost, *r = out[nd.right].cost;
+        const float *l = costs[nd.left].k, *r = costs[nd.right].k;
         float as[9]; // cost as k children, k = 2..8, and the left subtree's share
         uint32_t share[9];
         for (uint32_t k = 2; k <= 8; ++k)
@@ -273,17 +277,17 @@ std::vector<Collapse> choose_collapse(std::vector<Node2> &nodes, uint32_t n)
                 own = k;
         c.own_k = own;
         c.own_i = share[own];
-        c.cost[0] = area + as[own];
+        cost[0] = area + as[own];
         const float leaf = area * kTriCost * (float)nd.total;
-        if (nd.total <= WL_BVH8_MAX_LEAF_TRIS && leaf <= c.cost[0])
+        if (nd.total <= WL_BVH8_MAX_LEAF_TRIS && leaf <= cost[0])
         {
-            c.cost[0] = leaf;
+            cost[0] = leaf;
             nd.count = nd.total;
         }
         for (uint32_t k = 2; k <= 7; ++k)
         {
-            const bool fewer = c.cost[k - 2] <= as[k];
-            c.cost[k - 1] = fewer ? c.cost[k - 2] : as[k];
+            const bool fewer = cost[k - 2] <= as[k];
+            cost[k - 1] = fewer ? cost[k - 2] : as[k];
             if (!fewer)
                 c.split |= share[k] << (4 * (k - 2));
         }
@@ -575,6 +579,9 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
     b.next_node = 1;
     b.threads_left = std::max(0, nthreads - 1);
     b.build_range(0, 0, ntris);
+    // not needed any more, and about as large as the costs of the choice
+    std::vector<Aabb>().swap(b.pbox);
+    std::vector<float>().swap(b.cen);
 
     const uint32_t n2 = b.next_node;
     double sah;
@@ -585,16 +592,14 @@ bool build_bvh8(const float *tris, uint32_t ntris, int nthreads, Bvh8Host *out,
         // near ones first, come out either way (300 triangles that shrink by
         // 0.65 each: 34 levels, 24 greedily; 600 that shrink by 0.9: 27, 34
         // greedily, more than the traversal stack holds).
-        std::vector<uint32_t> leaf_of(n2);
-        for (uint32_t i = 0; i < n2; ++i)
-            leaf_of[i] = b.nodes[i].count;
         const std::vector<Collapse> choice = choose_collapse(b.nodes, n2);
         sah = collapse_bvh8(tris, ntris, b.nodes, b.prims, &choice, out);
         const bool fits = out->nodes.size() <= kMaxNodes;
         if (out->depth > WL_BVH8_SHALLOW_DEPTH || !fits)
         {
-            for (uint32_t i = 0; i < n2; ++i)
-                b.nodes[i].count = leaf_of[i];
+            for (uint32_t i = 0; i < n2; ++i) // leaves that the choice made
+                if (b.nodes[i].left != 0)
+                    b.nodes[i].count = 0;
             Bvh8Host greedy;
             const double greedy_sah = collapse_bvh8(tris, ntris, b.nodes, b.prims, nullptr,
                                                     &greedy);
